@@ -31,8 +31,8 @@
 //     rounded once to FP32 on assignment, as C++ does;
 //   * no multiply-add contraction anywhere in this file.
 // Gradient accumulators are the one place that sums in another order: the
-// contributions of a launch's shots are added in registers, and the chain
-// rule to (lambda, mu, rho) is applied once at the end.
+// contributions of a launch's shots are added up first, in shot order, and the
+// chain rule to (lambda, mu, rho) is applied once at the end.
 //
 // Reference kernels restated here: el_stress.cu:50-131, el_velocity.cu:45-117,
 // el_velocity_adj.cu:22-108, el_stress_adj.cu:22-104, utilities.cu:125-205,
@@ -119,26 +119,6 @@ __device__ __forceinline__ double ddiv2(double x, double d, double y) {
   return __builtin_fma(__builtin_fma(-d, q, x), y, q);
 }
 
-// A C-PML stretching coefficient K of one cell and its reciprocals; x / K is
-// x itself where K == 1 (outside the C-PML).
-struct Kdiv {
-  float K, r;
-  double r64;
-  bool one;
-};
-__device__ __forceinline__ Kdiv kdiv_of(float K) {
-  Kdiv k;
-  k.K = K;
-  k.one = K == 1.f;
-  k.r = k.one ? 1.f : 1.f / K;
-  k.r64 = k.one ? 1.0 : 1.0 / (double)K;
-  return k;
-}
-__device__ __forceinline__ float kdiv(float x, const Kdiv& k) { return k.one ? x : div2(x, k.K, k.r); }
-__device__ __forceinline__ double kdiv(double x, const Kdiv& k) {
-  return k.one ? x : ddiv2(x, (double)k.K, k.r64);
-}
-
 // ------------------------------------------------------------ descriptors
 struct Geo {
   int nz, nx, nzA, nPml, nSteps;
@@ -154,11 +134,6 @@ struct Geo {
 
 struct Mdl {
   const float *lam, *mu, *amu, *ba, *bb;
-};
-
-struct Pml {
-  const float *Kz, *az, *bz, *Kzh, *azh, *bzh;  // length nzA
-  const float *Kx, *ax, *bx, *Kxh, *axh, *bxh;  // length nx
 };
 
 // Wavefield arrays are [shot][component][cell]: the 5 components of a state
@@ -177,75 +152,6 @@ enum MemComp {
   kMemComps = 8
 };
 
-struct Src {
-  const int* zx;     // [shot][2] grid indices of the source
-  const float* amp;  // [shot][nSteps] windowed source rows (Src_Rec.cu:132-143)
-};
-
-// Residual injection folded into the adjoint stress update (one-row surveys
-// with one receiver per cell): at[plan shot][x] is the receiver of column x
-// in row z, or -1.
-struct Inj {
-  const float* res;  // time-major residual, row t at res + t * R; null: no injection
-  const int* at;
-  int z;
-};
-
-// One plan's shots in one launch.  Every per-shot pointer already points at
-// the part's first shot.
-struct Part {
-  Geo g;
-  Mdl m;
-  Pml c;
-  float* w;         // forward state [shot][5][cell] from the part's first shot
-  float* a;         // adjoint state, same layout
-  float* p;         // C-PML memory variables [shot][8][cell] (forward ones in
-                    // forward launches, adjoint ones in backward launches)
-  Src src;          // source rows: injected (forward) or removed (reversal)
-  Inj inj;
-  float* ring;      // boundary ring buffer (null: not saved)
-  float* acc;       // 5 gradient accumulators
-  float* stf_grad;  // [shot][nSteps]
-  float* illum;     // forward illumination (null: off)
-  const int* rec;   // [receiver][3] = (z, x, plan shot), from the part's first receiver
-  float* syn;       // seismograms + the part's first receiver (row t at + t * R)
-  int nrec;         // receivers of the part's shots
-  int gzU;          // tiles along z of the update-region tiling
-  int gzR;          // tiles along z of the ring-rectangle tiling
-};
-
-// Kernel argument: one part by value, or a table of parts in device memory.
-template <int NP>
-struct Parts;
-template <>
-struct Parts<1> {
-  Part p;
-  __device__ __forceinline__ const Part& get(int) const { return p; }
-};
-template <>
-struct Parts<0> {
-  const Part* p;
-  __device__ __forceinline__ const Part& get(int i) const { return p[i]; }
-};
-
-// Workgroup map entries: kind (3 bits), part (5 bits), tile or receiver
-// block (24 bits).  A launch's grid is 8 * L workgroups; workgroup b runs on
-// XCD b % 8, so the host lays out each XCD's list of work at b = 8 j + xcd.
-enum Kind : unsigned {
-  kNop = 0,
-  kStressFwd = 1,
-  kVelFwd = 2,
-  kRecord = 3,
-  kRevStress = 4,
-  kAdjVel = 5,
-  kAdjStress = 6,
-  kRevVel = 7,
-};
-constexpr int kMaxPartsTable = 31;
-__host__ __device__ inline unsigned wg_entry(unsigned kind, unsigned part, unsigned tile) {
-  return kind << 29 | part << 24 | tile;
-}
-
 // Boundary ring (Boundary.cu:17-41, utilities.cu:361-424): rows and columns
 // nPml-2 .. nPml+2 on each side of the interior, i.e. the band of width 5 of
 // the rectangle [nPml-2, nzA-nPml+1] x [nPml-2, nx-nPml+1].  Slot numbering is
@@ -263,62 +169,24 @@ __host__ __device__ inline int ring_slot(int z, int x, const Geo& g) {
   return -1;
 }
 
-// Ring layout [ring shot][held step][component][slot]; `s` counts from the
-// part's first shot.  The ring holds rnt consecutive steps: step it is row
-// it % rnt (all steps of the sweep when rnt = nSteps - 1, one checkpoint
-// segment otherwise).
-__device__ inline float* ring_ptr(float* ring, const Geo& g, int it, int comp, int s, int slot) {
-  const size_t row = ((size_t)g.rs0 + s) * g.rnt + (unsigned)it % (unsigned)g.rnt;
-  return ring + (row * 5 + comp) * (size_t)g.ringlen + slot;
-}
+// Ring layout [ring shot][held step][component][slot], components szz, sxz,
+// sxx, vz, vx.  The ring holds rnt consecutive steps: step it is row it % rnt
+// (all steps of the sweep when rnt = nSteps - 1, one checkpoint segment
+// otherwise).
 
 // Stencil loads and stores go through buffer resources: one scalar resource
 // per field of a part, the shot's byte offset in an SGPR (soffset) and the
-// cell's per-lane byte offset in a VGPR, with the z neighbours at immediate
-// offsets.  A wave's addresses then cost no per-lane 64-bit arithmetic.
+// cell's per-lane byte offset in a VGPR, z neighbours in one 16-byte load.  A wave's addresses then cost no per-lane 64-bit arithmetic.
 using Rsrc = __amdgpu_buffer_rsrc_t;
 __device__ __forceinline__ Rsrc rsrc(const float* p) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), (short)0, (int)0xffffffff,
                                            0x00020000);
 }
-// Per-lane byte offsets of a cell's stencil: z-2 (the z neighbours follow
-// 4 B apart) and the x neighbours x-2, x-1, x+1, x+2.
-struct Cell {
-  int zm2, xm2, xm1, xp1, xp2;
-};
-__device__ __forceinline__ Cell cell_of(unsigned bo, int nz) {
-  const int b = (int)bo, r = 4 * nz;
-  return Cell{b - 8, b - 2 * r, b - r, b + r, b + 2 * r};
-}
 __device__ __forceinline__ float ldb(Rsrc r, int so, int vo) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, vo, so, 0));
 }
-// A [shot][component][cell] array of one part: its buffer resource and the
-// bytes of one component.  Accessors take the shot's byte offset `so` and a
-// component.
-struct Arr {
-  Rsrc r;
-  int nb;
-};
-__device__ __forceinline__ Arr arr(const float* p, int nb) { return Arr{rsrc(p), nb}; }
-// z neighbour k (-2..2) and x neighbour k (-2, -1, 1, 2) of the cell
-__device__ __forceinline__ float lz(const Arr& A, int so, int comp, const Cell& c, int k) {
-  return ldb(A.r, so + comp * A.nb, c.zm2 + 4 * (k + 2));
-}
-__device__ __forceinline__ float lx(const Arr& A, int so, int comp, const Cell& c, int k) {
-  return ldb(A.r, so + comp * A.nb, k == -2 ? c.xm2 : k == -1 ? c.xm1 : k == 1 ? c.xp1 : c.xp2);
-}
-// z neighbours k0 .. k0+3 of the cell in one 16-byte load
-__device__ __forceinline__ f4 lz4(const Arr& A, int so, int comp, const Cell& c, int k0) {
-  return raw_load4(A.r, c.zm2 + 4 * (k0 + 2), so + comp * A.nb, 0);
-}
-__device__ __forceinline__ void st(const Arr& A, int so, int comp, const Cell& c, float v) {
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), A.r, c.zm2 + 8,
-                                        so + comp * A.nb, 0);
-}
-
 // Column of the calling thread in a tile whose first column is x0.  A
-// workgroup is 64 x tile_x threads, so each wave64 is one column: the column
+// workgroup is 64 threads deep, so each wave64 is one column: the column
 // is wave-uniform, and the x-direction C-PML coefficients and x branches it
 // selects are scalar.
 __device__ __forceinline__ int wave_col(int x0) {
@@ -334,1041 +202,7 @@ __device__ __forceinline__ float dad(float a, float b, float c, float d, float h
   return div1(-kC1 * (a - b) + kC2 * (c - d), h, rh);
 }
 
-// ------------------------------------------------------------------ forward
-// The kernels walk all shots of a part inside each thread, so model
-// parameters and C-PML coefficients are read once per cell.  Shots are taken
-// U at a time: every load of the U shots is issued before the first store,
-// so a wave keeps U shots' worth of reads in flight (the stores of shot s may
-// alias the loads of shot s+1 as far as the compiler knows, so it cannot
-// reorder them itself).
-
-// el_stress.cu:50-88 + add_source (utilities.cu:521-555) + from_bnd
-// (utilities.cu:361-391): the ring cells save sigma^it and v^it before the
-// update of step it.
-struct StressIn {
-  float vz0, vzm1, vzp1, vzm2, vzpx, vzp2x, vzmx;
-  float vx0, vxmx, vxpx, vxm2x, vxp1, vxp2, vxm1;
-  float szz, sxx, sxz;
-  float mvzz, mvxz, mvxx, mvzx;
-  int sz, sx;
-};
-
-template <int U>
-__device__ __forceinline__ void stress_fwd(const Part& P, int tile, int it) {
-  const Geo& g = P.g;
-  const int z = (tile % P.gzU) * kBZ + (int)threadIdx.x;
-  const int x = wave_col((tile / P.gzU) * (int)blockDim.y);
-  if (z < 2 || z > g.nzA - 3 || x < 2 || x > g.nx - 3) return;
-  const int nz = g.nz;
-  const long long i = (long long)x * nz + z;
-  const unsigned bo = (unsigned)i * 4u;  // byte offset of the cell in a per-shot array
-  const Cell C = cell_of(bo, nz);
-  const int Nb = (int)(g.N * 4);  // bytes per shot
-  const Arr W = arr(P.w, Nb);
-  const Arr M = arr(P.p, Nb);
-  const float lam = P.m.lam[i], mu = P.m.mu[i], amu = P.m.amu[i];
-  const double l2m = (double)lam + 2.0 * (double)mu;  // (d_Lambda + 2.0*d_Mu)
-  const bool pz = z < g.nPml || z > g.nzA - g.nPml - 1;
-  const bool px = x < g.nPml || x > g.nx - g.nPml - 1;
-  float bz = 0.f, az = 0.f, bzh = 0.f, azh = 0.f, bx = 0.f, ax = 0.f, bxh = 0.f, axh = 0.f;
-  Kdiv kz{}, kzh{}, kx{}, kxh{};
-  if (pz) {
-    bz = P.c.bz[z], az = P.c.az[z], kz = kdiv_of(P.c.Kz[z]);
-    bzh = P.c.bzh[z], azh = P.c.azh[z], kzh = kdiv_of(P.c.Kzh[z]);
-  }
-  if (px) {
-    bx = P.c.bx[x], ax = P.c.ax[x], kx = kdiv_of(P.c.Kx[x]);
-    bxh = P.c.bxh[x], axh = P.c.axh[x], kxh = kdiv_of(P.c.Kxh[x]);
-  }
-  const int slot = P.ring ? ring_slot(z, x, g) : -1;
-  const float dt = g.dt, dz = g.dz, dx = g.dx, rdz = g.rdz, rdx = g.rdx;
-  const double dt64 = (double)dt;
-  const int ns = g.ns;
-  for (int s0 = 0; s0 < ns; s0 += U) {
-    StressIn r[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = s0 + u;
-      if (s >= ns) break;
-      const int sw = s * kWaveComps * Nb, sm = s * kMemComps * Nb;
-      StressIn& q = r[u];
-      const f4 vzc = lz4(W, sw, kVz, C, -2), vxc = lz4(W, sw, kVx, C, -1);
-      q.vzm2 = vzc[0], q.vzm1 = vzc[1], q.vz0 = vzc[2], q.vzp1 = vzc[3];
-      q.vzpx = lx(W, sw, kVz, C, 1), q.vzp2x = lx(W, sw, kVz, C, 2), q.vzmx = lx(W, sw, kVz, C, -1);
-      q.vxm1 = vxc[0], q.vx0 = vxc[1], q.vxp1 = vxc[2], q.vxp2 = vxc[3];
-      q.vxmx = lx(W, sw, kVx, C, -1), q.vxpx = lx(W, sw, kVx, C, 1), q.vxm2x = lx(W, sw, kVx, C, -2);
-      q.szz = lz(W, sw, kSzz, C, 0), q.sxx = lz(W, sw, kSxx, C, 0), q.sxz = lz(W, sw, kSxz, C, 0);
-      if (pz) q.mvzz = lz(M, sm, kMvzz, C, 0), q.mvxz = lz(M, sm, kMvxz, C, 0);
-      if (px) q.mvxx = lz(M, sm, kMvxx, C, 0), q.mvzx = lz(M, sm, kMvzx, C, 0);
-      q.sz = P.src.zx[2 * s], q.sx = P.src.zx[2 * s + 1];
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = s0 + u;
-      if (s >= ns) break;
-      const int sw = s * kWaveComps * Nb, sm = s * kMemComps * Nb;
-      const StressIn& q = r[u];
-      float dvz_dz = dfw(q.vz0, q.vzm1, q.vzp1, q.vzm2, dz, rdz);
-      float dvx_dx = dfw(q.vx0, q.vxmx, q.vxpx, q.vxm2x, dx, rdx);
-      if (pz) {
-        const float mm = bz * q.mvzz + az * dvz_dz;
-        st(M, sm, kMvzz, C, mm);
-        dvz_dz = kdiv(dvz_dz, kz) + mm;
-      }
-      if (px) {
-        const float mm = bx * q.mvxx + ax * dvx_dx;
-        st(M, sm, kMvxx, C, mm);
-        dvx_dx = kdiv(dvx_dx, kx) + mm;
-      }
-      float szz = q.szz, sxx = q.sxx, sxz = q.sxz;
-      if (slot >= 0) {
-        *ring_ptr(P.ring, g, it, 0, s, slot) = szz;
-        *ring_ptr(P.ring, g, it, 1, s, slot) = sxz;
-        *ring_ptr(P.ring, g, it, 2, s, slot) = sxx;
-        *ring_ptr(P.ring, g, it, 3, s, slot) = q.vz0;
-        *ring_ptr(P.ring, g, it, 4, s, slot) = q.vx0;
-      }
-      szz = (float)((double)szz + (l2m * (double)dvz_dz + (double)(lam * dvx_dx)) * dt64);
-      sxx = (float)((double)sxx + ((double)(lam * dvz_dz) + l2m * (double)dvx_dx) * dt64);
-      float dvx_dz = dfw(q.vxp1, q.vx0, q.vxp2, q.vxm1, dz, rdz);
-      float dvz_dx = dfw(q.vzpx, q.vz0, q.vzp2x, q.vzmx, dx, rdx);
-      if (pz) {
-        const float mm = bzh * q.mvxz + azh * dvx_dz;
-        st(M, sm, kMvxz, C, mm);
-        dvx_dz = kdiv(dvx_dz, kzh) + mm;
-      }
-      if (px) {
-        const float mm = bxh * q.mvzx + axh * dvz_dx;
-        st(M, sm, kMvzx, C, mm);
-        dvz_dx = kdiv(dvz_dx, kxh) + mm;
-      }
-      sxz = sxz + amu * (dvx_dz + dvz_dx) * dt;
-      if (z == q.sz && x == q.sx) {
-        // add_source: szz += scale*amp*dt*gauss (float), sxx += RSXXZZ*scale*amp*dt*gauss
-        // (double); the 9x9 Gaussian is 1 at the centre and 0 elsewhere in FP32
-        const float amp = P.src.amp[(size_t)s * g.nSteps + it];
-        szz = szz + kSrcScale * amp * dt;
-        sxx = (float)((double)sxx + kRS * (double)kSrcScale * (double)amp * dt64);
-      }
-      st(W, sw, kSzz, C, szz);
-      st(W, sw, kSxx, C, sxx);
-      st(W, sw, kSxz, C, sxz);
-    }
-  }
-}
-
-// el_velocity.cu:45-82.  x-PML test is `x > nx - nPml` (el_velocity.cu:56,71).
-// With an illumination buffer, the part's sum over shots of vz^2 + vx^2 is
-// added to it (forward illumination; no reference counterpart).
-struct VelIn {
-  float szz0, szzp1, szzp2, szzm1;
-  float sxz0, sxzmx, sxzpx, sxzm2x, sxzm1, sxzp1, sxzm2;
-  float sxxpx, sxx0, sxxp2x, sxxmx;
-  float mszz, msxzz, msxzx, msxx;
-  float vz, vx;
-};
-
-template <int U>
-__device__ __forceinline__ void vel_fwd(const Part& P, int tile) {
-  const Geo& g = P.g;
-  const int z = (tile % P.gzU) * kBZ + (int)threadIdx.x;
-  const int x = wave_col((tile / P.gzU) * (int)blockDim.y);
-  if (z < 2 || z > g.nzA - 3 || x < 2 || x > g.nx - 3) return;
-  const int nz = g.nz;
-  const long long i = (long long)x * nz + z;
-  const unsigned bo = (unsigned)i * 4u;  // byte offset of the cell in a per-shot array
-  const Cell C = cell_of(bo, nz);
-  const int Nb = (int)(g.N * 4);  // bytes per shot
-  const Arr W = arr(P.w, Nb);
-  const Arr M = arr(P.p, Nb);
-  const float ba = P.m.ba[i], bb = P.m.bb[i];
-  const bool pz = z < g.nPml || z > g.nzA - g.nPml - 1;
-  const bool px = x < g.nPml || x > g.nx - g.nPml;
-  float bz = 0.f, az = 0.f, bzh = 0.f, azh = 0.f, bx = 0.f, ax = 0.f, bxh = 0.f, axh = 0.f;
-  Kdiv kz{}, kzh{}, kx{}, kxh{};
-  if (pz) {
-    bz = P.c.bz[z], az = P.c.az[z], kz = kdiv_of(P.c.Kz[z]);
-    bzh = P.c.bzh[z], azh = P.c.azh[z], kzh = kdiv_of(P.c.Kzh[z]);
-  }
-  if (px) {
-    bx = P.c.bx[x], ax = P.c.ax[x], kx = kdiv_of(P.c.Kx[x]);
-    bxh = P.c.bxh[x], axh = P.c.axh[x], kxh = kdiv_of(P.c.Kxh[x]);
-  }
-  const float dt = g.dt, dz = g.dz, dx = g.dx, rdz = g.rdz, rdx = g.rdx;
-  const int ns = g.ns;
-  float il = 0.f;  // illumination of this part's shots
-  for (int s0 = 0; s0 < ns; s0 += U) {
-    VelIn r[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = s0 + u;
-      if (s >= ns) break;
-      const int sw = s * kWaveComps * Nb, sm = s * kMemComps * Nb;
-      VelIn& q = r[u];
-      const f4 szc = lz4(W, sw, kSzz, C, -1), sxc = lz4(W, sw, kSxz, C, -2);
-      q.szzm1 = szc[0], q.szz0 = szc[1], q.szzp1 = szc[2], q.szzp2 = szc[3];
-      q.sxzm2 = sxc[0], q.sxzm1 = sxc[1], q.sxz0 = sxc[2], q.sxzp1 = sxc[3];
-      q.sxzmx = lx(W, sw, kSxz, C, -1), q.sxzpx = lx(W, sw, kSxz, C, 1), q.sxzm2x = lx(W, sw, kSxz, C, -2);
-      q.sxxpx = lx(W, sw, kSxx, C, 1), q.sxx0 = lz(W, sw, kSxx, C, 0), q.sxxp2x = lx(W, sw, kSxx, C, 2), q.sxxmx = lx(W, sw, kSxx, C, -1);
-      if (pz) q.mszz = lz(M, sm, kMszz, C, 0), q.msxzz = lz(M, sm, kMsxzz, C, 0);
-      if (px) q.msxzx = lz(M, sm, kMsxzx, C, 0), q.msxx = lz(M, sm, kMsxx, C, 0);
-      q.vz = lz(W, sw, kVz, C, 0), q.vx = lz(W, sw, kVx, C, 0);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = s0 + u;
-      if (s >= ns) break;
-      const int sw = s * kWaveComps * Nb, sm = s * kMemComps * Nb;
-      const VelIn& q = r[u];
-      float dszz_dz = dfw(q.szzp1, q.szz0, q.szzp2, q.szzm1, dz, rdz);
-      float dsxz_dx = dfw(q.sxz0, q.sxzmx, q.sxzpx, q.sxzm2x, dx, rdx);
-      if (pz) {
-        const float mm = bzh * q.mszz + azh * dszz_dz;
-        st(M, sm, kMszz, C, mm);
-        dszz_dz = kdiv(dszz_dz, kzh) + mm;
-      }
-      if (px) {
-        const float mm = bx * q.msxzx + ax * dsxz_dx;
-        st(M, sm, kMsxzx, C, mm);
-        dsxz_dx = kdiv(dsxz_dx, kx) + mm;
-      }
-      const float vz = q.vz + (dszz_dz + dsxz_dx) * ba * dt;
-      float dsxz_dz = dfw(q.sxz0, q.sxzm1, q.sxzp1, q.sxzm2, dz, rdz);
-      float dsxx_dx = dfw(q.sxxpx, q.sxx0, q.sxxp2x, q.sxxmx, dx, rdx);
-      if (pz) {
-        const float mm = bz * q.msxzz + az * dsxz_dz;
-        st(M, sm, kMsxzz, C, mm);
-        dsxz_dz = kdiv(dsxz_dz, kz) + mm;
-      }
-      if (px) {
-        const float mm = bxh * q.msxx + axh * dsxx_dx;
-        st(M, sm, kMsxx, C, mm);
-        dsxx_dx = kdiv(dsxx_dx, kxh) + mm;
-      }
-      const float vx = q.vx + (dsxz_dz + dsxx_dx) * bb * dt;
-      st(W, sw, kVz, C, vz);
-      st(W, sw, kVx, C, vx);
-      il += vz * vz + vx * vx;
-    }
-  }
-  if (P.illum) P.illum[i] += il;
-}
-
-// recording (utilities.cu:557-567): szz + RSXXZZ sxx (a double sum rounded to
-// FP32) at each receiver of the part, written to row it+1 of the seismograms;
-// one receiver per thread of the workgroup.
-__device__ __forceinline__ void record(const Part& P, int blk, int it) {
-  const int per = (int)(blockDim.x * blockDim.y);
-  const int r = blk * per + (int)(threadIdx.y * blockDim.x + threadIdx.x);
-  if (r >= P.nrec) return;
-  const Geo& g = P.g;
-  const int z = P.rec[3 * r], x = P.rec[3 * r + 1], s = P.rec[3 * r + 2] - g.s0;
-  const float* w = P.w + (size_t)s * kWaveComps * g.N + (long long)x * g.nz + z;
-  P.syn[(size_t)(it + 1) * g.R + r] = (float)((double)w[kSzz * g.N] + kRS * (double)w[kSxx * g.N]);
-}
-
-// ------------------------------------------------------------------ backward
-// Reverse-time re-materialisation (el_velocity.cu:84-117 with isFor = false)
-// fused with the ring restore of v (to_bnd, utilities.cu:394-424) and the
-// density-gradient accumulation.  The thread domain is the ring rectangle;
-// interior cells update, ring cells take the stored values.
-// acc_a += vz_adj (dszz/dz + dsxz/dx), acc_b += vx_adj (dsxz/dz + dsxx/dx).
-struct RevVelIn {
-  float szzp1, szz0, szzp2, szzm1;
-  float sxz0, sxzmx, sxzpx, sxzm2x, sxzm1, sxzp1, sxzm2;
-  float sxxpx, sxx0, sxxp2x, sxxmx;
-  float avz, avx, vz, vx;
-};
-
-template <int U>
-__device__ __forceinline__ void rev_vel(const Part& P, int tile, int it) {
-  const Geo& g = P.g;
-  const int z = (tile % P.gzR) * kBZ + (int)threadIdx.x + (g.nPml - 2);
-  const int x = wave_col((tile / P.gzR) * (int)blockDim.y) + (g.nPml - 2);
-  if (z > g.nzA - g.nPml + 1 || x > g.nx - g.nPml + 1) return;
-  const bool in = z >= g.nPml && z <= g.nzA - 1 - g.nPml && x >= g.nPml && x <= g.nx - 1 - g.nPml;
-  const int slot = ring_slot(z, x, g);
-  if (!in && slot < 0) return;
-  const int nz = g.nz;
-  const long long i = (long long)x * nz + z;
-  const unsigned bo = (unsigned)i * 4u;  // byte offset of the cell in a per-shot array
-  const Cell C = cell_of(bo, nz);
-  const int Nb = (int)(g.N * 4);  // bytes per shot
-  const Arr W = arr(P.w, Nb);
-  const Arr A = arr(P.a, Nb);
-  const float ba = P.m.ba[i], bb = P.m.bb[i];
-  const float dt = g.dt, dz = g.dz, dx = g.dx, rdz = g.rdz, rdx = g.rdx;
-  const int ns = g.ns;
-  float ga = 0.f, gb = 0.f;
-  for (int s0 = 0; s0 < ns; s0 += U) {
-    RevVelIn r[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = s0 + u;
-      if (s >= ns) break;
-      const int sw = s * kWaveComps * Nb;
-      RevVelIn& q = r[u];
-      if (in) {
-        const f4 szc = lz4(W, sw, kSzz, C, -1), sxc = lz4(W, sw, kSxz, C, -2);
-        q.szzm1 = szc[0], q.szz0 = szc[1], q.szzp1 = szc[2], q.szzp2 = szc[3];
-        q.sxzm2 = sxc[0], q.sxzm1 = sxc[1], q.sxz0 = sxc[2], q.sxzp1 = sxc[3];
-        q.sxzmx = lx(W, sw, kSxz, C, -1), q.sxzpx = lx(W, sw, kSxz, C, 1), q.sxzm2x = lx(W, sw, kSxz, C, -2);
-        q.sxxpx = lx(W, sw, kSxx, C, 1), q.sxx0 = lz(W, sw, kSxx, C, 0), q.sxxp2x = lx(W, sw, kSxx, C, 2), q.sxxmx = lx(W, sw, kSxx, C, -1);
-        q.avz = lz(A, sw, kVz, C, 0), q.avx = lz(A, sw, kVx, C, 0);
-      }
-      if (slot < 0) {
-        q.vz = lz(W, sw, kVz, C, 0), q.vx = lz(W, sw, kVx, C, 0);
-      } else {
-        q.vz = *ring_ptr(P.ring, g, it, 3, s, slot);
-        q.vx = *ring_ptr(P.ring, g, it, 4, s, slot);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = s0 + u;
-      if (s >= ns) break;
-      const int sw = s * kWaveComps * Nb;
-      const RevVelIn& q = r[u];
-      float vz = q.vz, vx = q.vx;
-      if (in) {
-        const float dszz_dz = dfw(q.szzp1, q.szz0, q.szzp2, q.szzm1, dz, rdz);
-        const float dsxz_dx = dfw(q.sxz0, q.sxzmx, q.sxzpx, q.sxzm2x, dx, rdx);
-        const float dsxz_dz = dfw(q.sxz0, q.sxzm1, q.sxzp1, q.sxzm2, dz, rdz);
-        const float dsxx_dx = dfw(q.sxxpx, q.sxx0, q.sxxp2x, q.sxxmx, dx, rdx);
-        const float fz = dszz_dz + dsxz_dx, fx = dsxz_dz + dsxx_dx;
-        ga += q.avz * fz;
-        gb += q.avx * fx;
-        if (slot < 0) {
-          vz = vz - fz * ba * dt;
-          vx = vx - fx * bb * dt;
-        }
-      }
-      st(W, sw, kVz, C, vz);
-      st(W, sw, kVx, C, vx);
-    }
-  }
-  if (in) {
-    P.acc[3 * g.N + i] += ga;
-    P.acc[4 * g.N + i] += gb;
-  }
-}
-
-// el_stress.cu:90-131 (isFor = false) preceded by add_source(-) and followed
-// by the ring restore of sigma.  acc_l += (szz_adj + sxx_adj)(dvz/dz + dvx/dx),
-// acc_m += szz_adj dvz/dz + sxx_adj dvx/dx, acc_s += sxz_adj (dvx/dz + dvz/dx).
-struct RevStressIn {
-  float vz0, vzm1, vzp1, vzm2, vzpx, vzp2x, vzmx;
-  float vx0, vxmx, vxpx, vxm2x, vxp1, vxp2, vxm1;
-  float aszz, asxx, asxz;
-  float szz, sxx, sxz;
-  int sz, sx;
-};
-
-template <int U>
-__device__ __forceinline__ void rev_stress(const Part& P, int tile, int it) {
-  const Geo& g = P.g;
-  const int z = (tile % P.gzR) * kBZ + (int)threadIdx.x + (g.nPml - 2);
-  const int x = wave_col((tile / P.gzR) * (int)blockDim.y) + (g.nPml - 2);
-  if (z > g.nzA - g.nPml + 1 || x > g.nx - g.nPml + 1) return;
-  const bool in = z >= g.nPml && z <= g.nzA - 1 - g.nPml && x >= g.nPml && x <= g.nx - 1 - g.nPml;
-  const int slot = ring_slot(z, x, g);
-  if (!in && slot < 0) return;
-  const int nz = g.nz;
-  const long long i = (long long)x * nz + z;
-  const unsigned bo = (unsigned)i * 4u;  // byte offset of the cell in a per-shot array
-  const Cell C = cell_of(bo, nz);
-  const int Nb = (int)(g.N * 4);  // bytes per shot
-  const Arr W = arr(P.w, Nb);
-  const Arr A = arr(P.a, Nb);
-  const float lam = P.m.lam[i], mu = P.m.mu[i], amu = P.m.amu[i];
-  const double l2m = (double)lam + 2.0 * (double)mu;
-  const float dt = g.dt, dz = g.dz, dx = g.dx, rdz = g.rdz, rdx = g.rdx;
-  const double dt64 = (double)dt;
-  const int ns = g.ns;
-  float gl = 0.f, gm = 0.f, gs = 0.f;
-  for (int s0 = 0; s0 < ns; s0 += U) {
-    RevStressIn r[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = s0 + u;
-      if (s >= ns) break;
-      const int sw = s * kWaveComps * Nb;
-      RevStressIn& q = r[u];
-      if (in) {
-        const f4 vzc = lz4(W, sw, kVz, C, -2), vxc = lz4(W, sw, kVx, C, -1);
-        q.vzm2 = vzc[0], q.vzm1 = vzc[1], q.vz0 = vzc[2], q.vzp1 = vzc[3];
-        q.vzpx = lx(W, sw, kVz, C, 1), q.vzp2x = lx(W, sw, kVz, C, 2), q.vzmx = lx(W, sw, kVz, C, -1);
-        q.vxm1 = vxc[0], q.vx0 = vxc[1], q.vxp1 = vxc[2], q.vxp2 = vxc[3];
-        q.vxmx = lx(W, sw, kVx, C, -1), q.vxpx = lx(W, sw, kVx, C, 1), q.vxm2x = lx(W, sw, kVx, C, -2);
-        q.aszz = lz(A, sw, kSzz, C, 0), q.asxx = lz(A, sw, kSxx, C, 0), q.asxz = lz(A, sw, kSxz, C, 0);
-      }
-      if (slot < 0) {
-        q.szz = lz(W, sw, kSzz, C, 0), q.sxx = lz(W, sw, kSxx, C, 0), q.sxz = lz(W, sw, kSxz, C, 0);
-        q.sz = P.src.zx[2 * s], q.sx = P.src.zx[2 * s + 1];
-      } else {
-        q.szz = *ring_ptr(P.ring, g, it, 0, s, slot);
-        q.sxz = *ring_ptr(P.ring, g, it, 1, s, slot);
-        q.sxx = *ring_ptr(P.ring, g, it, 2, s, slot);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = s0 + u;
-      if (s >= ns) break;
-      const int sw = s * kWaveComps * Nb;
-      const RevStressIn& q = r[u];
-      float szz = q.szz, sxx = q.sxx, sxz = q.sxz;
-      if (in) {
-        const float dvz_dz = dfw(q.vz0, q.vzm1, q.vzp1, q.vzm2, dz, rdz);
-        const float dvx_dx = dfw(q.vx0, q.vxmx, q.vxpx, q.vxm2x, dx, rdx);
-        const float dvx_dz = dfw(q.vxp1, q.vx0, q.vxp2, q.vxm1, dz, rdz);
-        const float dvz_dx = dfw(q.vzpx, q.vz0, q.vzp2x, q.vzmx, dx, rdx);
-        gl += (q.aszz + q.asxx) * (dvz_dz + dvx_dx);
-        gm += q.aszz * dvz_dz + q.asxx * dvx_dx;
-        gs += q.asxz * (dvx_dz + dvz_dx);
-        if (slot < 0) {
-          if (z == q.sz && x == q.sx) {
-            const float amp = P.src.amp[(size_t)s * g.nSteps + it];
-            szz = szz - kSrcScale * amp * dt;
-            sxx = (float)((double)sxx - kRS * (double)kSrcScale * (double)amp * dt64);
-          }
-          szz = (float)((double)szz - (l2m * (double)dvz_dz + (double)(lam * dvx_dx)) * dt64);
-          sxx = (float)((double)sxx - ((double)(lam * dvz_dz) + l2m * (double)dvx_dx) * dt64);
-          sxz = sxz - amu * (dvx_dz + dvz_dx) * dt;
-        }
-      }
-      st(W, sw, kSzz, C, szz);
-      st(W, sw, kSxx, C, sxx);
-      st(W, sw, kSxz, C, sxz);
-    }
-  }
-  if (in) {
-    P.acc[i] += gl;
-    P.acc[g.N + i] += gm;
-    P.acc[2 * g.N + i] += gs;
-  }
-}
-
-// el_velocity_adj.cu:22-108, plus source_grad (utilities.cu:582-593) for step
-// `it` < nSteps-1 (the adjoint stress it reads is not touched by this update).
-// The C-PML memory terms a*dpsi are evaluated only where a != 0; elsewhere
-// they are exactly zero in the reference as well, and adding a zero leaves
-// the sum unchanged.
-struct AdjVelIn {
-  float szz0, szzpx, szzp2x, szzmx, szzp1, szzp2, szzm1;
-  float sxx0, sxxpx, sxxp2x, sxxmx, sxxp1, sxxp2, sxxm1;
-  float sxz0, sxzm1, sxzp1, sxzm2, sxzmx, sxzpx, sxzm2x;
-  float q1[4], q2[4], q3[4], q4[4];  // vxx (x), vxz (z), vzz (z), vzx (x) stencils
-  float m_sxx, m_sxzz, m_sxzx, m_szz;
-  float vx, vz;
-  int sz, sx;
-};
-
-template <int U>
-__device__ __forceinline__ void adj_vel(const Part& P, int tile, int it) {
-  const Geo& g = P.g;
-  const int z = (tile % P.gzU) * kBZ + (int)threadIdx.x;
-  const int x = wave_col((tile / P.gzU) * (int)blockDim.y);
-  if (z < 2 || z > g.nzA - 3 || x < 2 || x > g.nx - 3) return;
-  const int nz = g.nz;
-  const long long i = (long long)x * nz + z;
-  const unsigned bo = (unsigned)i * 4u;  // byte offset of the cell in a per-shot array
-  const Cell C = cell_of(bo, nz);
-  const int Nb = (int)(g.N * 4);  // bytes per shot
-  const Arr A = arr(P.a, Nb);
-  const Arr M = arr(P.p, Nb);
-  const float lam = P.m.lam[i], mu = P.m.mu[i], amu = P.m.amu[i], ba = P.m.ba[i], bb = P.m.bb[i];
-  const double l2m = (double)lam + 2.0 * (double)mu;
-  const bool pz = z < g.nPml || z > g.nzA - g.nPml - 1;
-  const bool px = x < g.nPml || x > g.nx - g.nPml - 1;
-  const float ax = P.c.ax[x], bx = P.c.bx[x], axh = P.c.axh[x], bxh = P.c.bxh[x];
-  const float az = P.c.az[z], bz = P.c.bz[z], azh = P.c.azh[z], bzh = P.c.bzh[z];
-  const Kdiv kx = kdiv_of(P.c.Kx[x]), kz = kdiv_of(P.c.Kz[z]);
-  const float amu_kzh = kdiv(amu, kdiv_of(P.c.Kzh[z]));  // d_ave_Mu / d_K_z_half
-  const float amu_kxh = kdiv(amu, kdiv_of(P.c.Kxh[x]));  // d_ave_Mu / d_K_x_half
-  const float dt = g.dt, dz = g.dz, dx = g.dx, rdz = g.rdz, rdx = g.rdx;
-  const double dt64 = (double)dt;
-  const int ns = g.ns;
-  const bool stf = it < g.nSteps - 1 && P.stf_grad;
-  for (int s0 = 0; s0 < ns; s0 += U) {
-    AdjVelIn r[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = s0 + u;
-      if (s >= ns) break;
-      const int sw = s * kWaveComps * Nb, sm = s * kMemComps * Nb;
-      AdjVelIn& q = r[u];
-      const f4 szc = lz4(A, sw, kSzz, C, -1), sxc = lz4(A, sw, kSxx, C, -1), sxzc = lz4(A, sw, kSxz, C, -2);
-      q.szzm1 = szc[0], q.szz0 = szc[1], q.szzp1 = szc[2], q.szzp2 = szc[3];
-      q.szzpx = lx(A, sw, kSzz, C, 1), q.szzp2x = lx(A, sw, kSzz, C, 2), q.szzmx = lx(A, sw, kSzz, C, -1);
-      q.sxxm1 = sxc[0], q.sxx0 = sxc[1], q.sxxp1 = sxc[2], q.sxxp2 = sxc[3];
-      q.sxxpx = lx(A, sw, kSxx, C, 1), q.sxxp2x = lx(A, sw, kSxx, C, 2), q.sxxmx = lx(A, sw, kSxx, C, -1);
-      q.sxzm2 = sxzc[0], q.sxzm1 = sxzc[1], q.sxz0 = sxzc[2], q.sxzp1 = sxzc[3];
-      q.sxzmx = lx(A, sw, kSxz, C, -1), q.sxzpx = lx(A, sw, kSxz, C, 1), q.sxzm2x = lx(A, sw, kSxz, C, -2);
-      if (ax != 0.f) {  // psi_vxx at x+1, x, x+2, x-1
-        q.q1[0] = lx(M, sm, kMvxx, C, 1), q.q1[1] = lz(M, sm, kMvxx, C, 0), q.q1[2] = lx(M, sm, kMvxx, C, 2), q.q1[3] = lx(M, sm, kMvxx, C, -1);
-      }
-      if (azh != 0.f) {  // psi_vxz at z, z-1, z+1, z-2
-        const f4 t = lz4(M, sm, kMvxz, C, -2);
-        q.q2[0] = t[2], q.q2[1] = t[1], q.q2[2] = t[3], q.q2[3] = t[0];
-      }
-      if (az != 0.f) {  // psi_vzz at z+1, z, z+2, z-1
-        const f4 t = lz4(M, sm, kMvzz, C, -1);
-        q.q3[0] = t[2], q.q3[1] = t[1], q.q3[2] = t[3], q.q3[3] = t[0];
-      }
-      if (axh != 0.f) {  // psi_vzx at x, x-1, x+1, x-2
-        q.q4[0] = lz(M, sm, kMvzx, C, 0), q.q4[1] = lx(M, sm, kMvzx, C, -1), q.q4[2] = lx(M, sm, kMvzx, C, 1), q.q4[3] = lx(M, sm, kMvzx, C, -2);
-      }
-      if (px) q.m_sxx = lz(M, sm, kMsxx, C, 0), q.m_sxzx = lz(M, sm, kMsxzx, C, 0);
-      if (pz) q.m_sxzz = lz(M, sm, kMsxzz, C, 0), q.m_szz = lz(M, sm, kMszz, C, 0);
-      q.vx = lz(A, sw, kVx, C, 0), q.vz = lz(A, sw, kVz, C, 0);
-      q.sz = P.src.zx[2 * s], q.sx = P.src.zx[2 * s + 1];
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = s0 + u;
-      if (s >= ns) break;
-      const int sw = s * kWaveComps * Nb, sm = s * kMemComps * Nb;
-      const AdjVelIn& q = r[u];
-      if (stf && z == q.sz && x == q.sx)  // -(szz_adj + RSXXZZ sxx_adj) dt, double, stored as float
-        P.stf_grad[(size_t)s * g.nSteps + it] = (float)(-((double)q.szz0 + kRS * (double)q.sxx0) * dt64);
-      // update vx: a_x dpsi_xx/dx + lambda dszz/dx / K_x dt + (lambda + 2.0 mu) dsxx/dx / K_x dt
-      //            + a_z_half dpsi_xz/dz + ave_mu / K_z_half dsxz/dz dt
-      const float dszz_dx = dad(q.szzpx, q.szz0, q.szzp2x, q.szzmx, dx, rdx);
-      const float dsxx_dx = dad(q.sxxpx, q.sxx0, q.sxxp2x, q.sxxmx, dx, rdx);
-      const float dsxz_dz = dad(q.sxz0, q.sxzm1, q.sxzp1, q.sxzm2, dz, rdz);
-      float t = kdiv(lam * dszz_dx, kx) * dt;
-      if (ax != 0.f) t = ax * dad(q.q1[0], q.q1[1], q.q1[2], q.q1[3], dx, rdx) + t;
-      double S = (double)t + kdiv(l2m * (double)dsxx_dx, kx) * dt64;
-      if (azh != 0.f) S = S + (double)(azh * dad(q.q2[0], q.q2[1], q.q2[2], q.q2[3], dz, rdz));
-      S = S + (double)(amu_kzh * dsxz_dz * dt);
-      const float vx = (float)((double)q.vx + S);
-      st(A, sw, kVx, C, vx);
-      if (px) st(M, sm, kMsxx, C, bxh * q.m_sxx + bb * vx * dt);
-      if (pz) st(M, sm, kMsxzz, C, bz * q.m_sxzz + bb * vx * dt);
-      // update vz: a_z dpsi_zz/dz + (lambda + 2.0 mu) dszz/dz / K_z dt + lambda dsxx/dz / K_z dt
-      //            + a_x_half dpsi_zx/dx + ave_mu / K_x_half dsxz/dx dt
-      const float dszz_dz = dad(q.szzp1, q.szz0, q.szzp2, q.szzm1, dz, rdz);
-      const float dsxx_dz = dad(q.sxxp1, q.sxx0, q.sxxp2, q.sxxm1, dz, rdz);
-      const float dsxz_dx = dad(q.sxz0, q.sxzmx, q.sxzpx, q.sxzm2x, dx, rdx);
-      S = kdiv(l2m * (double)dszz_dz, kz) * dt64;
-      if (az != 0.f) S = (double)(az * dad(q.q3[0], q.q3[1], q.q3[2], q.q3[3], dz, rdz)) + S;
-      S = S + (double)(kdiv(lam * dsxx_dz, kz) * dt);
-      if (axh != 0.f) S = S + (double)(axh * dad(q.q4[0], q.q4[1], q.q4[2], q.q4[3], dx, rdx));
-      S = S + (double)(amu_kxh * dsxz_dx * dt);
-      const float vz = (float)((double)q.vz + S);
-      st(A, sw, kVz, C, vz);
-      if (px) st(M, sm, kMsxzx, C, bx * q.m_sxzx + ba * vz * dt);
-      if (pz) st(M, sm, kMszz, C, bzh * q.m_szz + ba * vz * dt);
-    }
-  }
-}
-
-// el_stress_adj.cu:22-104.  The 4 stress-side memory variables are updated
-// without PML gates in the reference; they are read only through a*dpsi
-// terms, i.e. where a != 0 (the C-PML layers) plus the 2-cell reach of the
-// stencil, so they are kept in that band (`zlive`/`xlive`) and nowhere else.
-// Residual injection folded into the update (res_injection,
-// utilities.cu:569-580): at a receiver's cell szz_adj += res and sxx_adj +=
-// RSXXZZ res before the update reads them (the update reads only its own
-// cell's stresses, so the sums are those of a separate injection pass).
-struct AdjStressIn {
-  float vz0, vzpx, vzp2x, vzmx, vzm1, vzp1, vzm2;
-  float vx0, vxp1, vxp2, vxm1, vxmx, vxpx, vxm2x;
-  float q1[4], q2[4], q3[4], q4[4];  // sxzx (x), sxzz (z), sxx (x), szz (z) stencils
-  float m_vzx, m_vxz, m_vxx, m_vzz;
-  float sxz, sxx, szz;
-};
-
-template <int U>
-__device__ __forceinline__ void adj_stress(const Part& P, int tile, int it) {
-  const Geo& g = P.g;
-  const int z = (tile % P.gzU) * kBZ + (int)threadIdx.x;
-  const int x = wave_col((tile / P.gzU) * (int)blockDim.y);
-  if (z < 2 || z > g.nzA - 3 || x < 2 || x > g.nx - 3) return;
-  const int nz = g.nz;
-  const long long i = (long long)x * nz + z;
-  const unsigned bo = (unsigned)i * 4u;  // byte offset of the cell in a per-shot array
-  const Cell C = cell_of(bo, nz);
-  const int Nb = (int)(g.N * 4);  // bytes per shot
-  const Arr A = arr(P.a, Nb);
-  const Arr M = arr(P.p, Nb);
-  const float lam = P.m.lam[i], mu = P.m.mu[i], amu = P.m.amu[i], ba = P.m.ba[i], bb = P.m.bb[i];
-  const double l2m = (double)lam + 2.0 * (double)mu;
-  const bool zlive = z <= g.nPml + 1 || z >= g.nzA - g.nPml - 2;
-  const bool xlive = x <= g.nPml + 1 || x >= g.nx - g.nPml - 2;
-  const float ax = P.c.ax[x], bx = P.c.bx[x], axh = P.c.axh[x], bxh = P.c.bxh[x];
-  const float az = P.c.az[z], bz = P.c.bz[z], azh = P.c.azh[z], bzh = P.c.bzh[z];
-  const Kdiv kx = kdiv_of(P.c.Kx[x]), kz = kdiv_of(P.c.Kz[z]);
-  const Kdiv kxh = kdiv_of(P.c.Kxh[x]), kzh = kdiv_of(P.c.Kzh[z]);
-  const float dt = g.dt, dz = g.dz, dx = g.dx, rdz = g.rdz, rdx = g.rdx;
-  const double dt64 = (double)dt;
-  const int ns = g.ns;
-  const bool inj_row = P.inj.res && z == P.inj.z;
-  const float* res_row = P.inj.res ? P.inj.res + (size_t)it * g.R : nullptr;
-  for (int s0 = 0; s0 < ns; s0 += U) {
-    AdjStressIn r[U];
-    float resv[U];
-    bool has[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = s0 + u;
-      resv[u] = 0.f;
-      has[u] = false;
-      if (s >= ns) break;
-      if (inj_row) {
-        const int k = P.inj.at[(size_t)(g.s0 + s) * g.nx + x];
-        if (k >= 0) {
-          resv[u] = res_row[k];
-          has[u] = true;
-        }
-      }
-      const int sw = s * kWaveComps * Nb, sm = s * kMemComps * Nb;
-      AdjStressIn& q = r[u];
-      const f4 vzc = lz4(A, sw, kVz, C, -2), vxc = lz4(A, sw, kVx, C, -1);
-      q.vzm2 = vzc[0], q.vzm1 = vzc[1], q.vz0 = vzc[2], q.vzp1 = vzc[3];
-      q.vzpx = lx(A, sw, kVz, C, 1), q.vzp2x = lx(A, sw, kVz, C, 2), q.vzmx = lx(A, sw, kVz, C, -1);
-      q.vxm1 = vxc[0], q.vx0 = vxc[1], q.vxp1 = vxc[2], q.vxp2 = vxc[3];
-      q.vxmx = lx(A, sw, kVx, C, -1), q.vxpx = lx(A, sw, kVx, C, 1), q.vxm2x = lx(A, sw, kVx, C, -2);
-      if (ax != 0.f) {  // psi_sxzx at x+1, x, x+2, x-1
-        q.q1[0] = lx(M, sm, kMsxzx, C, 1), q.q1[1] = lz(M, sm, kMsxzx, C, 0), q.q1[2] = lx(M, sm, kMsxzx, C, 2), q.q1[3] = lx(M, sm, kMsxzx, C, -1);
-      }
-      if (az != 0.f) {  // psi_sxzz at z+1, z, z+2, z-1
-        const f4 t = lz4(M, sm, kMsxzz, C, -1);
-        q.q2[0] = t[2], q.q2[1] = t[1], q.q2[2] = t[3], q.q2[3] = t[0];
-      }
-      if (axh != 0.f) {  // psi_sxx at x, x-1, x+1, x-2
-        q.q3[0] = lz(M, sm, kMsxx, C, 0), q.q3[1] = lx(M, sm, kMsxx, C, -1), q.q3[2] = lx(M, sm, kMsxx, C, 1), q.q3[3] = lx(M, sm, kMsxx, C, -2);
-      }
-      if (azh != 0.f) {  // psi_szz at z, z-1, z+1, z-2
-        const f4 t = lz4(M, sm, kMszz, C, -2);
-        q.q4[0] = t[2], q.q4[1] = t[1], q.q4[2] = t[3], q.q4[3] = t[0];
-      }
-      if (xlive) q.m_vzx = lz(M, sm, kMvzx, C, 0), q.m_vxx = lz(M, sm, kMvxx, C, 0);
-      if (zlive) q.m_vxz = lz(M, sm, kMvxz, C, 0), q.m_vzz = lz(M, sm, kMvzz, C, 0);
-      q.sxz = lz(A, sw, kSxz, C, 0), q.sxx = lz(A, sw, kSxx, C, 0), q.szz = lz(A, sw, kSzz, C, 0);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = s0 + u;
-      if (s >= ns) break;
-      const int sw = s * kWaveComps * Nb, sm = s * kMemComps * Nb;
-      const AdjStressIn& q = r[u];
-      // sxz += a_x dphi_xz_x/dx + dvz/dx / K_x ba dt + a_z dphi_xz_z/dz + dvx/dz / K_z bb dt
-      const float dvz_dx = dad(q.vzpx, q.vz0, q.vzp2x, q.vzmx, dx, rdx);
-      const float dvx_dz = dad(q.vxp1, q.vx0, q.vxp2, q.vxm1, dz, rdz);
-      float e = kdiv(dvz_dx, kx) * ba * dt;
-      if (ax != 0.f) e = ax * dad(q.q1[0], q.q1[1], q.q1[2], q.q1[3], dx, rdx) + e;
-      if (az != 0.f) e = e + az * dad(q.q2[0], q.q2[1], q.q2[2], q.q2[3], dz, rdz);
-      e = e + kdiv(dvx_dz, kz) * bb * dt;
-      const float sxz = q.sxz + e;
-      st(A, sw, kSxz, C, sxz);
-      if (xlive) st(M, sm, kMvzx, C, bxh * q.m_vzx + sxz * amu * dt);
-      if (zlive) st(M, sm, kMvxz, C, bzh * q.m_vxz + sxz * amu * dt);
-      const float dvx_dx = dad(q.vx0, q.vxmx, q.vxpx, q.vxm2x, dx, rdx);
-      const float dvz_dz = dad(q.vz0, q.vzm1, q.vzp1, q.vzm2, dz, rdz);
-      float sxx0 = q.sxx, szz0 = q.szz;
-      if (has[u]) {
-        szz0 = szz0 + resv[u];
-        sxx0 = (float)((double)sxx0 + kRS * (double)resv[u]);
-      }
-      // sxx += a_x_half dphi_xx/dx + bb dvx/dx / K_x_half dt; szz likewise in z
-      float t = kdiv(bb * dvx_dx, kxh) * dt;
-      if (axh != 0.f) t = axh * dad(q.q3[0], q.q3[1], q.q3[2], q.q3[3], dx, rdx) + t;
-      const float sxx = sxx0 + t;
-      t = kdiv(ba * dvz_dz, kzh) * dt;
-      if (azh != 0.f) t = azh * dad(q.q4[0], q.q4[1], q.q4[2], q.q4[3], dz, rdz) + t;
-      const float szz = szz0 + t;
-      st(A, sw, kSxx, C, sxx);
-      st(A, sw, kSzz, C, szz);
-      // psi_xx = b_x psi + lambda szz dt + (lambda + 2.0 mu) sxx dt;
-      // psi_zz = b_z psi + (lambda + 2.0 mu) szz dt + lambda sxx dt
-      if (xlive)
-        st(M, sm, kMvxx, C, (float)((double)(bx * q.m_vxx + lam * szz * dt) + l2m * (double)sxx * dt64));
-      if (zlive)
-        st(M, sm, kMvzz, C, (float)((double)(bz * q.m_vzz) + l2m * (double)szz * dt64 + (double)(lam * sxx * dt)));
-    }
-  }
-}
-
-// ------------------------------------------------------------ exact adjoint
-// No reference counterpart: the transpose of the forward time step
-// (el_stress_fwd, add_source, el_velocity_fwd, recording), taken operation by
-// operation, so that the gradient is the derivative of the discrete misfit
-// also where waves enter the C-PML and in zero-shear layers.  The adjoint
-// state keeps the reference's sign (the residual is injected with +, so it is
-// -dJ/d(state)) and the gradient sums keep the meaning of the reference
-// mode's, so k_finalize turns both into (lambda, mu, rho) gradients.
-//
-// A stencil difference f -> D f of the forward step becomes its transpose
-// acting on the coefficient-weighted adjoint, and a C-PML term
-// d~ = d / K + psi', psi' = b psi + a d becomes, for the adjoint P of psi,
-// d_adj = g / K + a (g + P), P <- b (g + P) (only where the forward updates
-// psi, with the forward's gates, including el_velocity.cu:56,71's
-// x > nx - nPml).  Each transposed update runs as two passes over the
-// update region: the first forms the weighted operands of every cell
-// (xt, zero outside the update region), the second applies the transposed
-// stencils to them.  The second pass of one update and the first of the next
-// touch only their own cell's adjoint, so they share a launch, and so does
-// the reverse re-materialisation step that reads the same forward field:
-//   k_exact_a(it): reverse velocity step it (v^{it+1} -> v^it from
-//     sigma^{it+1}), transposed stress update of step it+1 into v_adj,
-//     velocity operands of step it and the density sums from sigma^{it+1};
-//   k_exact_b(it): residual of sample it+1 (folded injection), transposed
-//     velocity update of step it into sigma_adj, stf gradient, stress
-//     operands of step it and the lambda / mu sums from v^it, reverse stress
-//     step it (sigma^{it+1} -> sigma^it from v^it).
-// Each reversal writes only its cell's own forward field, which the adjoint
-// half of its launch does not read.  xt holds two operand sets per shot
-// (slots 0-3: Azz, Axx, Axz, Azx of the stress update; 4-7: Bz, Bzx, Bxz, Bx
-// of the velocity update).  Outside the C-PML frame (cells whose row or
-// column is gated) Azx = Axz, Bzx = Bz and Bx = Bxz, so slots 3, 5 and 7 are
-// written and read only inside the frame, and a reader takes slots 2, 4 and 6
-// for neighbours outside it.
-__device__ __forceinline__ float pml_t(float g, const Kdiv& K, float a, float b, float& P) {
-  const float tot = g + P;
-  P = b * tot;
-  return kdiv(g, K) + a * tot;
-}
-// The transposed differences are written through dfw: for a stride st,
-// (D+)^T B at j = (c1 (B[j-st] - B[j]) - c2 (B[j-2st] - B[j+st])) / h and
-// (D-)^T B at j = (c1 (B[j] - B[j+st]) - c2 (B[j-st] - B[j+2st])) / h, for
-// D+ f = (c1 (f[k+1] - f[k]) - c2 (f[k+2] - f[k-1])) / h and
-// D- f = (c1 (f[k] - f[k-1]) - c2 (f[k+1] - f[k-2])) / h.
-
-// x neighbour k (-2..2) of the cell from operand slot `own` when the
-// neighbour lies in the C-PML frame (`f`), else from slot `base`; the slot
-// goes into the per-lane offset, so `f` may differ between lanes.
-__device__ __forceinline__ float lxf(const Arr& X, int sx, int own, int base, const Cell& C, int k,
-                                     bool f) {
-  const int v = k == 0 ? C.zm2 + 8 : k == -2 ? C.xm2 : k == -1 ? C.xm1 : k == 1 ? C.xp1 : C.xp2;
-  return ldb(X.r, sx, v + (f ? own : base) * X.nb);
-}
-
-// The cell of the calling thread: 64 x 4 tiles over the update region,
-// z fastest, in XCD bands (workgroup b runs on XCD b % 8, and XCD k takes
-// the k-th eighth of the tiles, so the columns a tile shares with its
-// neighbours stay in that XCD's L2).  The grid is 8 * ceil(tiles / 8)
-// workgroups of 64 x 4; false for threads outside the update region.
-__device__ __forceinline__ bool exact_cell(const Geo& g, int& z, int& x) {
-  const int gz = (g.nzA + kBZ - 1) / kBZ, gx = (g.nx + 3) / 4;
-  const int tiles = gz * gx, per = (tiles + 7) / 8;
-  const int b = (int)blockIdx.x, t = (b & 7) * per + (b >> 3);
-  if (t >= tiles) return false;
-  z = (t % gz) * kBZ + (int)threadIdx.x;
-  x = wave_col((t / gz) * 4);
-  return z >= 2 && z <= g.nzA - 3 && x >= 2 && x <= g.nx - 3;
-}
-
-__global__ __launch_bounds__(256) void k_exact_a(Part P, float* __restrict__ xt, int it, int first) {
-  const Geo& g = P.g;
-  int z, x;
-  if (!exact_cell(g, z, x)) return;
-  const int nz = g.nz;
-  const long long i = (long long)x * nz + z;
-  const bool in = z >= g.nPml && z <= g.nzA - 1 - g.nPml && x >= g.nPml && x <= g.nx - 1 - g.nPml;
-  const int slot = ring_slot(z, x, g);
-  const bool re = in || slot >= 0;  // the cell takes part in the reversal
-  const bool pz = z < g.nPml || z > g.nzA - g.nPml - 1;
-  const bool px = x < g.nPml || x > g.nx - g.nPml;  // el_velocity's gate
-  const Cell C = cell_of((unsigned)i * 4u, nz);
-  const int Nb = (int)(g.N * 4);
-  const Arr W = arr(P.w, Nb), A = arr(P.a, Nb), M = arr(P.p, Nb), X = arr(xt, Nb);
-  const float ba = P.m.ba[i], bb = P.m.bb[i];
-  const float dt = g.dt, dz = g.dz, dx = g.dx, rdz = g.rdz, rdx = g.rdx;
-  Kdiv kzh{}, kz{}, kx{}, kxh{};
-  float azh = 0.f, bzh = 0.f, az = 0.f, bz = 0.f, ax = 0.f, bx = 0.f, axh = 0.f, bxh = 0.f;
-  if (pz) {
-    kzh = kdiv_of(P.c.Kzh[z]), azh = P.c.azh[z], bzh = P.c.bzh[z];
-    kz = kdiv_of(P.c.Kz[z]), az = P.c.az[z], bz = P.c.bz[z];
-  }
-  if (px) {
-    kx = kdiv_of(P.c.Kx[x]), ax = P.c.ax[x], bx = P.c.bx[x];
-    kxh = kdiv_of(P.c.Kxh[x]), axh = P.c.axh[x], bxh = P.c.bxh[x];
-  }
-  float ga = 0.f, gb = 0.f;
-  for (int s = 0; s < g.ns; ++s) {
-    const int sw = s * kWaveComps * Nb, sm = s * kMemComps * Nb, sx = s * 8 * Nb;
-    // forward stresses sigma^{it+1} around the cell (interior cells)
-    float fz = 0.f, fx = 0.f;
-    if (in) {
-      const f4 szc = lz4(W, sw, kSzz, C, -1), sxc = lz4(W, sw, kSxz, C, -2);
-      const float sxzmx = lx(W, sw, kSxz, C, -1), sxzpx = lx(W, sw, kSxz, C, 1),
-                  sxzm2x = lx(W, sw, kSxz, C, -2);
-      const float sxxpx = lx(W, sw, kSxx, C, 1), sxx0 = lz(W, sw, kSxx, C, 0),
-                  sxxp2x = lx(W, sw, kSxx, C, 2), sxxmx = lx(W, sw, kSxx, C, -1);
-      const float dszz_dz = dfw(szc[2], szc[1], szc[3], szc[0], dz, rdz);
-      const float dsxz_dx = dfw(sxc[2], sxzmx, sxzpx, sxzm2x, dx, rdx);
-      const float dsxz_dz = dfw(sxc[2], sxc[1], sxc[3], sxc[0], dz, rdz);
-      const float dsxx_dx = dfw(sxxpx, sxx0, sxxp2x, sxxmx, dx, rdx);
-      fz = dszz_dz + dsxz_dx;
-      fx = dsxz_dz + dsxx_dx;
-    }
-    float wvz = 0.f, wvx = 0.f;
-    if (re) {
-      if (slot < 0) {
-        wvz = lz(W, sw, kVz, C, 0), wvx = lz(W, sw, kVx, C, 0);
-      } else {
-        wvz = *ring_ptr(P.ring, g, it, 3, s, slot);
-        wvx = *ring_ptr(P.ring, g, it, 4, s, slot);
-      }
-    }
-    float vz = lz(A, sw, kVz, C, 0), vx = lz(A, sw, kVx, C, 0);
-    if (!first) {
-      const f4 azz = lz4(X, sx, 0, C, -1);  // Azz at z-1 .. z+2
-      const f4 axz = lz4(X, sx, 2, C, -2);  // Axz at z-2 .. z+1
-      // Azx (slot 3 in the stress update's frame, else Axz)
-      auto fs = [&](int k) { return pz || x + k < g.nPml || x + k > g.nx - g.nPml - 1; };
-      const float azxm = lxf(X, sx, 3, 2, C, -1, fs(-1)), azx0 = lxf(X, sx, 3, 2, C, 0, fs(0)),
-                  azxm2 = lxf(X, sx, 3, 2, C, -2, fs(-2)), azxp = lxf(X, sx, 3, 2, C, 1, fs(1));
-      const float axx0 = lz(X, sx, 1, C, 0), axxp = lx(X, sx, 1, C, 1),
-                  axxm = lx(X, sx, 1, C, -1), axxp2 = lx(X, sx, 1, C, 2);
-      // (D-)^T Azz along z + (D+)^T Azx along x; (D-)^T Axx along x + (D+)^T Axz along z
-      vz = vz + (dfw(azz[1], azz[2], azz[0], azz[3], dz, rdz) + dfw(azxm, azx0, azxm2, azxp, dx, rdx));
-      vx = vx + (dfw(axx0, axxp, axxm, axxp2, dx, rdx) + dfw(axz[1], axz[2], axz[0], axz[3], dz, rdz));
-      st(A, sw, kVz, C, vz);
-      st(A, sw, kVx, C, vx);
-    }
-    const float gz = dt * ba * vz, gx = dt * bb * vx;
-    float oz = gz, ozx = gz, oxz = gx, ox = gx;
-    if (pz) {
-      float q = lz(M, sm, kMszz, C, 0);
-      oz = pml_t(gz, kzh, azh, bzh, q);
-      st(M, sm, kMszz, C, q);
-      q = lz(M, sm, kMsxzz, C, 0);
-      oxz = pml_t(gx, kz, az, bz, q);
-      st(M, sm, kMsxzz, C, q);
-    }
-    if (px) {
-      float q = lz(M, sm, kMsxzx, C, 0);
-      ozx = pml_t(gz, kx, ax, bx, q);
-      st(M, sm, kMsxzx, C, q);
-      q = lz(M, sm, kMsxx, C, 0);
-      ox = pml_t(gx, kxh, axh, bxh, q);
-      st(M, sm, kMsxx, C, q);
-    }
-    st(X, sx, 4, C, oz);
-    st(X, sx, 6, C, oxz);
-    if (pz || px) {  // the velocity update's frame
-      st(X, sx, 5, C, ozx);
-      st(X, sx, 7, C, ox);
-    }
-    if (in) {
-      ga += vz * fz;
-      gb += vx * fx;
-    }
-    if (re) {
-      if (slot < 0) {  // el_velocity.cu:84-117, isFor = false
-        wvz = wvz - fz * ba * dt;
-        wvx = wvx - fx * bb * dt;
-      }
-      st(W, sw, kVz, C, wvz);
-      st(W, sw, kVx, C, wvx);
-    }
-  }
-  if (in) {
-    P.acc[3 * g.N + i] += ga;
-    P.acc[4 * g.N + i] += gb;
-  }
-}
-
-__global__ __launch_bounds__(256) void k_exact_b(Part P, float* __restrict__ xt,
-                                                 const float* __restrict__ srcwin, int it) {
-  const Geo& g = P.g;
-  int z, x;
-  if (!exact_cell(g, z, x)) return;
-  const int nz = g.nz;
-  const long long i = (long long)x * nz + z;
-  const bool in = z >= g.nPml && z <= g.nzA - 1 - g.nPml && x >= g.nPml && x <= g.nx - 1 - g.nPml;
-  const int slot = ring_slot(z, x, g);
-  const bool re = in || slot >= 0;  // the cell takes part in the reversal
-  const bool pz = z < g.nPml || z > g.nzA - g.nPml - 1;
-  const bool px = x < g.nPml || x > g.nx - g.nPml - 1;  // el_stress's gate
-  const Cell C = cell_of((unsigned)i * 4u, nz);
-  const int Nb = (int)(g.N * 4);
-  const Arr W = arr(P.w, Nb), A = arr(P.a, Nb), M = arr(P.p, Nb), X = arr(xt, Nb);
-  const float lam = P.m.lam[i], mu = P.m.mu[i], amu = P.m.amu[i];
-  const double l2m64 = (double)lam + 2.0 * (double)mu;
-  const float l2m = (float)l2m64;
-  const float dt = g.dt, dz = g.dz, dx = g.dx, rdz = g.rdz, rdx = g.rdx;
-  const double dt64 = (double)dt;
-  Kdiv kz{}, kzh{}, kx{}, kxh{};
-  float az = 0.f, bz = 0.f, azh = 0.f, bzh = 0.f, ax = 0.f, bx = 0.f, axh = 0.f, bxh = 0.f;
-  if (pz) {
-    kz = kdiv_of(P.c.Kz[z]), az = P.c.az[z], bz = P.c.bz[z];
-    kzh = kdiv_of(P.c.Kzh[z]), azh = P.c.azh[z], bzh = P.c.bzh[z];
-  }
-  if (px) {
-    kx = kdiv_of(P.c.Kx[x]), ax = P.c.ax[x], bx = P.c.bx[x];
-    kxh = kdiv_of(P.c.Kxh[x]), axh = P.c.axh[x], bxh = P.c.bxh[x];
-  }
-  const bool inj_row = P.inj.res && z == P.inj.z;
-  const float* res_row = P.inj.res ? P.inj.res + (size_t)(it + 1) * g.R : nullptr;
-  float gl = 0.f, gm = 0.f, gs = 0.f;
-  for (int s = 0; s < g.ns; ++s) {
-    const int sw = s * kWaveComps * Nb, sm = s * kMemComps * Nb, sx = s * 8 * Nb;
-    const int zs = P.src.zx[2 * s], xs = P.src.zx[2 * s + 1];
-    // forward velocities v^it around the cell (interior cells)
-    float dvz_dz = 0.f, dvx_dx = 0.f, dvx_dz = 0.f, dvz_dx = 0.f;
-    if (in) {
-      const f4 vzc = lz4(W, sw, kVz, C, -2), vxc = lz4(W, sw, kVx, C, -1);
-      const float vzpx = lx(W, sw, kVz, C, 1), vzp2x = lx(W, sw, kVz, C, 2),
-                  vzmx = lx(W, sw, kVz, C, -1);
-      const float vxmx = lx(W, sw, kVx, C, -1), vxpx = lx(W, sw, kVx, C, 1),
-                  vxm2x = lx(W, sw, kVx, C, -2);
-      dvz_dz = dfw(vzc[2], vzc[1], vzc[3], vzc[0], dz, rdz);
-      dvx_dx = dfw(vxc[1], vxmx, vxpx, vxm2x, dx, rdx);
-      dvx_dz = dfw(vxc[2], vxc[1], vxc[3], vxc[0], dz, rdz);
-      dvz_dx = dfw(vzpx, vzc[2], vzp2x, vzmx, dx, rdx);
-    }
-    float wszz = 0.f, wsxx = 0.f, wsxz = 0.f;
-    if (re) {
-      if (slot < 0) {
-        wszz = lz(W, sw, kSzz, C, 0), wsxx = lz(W, sw, kSxx, C, 0), wsxz = lz(W, sw, kSxz, C, 0);
-      } else {
-        wszz = *ring_ptr(P.ring, g, it, 0, s, slot);
-        wsxz = *ring_ptr(P.ring, g, it, 1, s, slot);
-        wsxx = *ring_ptr(P.ring, g, it, 2, s, slot);
-      }
-    }
-    float szz = lz(A, sw, kSzz, C, 0), sxx = lz(A, sw, kSxx, C, 0), sxz = lz(A, sw, kSxz, C, 0);
-    if (inj_row) {
-      const int k = P.inj.at[(size_t)(g.s0 + s) * g.nx + x];
-      if (k >= 0) {
-        const float v = res_row[k];
-        szz = szz + v;
-        sxx = (float)((double)sxx + kRS * (double)v);
-      }
-    }
-    {
-      const f4 bzc = lz4(X, sx, 4, C, -2);   // Bz at z-2 .. z+1
-      const f4 bxzc = lz4(X, sx, 6, C, -1);  // Bxz at z-1 .. z+2
-      // Bzx and Bx (slots 5 and 7 in the velocity update's frame, else Bz and Bxz)
-      auto fv = [&](int k) { return pz || x + k < g.nPml || x + k > g.nx - g.nPml; };
-      const float bzx0 = lxf(X, sx, 5, 4, C, 0, fv(0)), bzxp = lxf(X, sx, 5, 4, C, 1, fv(1)),
-                  bzxm = lxf(X, sx, 5, 4, C, -1, fv(-1)), bzxp2 = lxf(X, sx, 5, 4, C, 2, fv(2));
-      const float bxm = lxf(X, sx, 7, 6, C, -1, fv(-1)), bx0 = lxf(X, sx, 7, 6, C, 0, fv(0)),
-                  bxm2 = lxf(X, sx, 7, 6, C, -2, fv(-2)), bxp = lxf(X, sx, 7, 6, C, 1, fv(1));
-      // (D+)^T Bz along z; (D-)^T Bzx along x + (D-)^T Bxz along z; (D+)^T Bx along x
-      szz = szz + dfw(bzc[1], bzc[2], bzc[0], bzc[3], dz, rdz);
-      sxz = sxz + (dfw(bzx0, bzxp, bzxm, bzxp2, dx, rdx) + dfw(bxzc[1], bxzc[2], bxzc[0], bxzc[3], dz, rdz));
-      sxx = sxx + dfw(bxm, bx0, bxm2, bxp, dx, rdx);
-    }
-    st(A, sw, kSzz, C, szz);
-    st(A, sw, kSxx, C, sxx);
-    st(A, sw, kSxz, C, sxz);
-    // d(szz, sxx)/d(stf) at the source: 1500^2 dt and the window (add_source)
-    if (P.stf_grad && z == zs && x == xs)
-      P.stf_grad[(size_t)s * g.nSteps + it] =
-          (float)(-(double)kSrcScale * dt64 * ((double)szz + kRS * (double)sxx) *
-                  (double)srcwin[it]);
-    const float Gzz = dt * (l2m * szz + lam * sxx);
-    const float Gxx = dt * (lam * szz + l2m * sxx);
-    const float Gs = dt * amu * sxz;
-    float ozz = Gzz, oxx = Gxx, oxz = Gs, ozx = Gs;
-    if (pz) {
-      float q = lz(M, sm, kMvzz, C, 0);
-      ozz = pml_t(Gzz, kz, az, bz, q);
-      st(M, sm, kMvzz, C, q);
-      q = lz(M, sm, kMvxz, C, 0);
-      oxz = pml_t(Gs, kzh, azh, bzh, q);
-      st(M, sm, kMvxz, C, q);
-    }
-    if (px) {
-      float q = lz(M, sm, kMvxx, C, 0);
-      oxx = pml_t(Gxx, kx, ax, bx, q);
-      st(M, sm, kMvxx, C, q);
-      q = lz(M, sm, kMvzx, C, 0);
-      ozx = pml_t(Gs, kxh, axh, bxh, q);
-      st(M, sm, kMvzx, C, q);
-    }
-    st(X, sx, 0, C, ozz);
-    st(X, sx, 1, C, oxx);
-    st(X, sx, 2, C, oxz);
-    if (pz || px) st(X, sx, 3, C, ozx);  // the stress update's frame
-    if (in) {
-      gl += (szz + sxx) * (dvz_dz + dvx_dx);
-      gm += szz * dvz_dz + sxx * dvx_dx;
-      gs += sxz * (dvx_dz + dvz_dx);
-    }
-    if (re) {
-      if (slot < 0) {  // add_source(-) then el_stress.cu:90-131, isFor = false
-        if (z == zs && x == xs) {
-          const float amp = P.src.amp[(size_t)s * g.nSteps + it];
-          wszz = wszz - kSrcScale * amp * dt;
-          wsxx = (float)((double)wsxx - kRS * (double)kSrcScale * (double)amp * dt64);
-        }
-        wszz = (float)((double)wszz - (l2m64 * (double)dvz_dz + (double)(lam * dvx_dx)) * dt64);
-        wsxx = (float)((double)wsxx - ((double)(lam * dvz_dz) + l2m64 * (double)dvx_dx) * dt64);
-        wsxz = wsxz - amu * (dvx_dz + dvz_dx) * dt;
-      }
-      st(W, sw, kSzz, C, wszz);
-      st(W, sw, kSxx, C, wsxx);
-      st(W, sw, kSxz, C, wsxz);
-    }
-  }
-  if (in) {
-    P.acc[i] += gl;
-    P.acc[g.N + i] += gm;
-    P.acc[2 * g.N + i] += gs;
-  }
-}
-
-// ------------------------------------------------------------ step kernels
-template <int NP>
-__device__ __forceinline__ const Part& part_of(const Parts<NP>& ps, unsigned e) {
-  return ps.get((int)((e >> 24) & 31u));
-}
-
-template <int NP, int U>
-__global__ __launch_bounds__(256) void k_fwd_stress(Parts<NP> ps, const unsigned* __restrict__ map,
-                                                    int it) {
-  const unsigned e = map[blockIdx.x];
-  if ((e >> 29) == kNop) return;
-  stress_fwd<U>(part_of(ps, e), (int)(e & 0xffffffu), it);
-}
-
-// the velocity update of step it and the recording of the stresses it read
-// (recording reads only stresses, which the velocity update does not touch)
-template <int NP, int U>
-__global__ __launch_bounds__(256) void k_fwd_vel(Parts<NP> ps, const unsigned* __restrict__ map,
-                                                 int it) {
-  const unsigned e = map[blockIdx.x];
-  const unsigned kind = e >> 29;
-  if (kind == kVelFwd)
-    vel_fwd<U>(part_of(ps, e), (int)(e & 0xffffffu));
-  else if (kind == kRecord)
-    record(part_of(ps, e), (int)(e & 0xffffffu), it);
-}
-
-// Backward pairs with disjoint reads and writes share a launch:
-//   a: rev_stress(it) + adj_vel(it)   (rev_stress reads the adjoint stress that
-//      adj_vel also only reads; adj_vel writes the adjoint velocity that
-//      rev_stress does not touch)
-//   b: adj_stress(it) + rev_vel(it-1) (rev_vel reads the adjoint velocity that
-//      adj_stress also only reads; adj_stress writes the adjoint stress that
-//      rev_vel does not touch)
-template <int NP, int U>
-__global__ __launch_bounds__(256) void k_bwd_a(Parts<NP> ps, const unsigned* __restrict__ map,
-                                               int it) {
-  const unsigned e = map[blockIdx.x];
-  const unsigned kind = e >> 29;
-  if (kind == kRevStress)
-    rev_stress<U>(part_of(ps, e), (int)(e & 0xffffffu), it);
-  else if (kind == kAdjVel)
-    adj_vel<U>(part_of(ps, e), (int)(e & 0xffffffu), it);
-}
-
-template <int NP, int U>
-__global__ __launch_bounds__(256) void k_bwd_b(Parts<NP> ps, const unsigned* __restrict__ map,
-                                               int it) {
-  const unsigned e = map[blockIdx.x];
-  const unsigned kind = e >> 29;
-  if (kind == kAdjStress)
-    adj_stress<U>(part_of(ps, e), (int)(e & 0xffffffu), it);
-  else if (kind == kRevVel)
-    rev_vel<U>(part_of(ps, e), (int)(e & 0xffffffu), it - 1);
-}
+#include "step_kernels.hpp"
 
 // res_injection (utilities.cu:569-580) for surveys whose receivers are not one
 // per cell in one row: one thread per injection cell adds its receivers'
@@ -1581,78 +415,6 @@ bool spacing_ok(float d) {
   return ok;
 }
 
-// ---------------------------------------------------- workgroup maps
-// Each XCD's ordered list of work; the launch grid interleaves them so that
-// workgroup b = 8 j + k is entry j of XCD k's list.
-struct Lists {
-  std::vector<unsigned> l[8];
-  size_t longest() const {
-    size_t n = 0;
-    for (const auto& v : l) n = std::max(n, v.size());
-    return n;
-  }
-  bool empty() const { return longest() == 0; }
-};
-
-// tiles [0, n) in 8 contiguous bands (z fastest, then x): neighbouring tiles,
-// which share halo columns, share an XCD's L2
-void band(Lists& L, unsigned kind, int part, int n) {
-  for (int k = 0; k < 8; k++)
-    for (int t = (int)((long long)n * k / 8); t < (int)((long long)n * (k + 1) / 8); t++)
-      L.l[k].push_back(wg_entry(kind, (unsigned)part, (unsigned)t));
-}
-
-// The update-region tiling, whose first `hl` and last `hr` tile columns are
-// heavier (the x-direction C-PML): each XCD gets one contiguous run of the
-// heavy tiles, first, then one contiguous run of the others.
-void balanced(Lists& L, unsigned kind, int part, int gz, int gx, int hl, int hr) {
-  std::vector<int> heavy, light;
-  for (int bx = 0; bx < gx; bx++) {
-    const bool h = bx < hl || bx >= gx - hr;
-    for (int bz = 0; bz < gz; bz++) (h ? heavy : light).push_back(bx * gz + bz);
-  }
-  const size_t H = heavy.size(), Ln = light.size();
-  for (int k = 0; k < 8; k++) {
-    for (size_t q = H * k / 8; q < H * (k + 1) / 8; q++)
-      L.l[k].push_back(wg_entry(kind, (unsigned)part, (unsigned)heavy[q]));
-    for (size_t q = Ln * k / 8; q < Ln * (k + 1) / 8; q++)
-      L.l[k].push_back(wg_entry(kind, (unsigned)part, (unsigned)light[q]));
-  }
-}
-
-// items [0, n) dealt round robin
-void dealt(Lists& L, unsigned kind, int part, int n) {
-  for (int t = 0; t < n; t++) L.l[t % 8].push_back(wg_entry(kind, (unsigned)part, (unsigned)t));
-}
-
-void append(Lists& A, const Lists& B) {
-  for (int k = 0; k < 8; k++) A.l[k].insert(A.l[k].end(), B.l[k].begin(), B.l[k].end());
-}
-
-// per XCD, the two lists interleaved in proportion to their lengths, so both
-// halves of a paired launch sweep their tiles at the same pace
-Lists interleave(const Lists& A, const Lists& B) {
-  Lists M;
-  for (int k = 0; k < 8; k++) {
-    const auto &a = A.l[k], &b = B.l[k];
-    const size_t na = a.size(), n = na + b.size();
-    size_t ia = 0, ib = 0;
-    for (size_t j = 0; j < n; j++) {
-      const bool takeA = ia < na && (ib >= b.size() || (j + 1) * na / n > ia);
-      M.l[k].push_back(takeA ? a[ia++] : b[ib++]);
-    }
-  }
-  return M;
-}
-
-std::vector<unsigned> flatten(const Lists& L) {
-  const size_t n = L.longest();
-  std::vector<unsigned> m(8 * n, wg_entry(kNop, 0, 0));
-  for (int k = 0; k < 8; k++)
-    for (size_t j = 0; j < L.l[k].size(); j++) m[8 * j + k] = L.l[k][j];
-  return m;
-}
-
 }  // namespace
 
 // A launch bracketed by timing events.
@@ -1666,13 +428,6 @@ struct TimedLaunch {
 struct GraphEntry {
   hipGraphExec_t exec = nullptr;
   std::vector<TimedLaunch> recs;
-};
-
-// Device-resident workgroup maps, part tables and captured time loops of a
-// job, kept across runs.
-struct DevMap {
-  unsigned* ptr = nullptr;
-  int n = 0;  // workgroups of the launch
 };
 
 // Bump allocator over a fixed device region (the scratch array of the
@@ -1699,24 +454,21 @@ struct Arena {
   }
 };
 
+// Device-resident argument tables and captured time loops of a job, kept
+// across runs.
 struct JobCache {
   int dev = 0;
   Arena* arena = nullptr;  // device memory comes from here instead of hipMalloc when set
-  std::map<std::string, DevMap> maps;
-  Part* table = nullptr;  // part tables of the multi-part launches of the last run
-  size_t table_cap = 0;
+  StepArgs* steps = nullptr;  // forward and backward launch arguments of the last run
+  BackArgs* backs = nullptr;
+  size_t steps_cap = 0, backs_cap = 0;
   std::map<std::string, GraphEntry> graphs;
   ~JobCache() {
     (void)hipSetDevice(dev);
     clear_graphs();
     if (arena) return;
-    for (auto& kv : maps) (void)hipFree(kv.second.ptr);
-    if (table) (void)hipFree(table);
-  }
-  Status device_alloc(void** p, size_t nb) {
-    if (arena) return arena->take(p, nb);
-    HIP_TRY(hipMalloc(p, nb));
-    return Status::Ok();
+    if (steps) (void)hipFree(steps);
+    if (backs) (void)hipFree(backs);
   }
   void clear_graphs() {
     for (auto& kv : graphs) {
@@ -1728,32 +480,19 @@ struct JobCache {
     }
     graphs.clear();
   }
-  Status map(const std::string& key, const Lists& L, DevMap& out) {
-    auto it = maps.find(key);
-    if (it != maps.end()) {
-      out = it->second;
-      return Status::Ok();
+  template <typename T>
+  Status upload(const std::vector<T>& a, T*& dev_ptr, size_t& cap) {
+    if (a.size() > cap) {
+      if (dev_ptr && !arena) HIP_TRY(hipFree(dev_ptr));
+      dev_ptr = nullptr;
+      cap = 0;
+      if (arena)
+        TRY(arena->take((void**)&dev_ptr, a.size() * sizeof(T)));
+      else
+        HIP_TRY(hipMalloc((void**)&dev_ptr, a.size() * sizeof(T)));
+      cap = a.size();
     }
-    const std::vector<unsigned> m = flatten(L);
-    DevMap dm;
-    dm.n = (int)m.size();
-    TRY(device_alloc((void**)&dm.ptr, std::max<size_t>(1, m.size()) * sizeof(unsigned)));
-    if (!m.empty())
-      HIP_TRY(hipMemcpy(dm.ptr, m.data(), m.size() * sizeof(unsigned), hipMemcpyHostToDevice));
-    maps[key] = dm;
-    out = dm;
-    return Status::Ok();
-  }
-  Status upload_table(const std::vector<Part>& parts) {
-    if (parts.size() > table_cap) {
-      if (table && !arena) HIP_TRY(hipFree(table));
-      table = nullptr;
-      table_cap = 0;
-      TRY(device_alloc((void**)&table, parts.size() * sizeof(Part)));
-      table_cap = parts.size();
-    }
-    if (!parts.empty())
-      HIP_TRY(hipMemcpy(table, parts.data(), parts.size() * sizeof(Part), hipMemcpyHostToDevice));
+    if (!a.empty()) HIP_TRY(hipMemcpy(dev_ptr, a.data(), a.size() * sizeof(T), hipMemcpyHostToDevice));
     return Status::Ok();
   }
 };
@@ -1766,19 +505,11 @@ struct DeviceState {
   int R = 0;
   std::vector<int> roff;  // first receiver of each shot (+ total)
   // engine settings (environment variables read at plan creation)
-  int tile_x = 4;          // x extent of a workgroup tile (blockDim.y)
-  bool xcd = true;         // XCD-banded workgroup order
-  bool balance = true;     // C-PML columns shared evenly by the XCDs (update-region launches)
-  bool mix = true;         // backward pair halves interleaved (pair a)
-  bool mix_b = true;       // ... (pair b)
-  bool pair_a = true;      // reverse stress + adjoint velocity in one launch
-  bool pair_b = true;      // adjoint stress + reverse velocity in one launch
-  int unroll = 1;          // shots whose loads a backward thread issues together
-  int unroll_fwd = 2;      // ... a forward thread
+  int tile_x = 4;          // columns of a half step's tile (blockDim.y) where chosen
+  bool tile_auto = true;   // not chosen
   int shot_group = -1;     // shots per forward launch (0: all, -1: automatic)
   int shot_group_bwd = -1; // shots per backward launch (0: all, -1: automatic)
   bool fold_inject = true; // residual injection inside the adjoint stress update
-  bool part_table = false; // single-part launches also read their part from device memory
   bool graphs = false;     // shot groups' time loops captured and replayed as graphs
                            // (measured no faster at 608x1780; timed runs stay eager)
   int ckpt_every = 0;      // 0: boundary ring every step; k > 0: checkpoints every k steps
@@ -1787,21 +518,29 @@ struct DeviceState {
   // model + tables
   float *lam = nullptr, *mu = nullptr, *den = nullptr, *amu = nullptr, *ba = nullptr,
         *bb = nullptr;
-  float* pml = nullptr;   // 6*nzA + 6*nx
+  // C-PML coefficients by row, then by column: K, 1/K, a, b and the half-cell
+  // K, 1/K, a, b; and 1/K in double
+  float* pmlc = nullptr;
+  double* pml64 = nullptr;
   float* win2 = nullptr;  // nSteps
   int* src = nullptr;     // [ns][2]
   float* srcamp = nullptr;  // [ns][nSteps] windowed source rows
   float* srcwin = nullptr;  // [nSteps] the source rows' window (exact adjoint's stf gradient)
   int* rec = nullptr;     // [R][3] (z, x, plan shot)
-  int* rec_at = nullptr;  // [ns][nx] receiver of each column (one-row surveys)
-  int rec_row = -1;
-  // residual injection cells (surveys the folded injection does not cover)
+  // residual injection: cells with their receivers (in receiver order), and by
+  // shot and column
   int *icell = nullptr, *iptr = nullptr, *irid = nullptr;
   std::vector<int> coff;  // first injection cell of each shot (+ total)
+  std::vector<int> icells, iptrs, irids;  // host copies until a gradient run needs them
+  ColInj* inj = nullptr;
+  bool inj_folded = false;  // the adjoint kernels inject (else k_res_inject does)
   // wavefields
   float *fwd = nullptr, *mem = nullptr, *adj = nullptr, *madj = nullptr;
   float* ring = nullptr;
   size_t ring_floats = 0;
+  // second state of the whole-step launches, for the shots of one launch
+  float *fwd2 = nullptr, *mem2 = nullptr, *adj2 = nullptr, *madj2 = nullptr;
+  int shots2 = 0, mshots2 = 0, ashots2 = 0, xshots2 = 0;  // shots of each
   float* xt = nullptr;  // exact adjoint: operands [backward group shot][8][cell]
   size_t xt_floats = 0;
   float* snap = nullptr;
@@ -1944,21 +683,10 @@ struct DeviceState {
     pending.clear();
   }
 
-  Pml pml_ptrs() const {
-    const int nzA = g.nzA, nx = g.nx;
-    const float* z = pml;
-    const float* x = pml + 6 * nzA;
-    return Pml{z, z + nzA, z + 2 * nzA, z + 3 * nzA, z + 4 * nzA, z + 5 * nzA,
-               x, x + nx,  x + 2 * nx,  x + 3 * nx,  x + 4 * nx,  x + 5 * nx};
-  }
   Mdl mdl() const { return Mdl{lam, mu, amu, ba, bb}; }
   size_t F() const { return (size_t)g.ns * g.N; }
   // first cell of shot s0 in a [shot][comps][cell] array
   float* shot(float* base, int comps, int s0) const { return base + (size_t)s0 * comps * g.N; }
-  int gzU() const { return (g.nzA + kBZ - 1) / kBZ; }
-  int gxU() const { return (g.nx + tile_x - 1) / tile_x; }
-  int gzR() const { return (g.ringH + kBZ - 1) / kBZ; }
-  int gxR() const { return (g.ringW + tile_x - 1) / tile_x; }
   // ~40 B per cell and shot of forward state stay cache-resident from step to
   // step; the backward holds forward and adjoint state (~64 B), and the exact
   // adjoint its two operand sets besides (+32 B).  224 MB of the 256 MB
@@ -2030,19 +758,11 @@ Status Plan::create(const std::string& para_fname, int gpu, int group_size, cons
   d_.reset(new DeviceState());
   DeviceState& d = *d_;
   d.dev = gpu;
+  d.tile_auto = !std::getenv("FWIFLOW_TILE_X");
   d.tile_x = std::max(1, std::min(4, env_int("FWIFLOW_TILE_X", 4)));  // <= 256 threads
-  d.xcd = env_int("FWIFLOW_XCD_REMAP", 1) != 0;
-  d.balance = env_int("FWIFLOW_XCD_BALANCE", 1) != 0 && d.xcd;
-  d.mix = env_int("FWIFLOW_PAIR_MIX", 1) != 0;
-  d.mix_b = env_int("FWIFLOW_PAIR_MIX_B", 1) != 0;
-  d.pair_a = env_int("FWIFLOW_PAIR_A", 1) != 0;
-  d.pair_b = env_int("FWIFLOW_PAIR_B", 1) != 0;
-  d.unroll = env_int("FWIFLOW_SHOT_UNROLL", 1) >= 2 ? 2 : 1;
-  d.unroll_fwd = env_int("FWIFLOW_SHOT_UNROLL_FWD", 2) >= 2 ? 2 : 1;
   d.shot_group = std::max(-1, env_int("FWIFLOW_SHOT_GROUP", -1));
   d.shot_group_bwd = std::max(-1, env_int("FWIFLOW_SHOT_GROUP_BWD", -1));
   d.fold_inject = env_int("FWIFLOW_FOLD_INJECT", 1) != 0;
-  d.part_table = env_int("FWIFLOW_PART_TABLE", 0) != 0;
   d.graphs = env_int("FWIFLOW_GRAPHS", 0) != 0;
   d.adjoint = env_int("FWIFLOW_EXACT_ADJOINT", 0) != 0 ? 1 : 0;
   if (in_scratch) {
@@ -2081,17 +801,33 @@ Status Plan::create(const std::string& para_fname, int gpu, int group_size, cons
   g.rnt = std::max(1, g.nSteps - 1);
 
   const size_t N = (size_t)g.N;
-  TRY(d.alloc(&d.lam, N));
-  TRY(d.alloc(&d.mu, N));
-  TRY(d.alloc(&d.den, N));
-  TRY(d.alloc(&d.amu, N));
-  TRY(d.alloc(&d.ba, N));
-  TRY(d.alloc(&d.bb, N));
-  std::vector<float> tab(6 * (size_t)g.nzA + 6 * (size_t)g.nx);
-  cpml_profiles(g.nzA, g.nPml, para.dz, para.f0, para.dt, tab.data());
-  cpml_profiles(g.nx, g.nPml, para.dx, para.f0, para.dt, tab.data() + 6 * g.nzA);
-  TRY(d.alloc(&d.pml, tab.size()));
-  HIP_TRY(hipMemcpy(d.pml, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice));
+  // one array [lam, mu, amu, ba, bb, den][NX][NZ]: one base address in the kernels
+  TRY(d.alloc(&d.lam, 6 * N));
+  d.mu = d.lam + N, d.amu = d.lam + 2 * N, d.ba = d.lam + 3 * N, d.bb = d.lam + 4 * N;
+  d.den = d.lam + 5 * N;
+  {
+    std::vector<float> tab(6 * ((size_t)g.nzA + g.nx)), c(8 * ((size_t)g.nzA + g.nx));
+    std::vector<double> c64((size_t)g.nzA + g.nx);
+    cpml_profiles(g.nzA, g.nPml, para.dz, para.f0, para.dt, tab.data());
+    cpml_profiles(g.nx, g.nPml, para.dx, para.f0, para.dt, tab.data() + 6 * g.nzA);
+    float* o = c.data();
+    double* o64 = c64.data();
+    for (int axis = 0; axis < 2; axis++) {
+      const int n = axis ? g.nx : g.nzA;
+      const float* p = tab.data() + (axis ? 6 * (size_t)g.nzA : 0);
+      for (int i = 0; i < n; i++) {
+        for (int h = 0; h < 2; h++, o += 4) {
+          const float* q = p + 3 * (size_t)h * n + i;
+          o[0] = q[0], o[1] = 1.f / q[0], o[2] = q[n], o[3] = q[2 * (size_t)n];
+        }
+        *o64++ = 1.0 / (double)p[i];
+      }
+    }
+    TRY(d.alloc(&d.pmlc, c.size()));
+    TRY(d.alloc(&d.pml64, c64.size()));
+    HIP_TRY(hipMemcpy(d.pmlc, c.data(), c.size() * sizeof(float), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(d.pml64, c64.data(), c64.size() * sizeof(double), hipMemcpyHostToDevice));
+  }
   std::vector<float> w2(g.nSteps);
   window_squared(g.nSteps, para.dt, 0.005f, w2.data());
   TRY(d.alloc(&d.win2, w2.size()));
@@ -2116,46 +852,29 @@ Status Plan::create(const std::string& para_fname, int gpu, int group_size, cons
   }
   d.roff[g.ns] = (int)r;
   {
-    // one-row surveys with at most one receiver per cell get the injection
-    // inside the adjoint stress update
-    bool one_row = d.R > 0;
-    const int row = d.R > 0 ? rec[0] : -1;
-    std::vector<int> at((size_t)g.ns * g.nx, -1);
-    for (int k = 0; k < d.R && one_row; k++) {
-      int& slot = at[(size_t)rec[3 * k + 2] * g.nx + rec[3 * k + 1]];
-      if (rec[3 * k] != row || slot >= 0) one_row = false;
-      slot = k;
-    }
-    if (one_row && d.fold_inject) {
-      TRY(d.alloc(&d.rec_at, at.size()));
-      HIP_TRY(hipMemcpy(d.rec_at, at.data(), at.size() * sizeof(int), hipMemcpyHostToDevice));
-      d.rec_row = row;
-    }
-  }
-  {
-    // injection cells of each shot, receivers of a cell in receiver order
-    std::vector<int> cells, ptr{0}, rid;
+    // injection cells of each shot, receivers of a cell in receiver order.  The
+    // adjoint kernels inject where every receiver lies in the update region,
+    // and for one-row surveys with one receiver per cell also where some do
+    // not (those are then left out).
+    bool one_row = d.R > 0, inside = true;
+    d.iptrs.push_back(0);
     d.coff.assign(g.ns + 1, 0);
     for (int s = 0; s < g.ns; s++) {
-      d.coff[s] = (int)cells.size() / 3;
+      d.coff[s] = (int)d.icells.size() / 3;
       std::map<std::pair<int, int>, std::vector<int>> by;  // (x, z) -> receivers
       for (int k = d.roff[s]; k < d.roff[s + 1]; k++)
         by[{rec[3 * k + 1], rec[3 * k]}].push_back(k);
       for (auto& kv : by) {
-        cells.insert(cells.end(), {s, kv.first.second, kv.first.first});
-        rid.insert(rid.end(), kv.second.begin(), kv.second.end());
-        ptr.push_back((int)rid.size());
+        const int z = kv.first.second, x = kv.first.first;
+        one_row = one_row && z == rec[0] && kv.second.size() == 1;
+        inside = inside && z >= 2 && z <= g.nzA - 3 && x >= 2 && x <= g.nx - 3;
+        d.icells.insert(d.icells.end(), {s, z, x});
+        d.irids.insert(d.irids.end(), kv.second.begin(), kv.second.end());
+        d.iptrs.push_back((int)d.irids.size());
       }
     }
-    d.coff[g.ns] = (int)cells.size() / 3;
-    TRY(d.alloc(&d.icell, std::max<size_t>(1, cells.size())));
-    TRY(d.alloc(&d.iptr, ptr.size()));
-    TRY(d.alloc(&d.irid, std::max<size_t>(1, rid.size())));
-    if (!cells.empty())
-      HIP_TRY(hipMemcpy(d.icell, cells.data(), cells.size() * sizeof(int), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(d.iptr, ptr.data(), ptr.size() * sizeof(int), hipMemcpyHostToDevice));
-    if (!rid.empty())
-      HIP_TRY(hipMemcpy(d.irid, rid.data(), rid.size() * sizeof(int), hipMemcpyHostToDevice));
+    d.coff[g.ns] = (int)d.icells.size() / 3;
+    d.inj_folded = d.fold_inject && (one_row || inside);
   }
   TRY(d.alloc(&d.src, src.size()));
   HIP_TRY(hipMemcpy(d.src, src.data(), src.size() * sizeof(int), hipMemcpyHostToDevice));
@@ -2216,6 +935,31 @@ Status Plan::create(const std::string& para_fname, int gpu, int group_size, cons
   TRY(d.alloc(&d.syn, std::max<size_t>(1, (size_t)g.nSteps * d.R)));
   TRY(d.alloc(&d.misfit, 1));
   return Status::Ok();
+}
+
+// injection tables, on the first gradient run
+static Status ensure_injection(DeviceState& d) {
+  if (d.inj) return Status::Ok();
+  std::vector<ColInj> col((size_t)d.g.ns * d.g.nx, ColInj{0, 0, 0, -1});
+  if (d.inj_folded)
+    for (int c = 0; c < (int)d.icells.size() / 3; c++) {
+      ColInj& q = col[(size_t)d.icells[3 * c] * d.g.nx + d.icells[3 * c + 2]];
+      if (!q.n++) {
+        q.first = c, q.z = d.icells[3 * c + 1];
+        q.rid = d.iptrs[c + 1] - d.iptrs[c] == 1 ? d.irids[d.iptrs[c]] : -1;
+      } else {
+        q.rid = -1;
+      }
+    }
+  auto put = [&](auto*& p, const auto& v) -> Status {
+    TRY(d.alloc(&p, std::max<size_t>(1, v.size())));
+    if (!v.empty()) HIP_TRY(hipMemcpy(p, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice));
+    return Status::Ok();
+  };
+  TRY(put(d.icell, d.icells));
+  TRY(put(d.iptr, d.iptrs));
+  TRY(put(d.irid, d.irids));
+  return put(d.inj, col);
 }
 
 Status Plan::set_model(const double* Lambda, const double* Mu, const double* Den, bool zfast) {
@@ -2329,6 +1073,7 @@ Status Plan::set_launch(int tile_x, int shots_fwd, int shots_bwd) {
   if (tile_x < 1 || tile_x > 4) return Status::Err(FWIFLOW_ERR_ARG, "tile width must be 1..4");
   if (shots_fwd < -1 || shots_bwd < -1)
     return Status::Err(FWIFLOW_ERR_ARG, "shots per launch must be >= -1");
+  d_->tile_auto = false;
   d_->tile_x = tile_x;
   d_->shot_group = shots_fwd;
   d_->shot_group_bwd = shots_bwd;
@@ -2454,7 +1199,7 @@ static Status condition_residual(DeviceState& d, const Para& para, bool keep, in
 // One run of calc_id over one or several plans on one device.  The plans'
 // shots are lined up in rows (row r = shot r of every plan that has one); a
 // launch of a time-step kernel covers a group of rows of every plan, each
-// plan one part of the launch's workgroup map.
+// plan one part of the launch.
 //
 // Gradient runs take the rows in sweeps (super-groups): a sweep runs the
 // forward of its rows, their residual and their backward before the next
@@ -2482,21 +1227,35 @@ std::vector<RowRange> split_even(int a, int b, int per) {
   return v;
 }
 
+// every 64th step of each launch kind is bracketed by timing events (when
+// timing is on): events between launches cost the stream about 2% at every
+// 8th step
+constexpr int sample_every = 64;
+constexpr int kMaxPartsTable = 31;  // plans of a job
+// Where a time step is one launch instead of two, in waves of a half-step
+// launch (64 depth cells x 1 column x 1 shot each).  Forward: one launch less
+// and no second read of the first half's results, against the rim that is
+// computed twice and a second copy of the state in the caches.  Measured, two
+// launches / one: 168 waves 1.89 / 1.20 ms, 792: 14.6 / 12.4, 2046: 10.6 /
+// 10.1, 10752: 39.2 / 38.0, 23136: 45.5 / 44.9, 36500: 60.1 / 59.8, 53760:
+// 93 / 100, 142400: 59 / 79.  Backward (adjoint and reversal both recompute
+// their rim, twice the state is copied, and a thread walks all shots): one
+// shot of 792 waves 12.4 / 10.8 ms, 682: 6.98 / 6.61, 1792: 7.89 / 7.71, 3300:
+// 11.7 / 12.0; two shots of 168 waves each 7.37 / 7.00, 792: 16.0 / 14.6,
+// 1792: 10.1 / 10.8; four of 168: 8.3 / 10.3.
+constexpr double kWholeFwdWaves = 16384, kWholeBwdWaves = 2048;
+constexpr int kWholeBwdShots = 2;
+
 enum Phase { kPhFwd = 0, kPhRec = 1, kPhBwd = 2 };
 
-// the parts of one group of rows in one phase
+// One group of rows in one phase: its parts (plan shots [s0, s0 + n) of a
+// member) and their launch arguments.  steps / backs: index of the first
+// part's entry in the argument tables; the entries of the whole-step launches,
+// one set per combination of state buffers, follow those of the half steps.
 struct GroupParts {
-  std::vector<Part> parts;
-  std::vector<int> member;  // member of each part
-  size_t table_off = 0;     // offset of the parts in the job's device table
-  std::string key;          // row range, for the map cache
-};
-
-struct StepLaunch {
-  const Part* table = nullptr;  // device table (multi-part)
-  const Part* single = nullptr;
-  const unsigned* map = nullptr;
-  int nwg = 0;
+  std::vector<int> member, s0, n;
+  std::vector<StepArgs> args;
+  size_t steps = 0, backs = 0;
 };
 
 class Runner {
@@ -2509,54 +1268,77 @@ class Runner {
   JobCache& cache;
   DeviceState* d0 = nullptr;
   hipStream_t st = nullptr;
-  dim3 blk;
   int nSteps = 0, rows = 0, gf = 1, gb = 1, S = 1, K = 0, nsnap = 0;
+  // shots per slice and slices of a forward launch, threads per cell of a backward one
+  int sf_ = 1, nf_ = 1, nb_ = 1;
   bool if_res = false, withAdj = false, ckpt = false;
-  std::vector<Part> table;  // host copy of every multi-part group's parts
+  int tile_ = 2;  // columns of a half step's workgroup
+  bool whole_f_ = false, whole_b_ = false;  // whole-step launches (forward, reference's adjoint)
+  std::vector<StepArgs> steps_;             // host copies of the argument tables
+  std::vector<BackArgs> backs_;
+  float* xt_ = nullptr;                     // exact adjoint operands of the running group
+  const float* srcwin_ = nullptr;           // and the source window
 
   int shots_in(const Member& m, int r) const { return std::min(r, m.d->g.ns); }
   GroupParts parts_of(RowRange rr, int sg0, Phase ph);
-  Status maps_of(const GroupParts& gp, const char* kind, DevMap& out);
-  StepLaunch step(const GroupParts& gp, const DevMap& m) const {
-    StepLaunch s;
-    s.map = m.ptr;
-    s.nwg = m.n;
-    if (gp.parts.size() == 1 && !d0->part_table)
-      s.single = &gp.parts[0];
+  double waves(int shots) const;
+  void slice(int shots, int& per, int& n) const;
+  int threads_per_cell(int shots) const;
+  int ring_at(int it) const { return withAdj ? it % (ckpt ? K : std::max(1, nSteps - 1)) : -1; }
+
+  // launches: half steps (in place)
+  template <typename Ker, typename... A>
+  void go(Ker k, dim3 grid, dim3 block, A... a) {
+    if (d0->kernel_start)
+      hipExtLaunchKernelGGL(k, grid, block, 0, st, d0->kernel_start, d0->kernel_end, 0, a...);
     else
-      s.table = cache.table + gp.table_off;
-    return s;
+      hipLaunchKernelGGL(k, grid, block, 0, st, a...);
   }
-  void fwd_stress(const StepLaunch& s, int it, int U);
-  void fwd_vel(const StepLaunch& s, int it, int U);
-  void bwd_a(const StepLaunch& s, int it, int U);
-  void bwd_b(const StepLaunch& s, int it, int U);
-  void exact_a(const Part& P, int it, int first);
-  void exact_b(const Part& P, int it);
-  float* xt_ = nullptr;            // exact adjoint operands of the running group
-  const float* srcwin_ = nullptr;  // and the source window
-  Status snapshot(const GroupParts& gp, int sg0, int j, bool save);
+  // grid of a half-step launch: `kinds` strips per tile row, and rows for the
+  // extra items (ring, receivers, illumination) of the parts
+  dim3 half_grid(const GroupParts& gp, int kinds, bool ring, bool rec, bool illum, int places) const;
+  void half_stress(const GroupParts& gp, int it, int ring);
+  void half_vel(const GroupParts& gp, int it, int ring);
+  void half_a(const GroupParts& gp, int it, int ring, int kinds);
+  void half_b(const GroupParts& gp, int it, int ring, int kinds);
+  void exact_a(const GroupParts& gp, int it, int first);
+  void exact_b(const GroupParts& gp, int it);
+  template <bool Save>
+  void ring_all(const GroupParts& gp, int it, int c0, int c1);
+  // whole steps: `odd` launches read the second state buffers
+  dim3 whole_grid(const GroupParts& gp, bool backward) const;
+  void step_fwd(const GroupParts& gp, int odd, int it);
+  void step_bwd(const GroupParts& gp, int fodd, int aodd, int it);
+  void record_last(const GroupParts& gp, int it);
+  void illum_last(const GroupParts& gp);
+  Status clear_second(const GroupParts& gp);
+  // forward steps [t0, t1) of a group, `before(it, odd)` before each; they end
+  // in the main state buffers
+  Status forward(const GroupParts& gp, int t0, int t1,
+                 const std::function<Status(int, int)>& before);
+
+  Status snapshot(const GroupParts& gp, int sg0, int j, bool save, int odd);
   // run `body` (launches only, no memsets) as a graph captured on first use
   Status replay(const std::string& key, const std::function<void()>& body);
-  std::string graph_key(const char* phase, const GroupParts& gp,
-                        std::initializer_list<const DevMap*> maps) const;
+  std::string graph_key(const char* phase, const GroupParts& gp) const;
 };
 
-std::string Runner::graph_key(const char* phase, const GroupParts& gp,
-                              std::initializer_list<const DevMap*> maps) const {
-  // FNV-1a over everything the captured launches bake in: parts, maps,
-  // unroll factors and whether launches are timed
+std::string Runner::graph_key(const char* phase, const GroupParts& gp) const {
+  // FNV-1a over everything the captured launches bake in
   unsigned long long h = 1469598103934665603ULL;
   auto mix = [&](const void* p, size_t n) {
     const unsigned char* b = (const unsigned char*)p;
     for (size_t i = 0; i < n; i++) h = (h ^ b[i]) * 1099511628211ULL;
   };
-  for (const Part& P : gp.parts) mix(&P, sizeof(Part));
-  for (const DevMap* m : maps) mix(m, sizeof(DevMap));
-  const int flags[4] = {d0->unroll, d0->unroll_fwd, d0->timing ? 1 : 0, nSteps};
+  mix(gp.args.data(), gp.args.size() * sizeof(StepArgs));
+  const void* ptrs[4] = {cache.steps, cache.backs, xt_, srcwin_};
+  mix(ptrs, sizeof(ptrs));
+  const size_t offs[2] = {gp.steps, gp.backs};
+  mix(offs, sizeof(offs));
+  const int flags[] = {d0->timing ? 1 : 0, nSteps, sf_, nf_, nb_, whole_f_, whole_b_,
+                       tile_, withAdj};
   mix(flags, sizeof(flags));
-  if (gp.parts.size() > 1 || d0->part_table) mix(&cache.table, sizeof(cache.table));
-  return std::string(phase) + "/" + gp.key + "/" + std::to_string(h);
+  return std::string(phase) + "/" + std::to_string(h);
 }
 
 Status Runner::replay(const std::string& key, const std::function<void()>& body) {
@@ -2596,168 +1378,258 @@ Status Runner::replay(const std::string& key, const std::function<void()>& body)
   return Status::Ok();
 }
 
-// a sampled launch (timing on) goes through hipExtLaunchKernel with the
-// plan's kernel_start / kernel_end events
-#define STEP_LAUNCH_ONE(K, a)                                                               \
-  do {                                                                                      \
-    if (d0->kernel_start)                                                                   \
-      hipExtLaunchKernelGGL(K, grid, blk, 0, st, d0->kernel_start, d0->kernel_end, 0, a,    \
-                            s.map, it);                                                     \
-    else                                                                                    \
-      hipLaunchKernelGGL(K, grid, blk, 0, st, a, s.map, it);                                \
-  } while (0)
-#define STEP_LAUNCH(KER)                                                                    \
-  do {                                                                                      \
-    if (!s.nwg) break;                                                                      \
-    const dim3 grid((unsigned)s.nwg);                                                       \
-    if (s.single) {                                                                         \
-      const Parts<1> a{*s.single};                                                          \
-      if (U == 2)                                                                           \
-        STEP_LAUNCH_ONE((KER<1, 2>), a);                                                    \
-      else                                                                                  \
-        STEP_LAUNCH_ONE((KER<1, 1>), a);                                                    \
-    } else {                                                                                \
-      const Parts<0> a{s.table};                                                            \
-      if (U == 2)                                                                           \
-        STEP_LAUNCH_ONE((KER<0, 2>), a);                                                    \
-      else                                                                                  \
-        STEP_LAUNCH_ONE((KER<0, 1>), a);                                                    \
-    }                                                                                       \
-  } while (0)
+double Runner::waves(int shots) const {
+  double w = 0;
+  for (const Member& m : M)
+    w += (double)((m.d->g.nzA + kBZ - 1) / kBZ) * m.d->g.nx * std::min(shots, m.d->g.ns);
+  return w;
+}
 
-void Runner::fwd_stress(const StepLaunch& s, int it, int U) { STEP_LAUNCH(k_fwd_stress); }
-void Runner::fwd_vel(const StepLaunch& s, int it, int U) { STEP_LAUNCH(k_fwd_vel); }
-void Runner::bwd_a(const StepLaunch& s, int it, int U) { STEP_LAUNCH(k_bwd_a); }
-void Runner::bwd_b(const StepLaunch& s, int it, int U) { STEP_LAUNCH(k_bwd_b); }
-#undef STEP_LAUNCH
-#undef STEP_LAUNCH_ONE
+// A forward launch's shots are cut into slices, each with its own workgroups,
+// so that small grids bring enough waves to hide a cell's loads: about
+// kSliceWaves, but slices of two shots at least once the chip's 1024 SIMDs
+// have four waves each, since the second shot of a thread shares the first
+// one's model loads and indexing.  224x448, 30 shots: objective 98.8 ms at
+// 8192 waves, 96.8 at 16384, 97.3 at 32768, 102.3 at 65536; 6 shots of it in
+// slices of two / one: gradient 39.2 / 41.8 ms; 580x1780 (17800 waves a shot):
+// 58.7 ms at 8192 .. 32768, 60.1 at 65536.
+constexpr double kSliceWaves = 16384, kPairWaves = 4096;
+void Runner::slice(int shots, int& per, int& n) const {
+  n = std::max(1, std::min(shots, (int)std::ceil(kSliceWaves / waves(1))));
+  per = (shots + n - 1) / n;
+  if (per == 1 && waves(shots) >= 2 * kPairWaves) per = std::min(2, shots);
+  n = (shots + per - 1) / per;
+}
 
-// exact-adjoint launches: 64 x 4 workgroups over the update region
-// (with the reversal of the step: the plan's ring is that of a gradient run)
-#define EXACT_LAUNCH(K, ...)                                                                \
-  do {                                                                                      \
-    const int tiles_ = ((P.g.nzA + kBZ - 1) / kBZ) * ((P.g.nx + 3) / 4);                   \
-    const dim3 grid((unsigned)(8 * ((tiles_ + 7) / 8)));                                    \
-    const dim3 b4(kBZ, 4);                                                                  \
-    if (d0->kernel_start)                                                                   \
-      hipExtLaunchKernelGGL(K, grid, b4, 0, st, d0->kernel_start, d0->kernel_end, 0, P,     \
-                            __VA_ARGS__);                                                   \
-    else                                                                                    \
-      hipLaunchKernelGGL(K, grid, b4, 0, st, P, __VA_ARGS__);                               \
-  } while (0)
-void Runner::exact_a(const Part& P, int it, int first) { EXACT_LAUNCH(k_exact_a, xt_, it, first); }
-void Runner::exact_b(const Part& P, int it) { EXACT_LAUNCH(k_exact_b, xt_, srcwin_, it); }
-#undef EXACT_LAUNCH
+// Threads per cell of a backward launch: its shots run side by side in a
+// workgroup where one thread a cell would leave the SIMDs short of waves; 1, 2
+// or 4 (a sum's round of 8 shots divides evenly), with two shots a thread at
+// least.  1 / 2 / 4 threads, ms: 280 waves a shot, 24 shots 38.8 / 28.0 / 23.8
+// (8: 23.4); 682, 20 shots 48.1 / 38.8 / 36.0 (8: 38.4); 1792, 15 shots, exact
+// adjoint 113 / 107 / 99.6 (8: 112); 1792, 6 shots 39.6 / 39.3 / 43.7; 3300, 12
+// shots 63.2 / 62.3 / 63.5; 4562, 8 shots 61.9 / 59.6 / 65.0; 5784, 4 shots
+// 44.4 / 45.6 / 51.8; 17800, 3 shots 535 / 600 / 759.
+int Runner::threads_per_cell(int shots) const {
+  const double most = std::min({4.0, shots / 2.0, 10240 / waves(1), 16.0 / tile_});
+  return most >= 4 ? 4 : most >= 2 ? 2 : 1;
+}
 
 GroupParts Runner::parts_of(RowRange rr, int sg0, Phase ph) {
   GroupParts gp;
-  gp.key = std::to_string(rr.r0) + ":" + std::to_string(rr.r1);
+  std::vector<BackArgs> back;
   for (size_t mi = 0; mi < M.size(); mi++) {
     DeviceState& d = *M[mi].d;
+    const Geo& g = d.g;
     const int s0 = shots_in(M[mi], rr.r0), s1 = shots_in(M[mi], rr.r1);
     if (s1 <= s0) continue;
-    const int n = s1 - s0;
-    Part P{};
-    P.g = d.g;
-    P.g.ns = n;
-    P.g.s0 = s0;
-    P.g.rs0 = s0 - shots_in(M[mi], sg0);
-    P.g.rnt = ckpt ? K : std::max(1, nSteps - 1);
-    P.m = d.mdl();
-    P.c = d.pml_ptrs();
-    P.w = d.shot(d.fwd, kWaveComps, s0);
-    P.a = d.adj ? d.shot(d.adj, kWaveComps, s0) : nullptr;
-    P.p = d.shot(ph == kPhBwd && ckpt ? d.madj : d.mem, kMemComps, s0);
-    const float* amp = (ph == kPhBwd && d.src_updated) ? d.srcout : d.srcamp;
-    P.src = Src{d.src + 2 * s0, amp + (size_t)s0 * nSteps};
-    P.inj = Inj{d.rec_at && ph == kPhBwd ? d.res : nullptr, d.rec_at, d.rec_row};
-    const bool ring = withAdj && ((ph == kPhFwd && !ckpt) || ph == kPhRec || ph == kPhBwd);
-    P.ring = ring ? d.ring : nullptr;
-    P.acc = d.acc;
-    P.stf_grad = d.stf_grad ? d.stf_grad + (size_t)s0 * nSteps : nullptr;
-    P.illum = ph == kPhFwd && d.illum_on ? d.illum : nullptr;
-    P.rec = d.rec + 3 * (size_t)d.roff[s0];
-    P.syn = d.syn + d.roff[s0];
-    P.nrec = d.roff[s1] - d.roff[s0];
-    P.gzU = d.gzU();
-    P.gzR = d.gzR();
-    gp.parts.push_back(P);
     gp.member.push_back((int)mi);
-    gp.key += "|" + std::to_string(mi) + ":" + std::to_string(s0) + "-" + std::to_string(s1);
+    gp.s0.push_back(s0);
+    gp.n.push_back(s1 - s0);
+    StepArgs a{};
+    float* const mem = d.shot(ph == kPhBwd && ckpt ? d.madj : d.mem, kMemComps, s0);
+    a.wo = d.shot(d.fwd, kWaveComps, s0), a.wi = a.wo;
+    a.mo = mem, a.mi = mem;
+    a.md = d.lam, a.zc = d.pmlc, a.xc = d.pmlc + 8 * (size_t)g.nzA;
+    a.zx = d.src + 2 * s0;
+    a.amp = (ph == kPhBwd && d.src_updated ? d.srcout : d.srcamp) + (size_t)s0 * nSteps;
+    const bool ring = withAdj && ((ph == kPhFwd && !ckpt) || ph == kPhRec || ph == kPhBwd);
+    a.ring = ring ? d.ring : nullptr;
+    a.illum = ph == kPhFwd && d.illum_on ? d.illum : nullptr;
+    a.rec = d.rec + 3 * (size_t)d.roff[s0];
+    a.syn = d.syn + d.roff[s0];
+    a.nz = g.nz, a.nx = g.nx, a.nzA = g.nzA, a.nPml = g.nPml;
+    a.ns = s1 - s0, a.nSteps = nSteps, a.s0 = s0;
+    a.nrec = ph == kPhFwd ? d.roff[s1] - d.roff[s0] : 0;  // recorded once
+    a.dt = g.dt, a.dz = g.dz, a.dx = g.dx, a.rdz = g.rdz, a.rdx = g.rdx;
+    a.Nb = (int)(g.N * 4), a.R = d.R, a.ringW = g.ringW, a.ringH = g.ringH, a.ringlen = g.ringlen;
+    a.rs0 = s0 - shots_in(M[mi], sg0);
+    a.rnt = ckpt ? K : std::max(1, nSteps - 1);
+    a.gz = (g.nzA - 4 + kCoreZ - 1) / kCoreZ;
+    a.gx = (g.nx - 4 + kCoreX - 1) / kCoreX;
+    a.per = (a.gx + 7) / 8;
+    a.hgz = (g.nzA + kBZ - 1) / kBZ;
+    a.hgx = (g.nx - 4 + tile_ - 1) / tile_;
+    a.hper = (a.hgx + 7) / 8;
+    gp.args.push_back(a);
+    if (ph != kPhBwd) continue;
+    BackArgs b{};
+    b.s = a;
+    b.ao = d.shot(d.adj, kWaveComps, s0), b.ai = b.ao;
+    b.zd = d.pml64, b.xd = d.pml64 + g.nzA;
+    b.res = d.res, b.inj = d.inj, b.icell = d.icell, b.iptr = d.iptr, b.irid = d.irid;
+    b.acc = d.acc, b.stf_grad = d.stf_grad + (size_t)s0 * nSteps;
+    b.rgz = (g.ringH + kCoreZ - 1) / kCoreZ;
+    b.rgx = (g.ringW + kCoreX - 1) / kCoreX;
+    b.rper = (b.rgx + 7) / 8;
+    back.push_back(b);
   }
-  if (gp.parts.size() > 1 || d0->part_table) {
-    gp.table_off = table.size();
-    table.insert(table.end(), gp.parts.begin(), gp.parts.end());
+  if (ph != kPhBwd) {
+    gp.steps = steps_.size();
+    steps_.insert(steps_.end(), gp.args.begin(), gp.args.end());
+    for (int odd = 0; whole_f_ && odd < 2; odd++)
+      for (size_t q = 0; q < gp.args.size(); q++) {
+        const DeviceState& d = *M[gp.member[q]].d;
+        StepArgs a = gp.args[q];
+        if (odd)
+          a.wi = d.fwd2, a.mi = d.mem2;
+        else
+          a.wo = d.fwd2, a.mo = d.mem2;
+        steps_.push_back(a);
+      }
+  } else {
+    gp.backs = backs_.size();
+    backs_.insert(backs_.end(), back.begin(), back.end());
+    for (int v = 0; whole_b_ && v < 4; v++)
+      for (size_t q = 0; q < back.size(); q++) {
+        const DeviceState& d = *M[gp.member[q]].d;
+        BackArgs b = back[q];
+        float* const m2 = ckpt ? d.madj2 : d.mem2;
+        if (v & 1)
+          b.s.wi = d.fwd2;
+        else
+          b.s.wo = d.fwd2;
+        if (v & 2)
+          b.s.mi = m2, b.ai = d.adj2;
+        else
+          b.s.mo = m2, b.ao = d.adj2;
+        backs_.push_back(b);
+      }
   }
   return gp;
 }
 
-// Workgroup map of one launch kind over the parts of a group:
-//   "S" forward stress, "V" forward velocity + recording, "W" forward velocity,
-//   "A" reverse stress + adjoint velocity, "B" adjoint stress + reverse velocity,
-//   "AV" adjoint velocity, "AS" adjoint stress, "RV" reverse velocity.
-Status Runner::maps_of(const GroupParts& gp, const char* kind, DevMap& out) {
-  const std::string key = std::string(kind) + "/" + gp.key + "/" + std::to_string(d0->tile_x);
-  const std::string k = kind;
-  Lists all;
-  for (size_t q = 0; q < gp.parts.size(); q++) {
-    const DeviceState& d = *M[gp.member[q]].d;
-    const int part = (int)q;
-    auto upd = [&](unsigned kd) {
-      Lists L;
-      const int gz = d.gzU(), gx = d.gxU();
-      if (!d.xcd)
-        dealt(L, kd, part, gz * gx);
-      else if (d.balance)
-        balanced(L, kd, part, gz, gx, (d.g.nPml + d.tile_x - 1) / d.tile_x,
-                 gx - (d.g.nx - d.g.nPml) / d.tile_x);
-      else
-        band(L, kd, part, gz * gx);
-      return L;
-    };
-    auto rng = [&](unsigned kd) {
-      Lists L;
-      if (d.xcd)
-        band(L, kd, part, d.gzR() * d.gxR());
-      else
-        dealt(L, kd, part, d.gzR() * d.gxR());
-      return L;
-    };
-    Lists L;
-    if (k == "S") {
-      L = upd(kStressFwd);
-    } else if (k == "V" || k == "W") {
-      L = upd(kVelFwd);
-      if (k == "V") {
-        Lists r;
-        const int per = kBZ * d.tile_x;  // receivers per recording workgroup
-        dealt(r, kRecord, part, (gp.parts[q].nrec + per - 1) / per);
-        append(L, r);
-      }
-    } else if (k == "A") {
-      const Lists a = rng(kRevStress), b = upd(kAdjVel);
-      if (d.mix)
-        L = interleave(a, b);
-      else
-        L = a, append(L, b);
-    } else if (k == "B") {
-      const Lists a = upd(kAdjStress), b = rng(kRevVel);
-      if (d.mix_b)
-        L = interleave(a, b);
-      else
-        L = a, append(L, b);
-    } else if (k == "R") {
-      L = rng(kRevStress);
-    } else if (k == "AV") {
-      L = upd(kAdjVel);
-    } else if (k == "AS") {
-      L = upd(kAdjStress);
-    } else if (k == "RV") {
-      L = rng(kRevVel);
-    }
-    append(all, L);
+// Columns of a chunk: a strip's rim is read again by the strips above and
+// below it, from the L2 if they run soon enough.  580x1780, ms: no chunks
+// gradient 531, modelling 59.0; 128 columns 510 / 58.3, 32: 501 / 58.1, 16:
+// 496 / 57.7, 8: 497 / 57.6, 2: 528 / 58.4.  Smaller grids: 364x964 44.5 -> 43.8,
+// the two-grid job 59.7 -> 57.3, 224x448 x 30 shots 99.2 -> 96.2.
+constexpr int kChunk = 16;
+dim3 Runner::half_grid(const GroupParts& gp, int kinds, bool ring, bool rec, bool illum,
+                       int places) const {
+  int per = 1, y = 1;
+  for (const StepArgs& a : gp.args) per = std::max(per, a.hper);
+  // chunks of at most kChunk columns, evenly filled
+  const int most = std::max(1, kChunk / tile_), n = (per + most - 1) / most;
+  const int x = (per + n - 1) / n, chunks = (per + x - 1) / x;
+  const int row = kBZ * tile_ * 8 * x * chunks;  // items of a grid row of every chunk
+  for (const StepArgs& a : gp.args) {
+    const int items = ((ring || rec || illum) && a.ring ? (a.ringlen + 63) / 64 * 64 : 0) +
+                      (rec ? a.nrec : 0) + (illum && a.illum && nf_ > 1 ? a.Nb / 4 : 0);
+    y = std::max(y, kinds * a.hgz + (items + row - 1) / row);
   }
-  return cache.map(key, all, out);
+  return dim3((unsigned)(8 * x), (unsigned)y, (unsigned)(chunks * places));
+}
+void Runner::half_stress(const GroupParts& gp, int it, int ring) {
+  const int pf = nf_ * (int)gp.args.size();
+  go(k_half_stress<2>, half_grid(gp, 1, ring >= 0, false, true, pf), dim3(kBZ, tile_),
+     cache.steps + gp.steps, it, ring, nf_, sf_, pf);
+}
+void Runner::half_vel(const GroupParts& gp, int it, int ring) {
+  const int pf = nf_ * (int)gp.args.size();
+  go(k_half_vel<2>, half_grid(gp, 1, ring >= 0, true, false, pf), dim3(kBZ, tile_),
+     cache.steps + gp.steps, it, ring, nf_, sf_, pf);
+}
+void Runner::half_a(const GroupParts& gp, int it, int ring, int kinds) {
+  go(nb_ > 1 ? k_half_bwd_a<true> : k_half_bwd_a<false>, half_grid(gp, 2, ring >= 0, false, false, (int)gp.args.size()),
+     dim3(kBZ, tile_, nb_), cache.backs + gp.backs, it, ring, kinds, (int)gp.args.size());
+}
+void Runner::half_b(const GroupParts& gp, int it, int ring, int kinds) {
+  go(nb_ > 1 ? k_half_bwd_b<true> : k_half_bwd_b<false>, half_grid(gp, 2, ring >= 0, false, false, (int)gp.args.size()),
+     dim3(kBZ, tile_, nb_), cache.backs + gp.backs, it, ring, kinds, (int)gp.args.size());
+}
+// exact adjoint (with the reversal of the step)
+void Runner::exact_a(const GroupParts& gp, int it, int first) {
+  go(nb_ > 1 ? k_exact_a<true> : k_exact_a<false>, half_grid(gp, 1, true, false, false, (int)gp.args.size()),
+     dim3(kBZ, tile_, nb_), cache.backs + gp.backs, xt_, it, ring_at(it), first,
+     (int)gp.args.size());
+}
+void Runner::exact_b(const GroupParts& gp, int it) {
+  go(nb_ > 1 ? k_exact_b<true> : k_exact_b<false>, half_grid(gp, 1, true, false, false, (int)gp.args.size()),
+     dim3(kBZ, tile_, nb_), cache.backs + gp.backs, xt_, srcwin_, it, ring_at(it),
+     (int)gp.args.size());
+}
+
+dim3 Runner::whole_grid(const GroupParts& gp, bool backward) const {
+  int x = 8, y = 1;
+  for (size_t q = 0; q < gp.args.size(); q++) {
+    const StepArgs& a = gp.args[q];
+    x = std::max(x, 8 * a.per);
+    if (backward) y = std::max(y, a.gz + backs_[gp.backs + q].rgz);
+  }
+  if (!backward) {
+    const int row = kBZ * kStepW * x;
+    for (const StepArgs& a : gp.args) {
+      const int items = (a.ring ? (a.ringlen + 63) / 64 * 64 : 0) + (a.nrec + 63) / 64 * 64 +
+                        (a.illum && nf_ > 1 ? a.Nb / 4 : 0);
+      y = std::max(y, a.gz + (items + row - 1) / row);
+    }
+  }
+  return dim3((unsigned)x, (unsigned)y, (unsigned)((backward ? 1 : nf_) * (int)gp.args.size()));
+}
+void Runner::step_fwd(const GroupParts& gp, int odd, int it) {
+  const StepArgs* t = cache.steps + gp.steps + (size_t)(1 + odd) * gp.args.size();
+  const dim3 grid = whole_grid(gp, false), b(kBZ, kStepW);
+  const int ring = gp.args[0].ring ? ring_at(it) : -1;
+  go(k_step_fwd, grid, b, t, it, ring, nf_, sf_);
+}
+void Runner::step_bwd(const GroupParts& gp, int fodd, int aodd, int it) {
+  const BackArgs* t = cache.backs + gp.backs + (size_t)(1 + fodd + 2 * aodd) * gp.args.size();
+  const dim3 grid = whole_grid(gp, true), b(kBZ, kStepW);
+  go(k_step_bwd, grid, b, t, it, ring_at(it));
+}
+
+Status Runner::forward(const GroupParts& gp, int t0, int t1,
+                       const std::function<Status(int, int)>& before) {
+  const bool ring = !gp.args.empty() && gp.args[0].ring;
+  auto row = [&](int it) { return ring ? ring_at(it) : -1; };
+  if (!whole_f_ && ring && t1 > t0) ring_all<true>(gp, t0, 0, 3);  // the stresses that step t0 reads
+  for (int it = t0; it < t1; it++) {
+    const bool smp = it % sample_every == 0;
+    const int odd = whole_f_ ? (t1 - it) & 1 : 0;
+    TRY(before(it, odd));
+    if (whole_f_) {
+      d0->launch("step_fwd", smp, [&] { step_fwd(gp, odd, it); });
+    } else {
+      d0->launch("stress_fwd", smp, [&] { half_stress(gp, it, row(it)); });
+      d0->launch("vel_fwd", smp, [&] { half_vel(gp, it, it + 1 < t1 ? row(it + 1) : -1); });
+    }
+  }
+  return Status::Ok();
+}
+
+// ring components [c0, c1) of step it saved from the main state buffers
+template <bool Save>
+void Runner::ring_all(const GroupParts& gp, int it, int c0, int c1) {
+  int n = 0;
+  for (const StepArgs& a : gp.args) n = std::max(n, a.ringlen);
+  hipLaunchKernelGGL((k_ring<Save>), dim3((n + 255) / 256, 1, (unsigned)gp.args.size()), dim3(256), 0,
+                     st, cache.steps + gp.steps, ring_at(it), c0, c1);
+}
+
+void Runner::record_last(const GroupParts& gp, int it) {
+  int n = 0;
+  for (const StepArgs& a : gp.args) n = std::max(n, a.nrec);
+  if (n)
+    hipLaunchKernelGGL(k_record, dim3((n + 255) / 256, 1, (unsigned)gp.args.size()), dim3(256), 0, st,
+                       cache.steps + gp.steps, it);
+}
+
+void Runner::illum_last(const GroupParts& gp) {
+  int n = 0;
+  for (const StepArgs& a : gp.args) n = std::max(n, a.illum ? a.Nb / 4 : 0);
+  if (n)
+    hipLaunchKernelGGL(k_illum, dim3((n + 255) / 256, 1, (unsigned)gp.args.size()), dim3(256), 0, st,
+                       cache.steps + gp.steps);
+}
+
+Status Runner::clear_second(const GroupParts& gp) {
+  for (size_t q = 0; q < gp.member.size(); q++) {
+    DeviceState& d = *M[gp.member[q]].d;
+    const size_t n = (size_t)gp.n[q] * d.g.N * sizeof(float);
+    HIP_TRY(hipMemsetAsync(d.fwd2, 0, kWaveComps * n, st));
+    HIP_TRY(hipMemsetAsync(d.mem2, 0, kMemComps * n, st));
+  }
+  return Status::Ok();
 }
 
 // Checkpoint j >= 1 of the shots of a group: the 5 wavefield components and
@@ -2765,17 +1637,17 @@ Status Runner::maps_of(const GroupParts& gp, const char* kind, DevMap& out) {
 // [j-1] x {wavefields [shot of the sweep][5][cell], memory variables
 // [shot of the sweep][8][cell]}: a group's shots are one contiguous block of
 // each.
-Status Runner::snapshot(const GroupParts& gp, int sg0, int j, bool save) {
-  for (size_t q = 0; q < gp.parts.size(); q++) {
+Status Runner::snapshot(const GroupParts& gp, int sg0, int j, bool save, int odd) {
+  for (size_t q = 0; q < gp.member.size(); q++) {
     DeviceState& d = *M[gp.member[q]].d;
-    const int s0 = gp.parts[q].g.s0, n = gp.parts[q].g.ns;
+    const int s0 = gp.s0[q], n = gp.n[q];
     const int rows_m = std::min(S, d.g.ns), rs = s0 - shots_in(M[gp.member[q]], sg0);
     const size_t N = (size_t)d.g.N;
     float* cp = d.snap + (size_t)(j - 1) * (kWaveComps + kMemComps) * rows_m * N;
     float* cw = cp + (size_t)rs * kWaveComps * N;
     float* cm = cp + (size_t)rows_m * kWaveComps * N + (size_t)rs * kMemComps * N;
-    float* fw = d.shot(d.fwd, kWaveComps, s0);
-    float* fm = d.shot(d.mem, kMemComps, s0);
+    float* fw = odd ? d.fwd2 : d.shot(d.fwd, kWaveComps, s0);
+    float* fm = odd ? d.mem2 : d.shot(d.mem, kMemComps, s0);
     const size_t bw = (size_t)n * kWaveComps * N * sizeof(float);
     const size_t bm = (size_t)n * kMemComps * N * sizeof(float);
     HIP_TRY(hipMemcpyAsync(save ? cw : fw, save ? fw : cw, bw, hipMemcpyDeviceToDevice, st));
@@ -2810,7 +1682,6 @@ Status Runner::run(int calc_id) {
     return Status::Err(FWIFLOW_ERR_ARG, "at most " + std::to_string(kMaxPartsTable) + " plans per job");
   HIP_TRY(hipSetDevice(d0->dev));
   st = d0->stream;
-  blk = dim3(kBZ, d0->tile_x);
   nSteps = d0->g.nSteps;
   if_res = calc_id != 2;
   withAdj = calc_id == 1;
@@ -2846,19 +1717,32 @@ Status Runner::run(int calc_id) {
   if (cap < 1) return Status::Err(FWIFLOW_ERR_SHAPE, "grid too large for one shot per launch");
   gf = std::min(gf, cap);
   gb = std::min(gb, cap);
+  // two columns a workgroup unless the caller chose: against four, 580x1780
+  // 59.5 / 59.8 ms, 364x964 44.4 / 45.2, 224x448 39.6 / 41.8 (smaller steps of
+  // the work that the SIMDs share out)
+  tile_ = c0.tile_auto ? 2 : c0.tile_x;
+  slice(gf, sf_, nf_);
+  nb_ = threads_per_cell(gb);
+  whole_f_ = !c0.arena && waves(gf) <= kWholeFwdWaves;
+  whole_b_ = !c0.arena && withAdj && gb <= kWholeBwdShots && waves(gb) <= kWholeBwdWaves;
+  for (const Member& m : M) whole_b_ = whole_b_ && !m.d->adjoint && m.d->inj_folded;
   // memory plan of a gradient run: rows per sweep S and checkpoint interval K
   const int steps = std::max(1, nSteps - 1);  // forward steps 0 .. nSteps-2
   double budget = c0.ring_budget;
   if (withAdj && c0.arena && M.size() == 1) {
     // scratch-backed plan: ring + checkpoints get what the scratch array has
     // left after the gradient run's other buffers (adjoint fields, C-PML
-    // adjoint memory variables, accumulators, misfit partials, maps)
+    // adjoint memory variables, accumulators, misfit partials, injection and
+    // argument tables)
     const DeviceState& d = c0;
     const double N = (double)d.g.N, F = (double)d.F();
     const double other = 4.0 * ((d.adj ? 0 : 5 * F) + (d.madj ? 0 : 8 * F) +
                                 (d.acc ? 0 : 5 * N) + (d.grad ? 0 : 3 * N) +
                                 (d.stf_grad ? 0 : (double)d.g.ns * nSteps) +
                                 (d.illum_on && !d.illum ? N : 0)) +
+                         (d.inj ? 0 : sizeof(ColInj) * (double)d.g.ns * d.g.nx +
+                                          4.0 * (d.icells.size() + d.iptrs.size() + d.irids.size())) +
+                         (2 * sizeof(StepArgs) + sizeof(BackArgs)) * (double)rows +
                          8.0 * rows * kPartials + (1 << 20);
     budget = std::min(budget, std::max(1.0, (double)d.arena->free_bytes() - other));
   }
@@ -2940,6 +1824,27 @@ Status Runner::run(int calc_id) {
       d.last_ring_bytes = (long long)(rf * sizeof(float));
       d.last_snap_bytes = (long long)(sf * sizeof(float));
     }
+    // the second states start out zero and stay zero outside the update region
+    auto second = [&](float*& p, int& have, int need, int comps) -> Status {
+      if (have >= need) return Status::Ok();
+      d.release(p, (size_t)have * comps * N);
+      have = 0;
+      TRY(d.alloc(&p, (size_t)need * comps * N));
+      have = need;
+      HIP_TRY(hipMemsetAsync(p, 0, (size_t)need * comps * N * sizeof(float), st));
+      return Status::Ok();
+    };
+    if (whole_f_ || whole_b_) {
+      const int n2 = std::min(d.g.ns, whole_b_ || ckpt ? std::max(gf, gb) : gf);
+      TRY(second(d.fwd2, d.shots2, n2, kWaveComps));
+      TRY(second(d.mem2, d.mshots2, n2, kMemComps));
+    }
+    if (whole_b_) {
+      const int n2 = std::min(d.g.ns, gb);
+      TRY(second(d.adj2, d.ashots2, n2, kWaveComps));
+      if (ckpt) TRY(second(d.madj2, d.xshots2, n2, kMemComps));
+    }
+    if (withAdj) TRY(ensure_injection(d));
     const int npart = (int)sweeps.size() * kPartials;
     if (d.npartial < npart) {
       d.release(d.partial, (size_t)d.npartial);
@@ -2957,7 +1862,6 @@ Status Runner::run(int calc_id) {
     }
   }
   // parts of every group (pointing at the buffers above)
-  table.clear();
   std::vector<std::vector<GroupParts>> FG(sweeps.size()), RG(sweeps.size()), BG(sweeps.size());
   for (size_t j = 0; j < sweeps.size(); j++) {
     for (RowRange rr : FR[j]) FG[j].push_back(parts_of(rr, sweeps[j].r0, kPhFwd));
@@ -2966,7 +1870,8 @@ Status Runner::run(int calc_id) {
       if (ckpt) RG[j].push_back(parts_of(rr, sweeps[j].r0, kPhRec));
     }
   }
-  if (!table.empty()) TRY(cache.upload_table(table));
+  TRY(cache.upload(steps_, cache.steps, cache.steps_cap));
+  TRY(cache.upload(backs_, cache.backs, cache.backs_cap));
   // clear the run's state
   for (const Member& m : M) {
     DeviceState& d = *m.d;
@@ -2981,35 +1886,20 @@ Status Runner::run(int calc_id) {
       HIP_TRY(hipMemsetAsync(d.stf_grad, 0, (size_t)d.g.ns * nSteps * sizeof(float), st));
     }
   }
-  const int Uf = d0->unroll_fwd, Ub = d0->unroll;
-  // every 64th step of each launch kind is bracketed by timing events (when
-  // timing is on): events between launches cost the stream about 2% at
-  // every 8th step
-  const int sample_every = 64;
   for (size_t j = 0; j < sweeps.size(); j++) {
     const RowRange sw = sweeps[j];
     // ------------------------------------------------------ forward
     for (const GroupParts& gp : FG[j]) {
-      DevMap mS, mV;
-      TRY(maps_of(gp, "S", mS));
-      TRY(maps_of(gp, "V", mV));
-      const StepLaunch sS = step(gp, mS), sV = step(gp, mV);
-      if (ckpt) {  // checkpoint copies between the steps: no graph
-        for (int it = 0; it <= nSteps - 2; it++) {
-          const bool smp = it % sample_every == 0;
-          if (it > 0 && it % K == 0) TRY(snapshot(gp, sw.r0, it / K, true));
-          d0->launch("stress_fwd", smp, [&] { fwd_stress(sS, it, Uf); });
-          d0->launch("vel_fwd", smp, [&] { fwd_vel(sV, it, Uf); });
-        }
-      } else {
-        TRY(replay(graph_key("F", gp, {&mS, &mV}), [&] {
-          for (int it = 0; it <= nSteps - 2; it++) {
-            const bool smp = it % sample_every == 0;
-            d0->launch("stress_fwd", smp, [&] { fwd_stress(sS, it, Uf); });
-            d0->launch("vel_fwd", smp, [&] { fwd_vel(sV, it, Uf); });
-          }
-        }));
-      }
+      if (whole_f_ && (steps & 1)) TRY(clear_second(gp));
+      auto save = [&](int it, int odd) -> Status {
+        return ckpt && it > 0 && it % K == 0 ? snapshot(gp, sw.r0, it / K, true, odd) : Status::Ok();
+      };
+      if (ckpt)  // checkpoint copies between the steps: no graph
+        TRY(forward(gp, 0, nSteps - 1, save));
+      else
+        TRY(replay(graph_key("F", gp), [&] { (void)forward(gp, 0, nSteps - 1, save); }));
+      if (whole_f_) record_last(gp, nSteps - 1);
+      if (nf_ > 1 && nSteps > 1) illum_last(gp);
     }
     HIP_TRY(hipGetLastError());
     // ------------------------------------------------------ residual
@@ -3033,35 +1923,18 @@ Status Runner::run(int calc_id) {
     // ------------------------------------------------------ backward
     for (size_t q = 0; q < BG[j].size(); q++) {
       const GroupParts& gp = BG[j][q];
-      for (size_t p = 0; p < gp.parts.size(); p++) {
+      for (size_t p = 0; p < gp.member.size(); p++) {
         DeviceState& d = *M[gp.member[p]].d;
-        const int s0 = gp.parts[p].g.s0, n = gp.parts[p].g.ns;
+        const int s0 = gp.s0[p], n = gp.n[p];
         TRY(d.zero_shots(d.adj, kWaveComps, s0, n, st));
         TRY(d.zero_shots(ckpt ? d.madj : d.mem, kMemComps, s0, n, st));
       }
-      DevMap mA, mB, mAV, mAS, mRV, mRS, mRW, mR;
-      TRY(maps_of(gp, "A", mA));
-      TRY(maps_of(gp, "R", mR));
-      TRY(maps_of(gp, "B", mB));
-      TRY(maps_of(gp, "AV", mAV));
-      TRY(maps_of(gp, "AS", mAS));
-      TRY(maps_of(gp, "RV", mRV));
-      const StepLaunch sA = step(gp, mA), sB = step(gp, mB), sAV = step(gp, mAV),
-                       sAS = step(gp, mAS), sRV = step(gp, mRV), sR = step(gp, mR);
-      StepLaunch sRS, sRW;
-      if (ckpt) {
-        TRY(maps_of(RG[j][q], "S", mRS));
-        TRY(maps_of(RG[j][q], "W", mRW));
-        sRS = step(RG[j][q], mRS);
-        sRW = step(RG[j][q], mRW);
-      }
       // residual injection of step t for plans without the folded injection
       auto inject = [&](int t) {
-        for (size_t p = 0; p < gp.parts.size(); p++) {
+        for (size_t p = 0; p < gp.member.size(); p++) {
           DeviceState& d = *M[gp.member[p]].d;
-          if (d.rec_at) continue;
-          const int s0 = gp.parts[p].g.s0, s1 = s0 + gp.parts[p].g.ns;
-          const int c0 = d.coff[s0], nc = d.coff[s1] - c0;
+          if (d.inj_folded) continue;
+          const int c0 = d.coff[gp.s0[p]], nc = d.coff[gp.s0[p] + gp.n[p]] - c0;
           if (nc > 0)
             hipLaunchKernelGGL(k_res_inject, dim3((nc + 255) / 256), dim3(256), 0, st, d.g,
                                d.adj, d.icell, d.iptr, d.irid, c0, nc,
@@ -3073,98 +1946,84 @@ Status Runner::run(int calc_id) {
       // re-materialises (v^it, sigma^it) in its two launches.  No initial
       // adjoint step: sample 0 is not recorded, and sample it+1 enters at
       // reverse step it.
-      const Part* xp = gp.parts.empty() ? nullptr : &gp.parts[0];
       auto xsegment = [&](int t0, int t1) {
         for (int it = t1 - 1; it >= t0; it--) {
           const bool smp = it % sample_every == 0;
-          d0->launch("exact_a", smp, [&] { exact_a(*xp, it, it == nSteps - 2 ? 1 : 0); });
+          d0->launch("exact_a", smp, [&] { exact_a(gp, it, it == nSteps - 2 ? 1 : 0); });
           inject(it + 1);
-          d0->launch("exact_b", smp, [&] { exact_b(*xp, it); });
+          d0->launch("exact_b", smp, [&] { exact_b(gp, it); });
         }
       };
       if (d0->adjoint) {
-        for (size_t p = 0; p < gp.parts.size(); p++) {
+        for (size_t p = 0; p < gp.member.size(); p++) {
           DeviceState& d = *M[gp.member[p]].d;
-          HIP_TRY(hipMemsetAsync(d.xt, 0, (size_t)gp.parts[p].g.ns * 8 * d.g.N * sizeof(float), st));
+          HIP_TRY(hipMemsetAsync(d.xt, 0, (size_t)gp.n[p] * 8 * d.g.N * sizeof(float), st));
         }
         xt_ = d0->xt;
         srcwin_ = d0->srcwin;
       }
       if (d0->adjoint && !ckpt) {
-        if (nSteps >= 2)
-          TRY(replay(graph_key("X", gp, {}) + "/" + std::to_string((uintptr_t)xt_),
-                     [&] { xsegment(0, steps); }));
+        if (nSteps >= 2) TRY(replay(graph_key("X", gp), [&] { xsegment(0, steps); }));
         HIP_TRY(hipGetLastError());
         continue;
       }
+      // the initial adjoint step at t = nSteps-1 (libCUFD.cu:353-373), in place;
+      // adj_stress shares its launch with the first reversal where half steps follow
+      auto initial = [&] {
+        half_a(gp, nSteps - 1, -1, 1);
+        inject(nSteps - 1);
+        if (nSteps < 2 || whole_b_) half_b(gp, nSteps - 1, -1, 1);
+      };
       // reverse steps t1-1 .. t0 of one segment; `last` is the segment that
       // ends at nSteps-1
+      int aodd = 0;  // whole steps: the adjoint state is in its second buffers
       auto segment = [&](int t0, int t1, bool last) {
-        if (last)
-          bwd_b(sB, nSteps - 1, Ub);  // adj_stress(nSteps-1) + rev_vel(nSteps-2)
-        else
-          bwd_b(sRV, t1, Ub);         // rev_vel(t1-1)
+        if (whole_b_) {
+          int fodd = 0;
+          for (int it = t1 - 1; it >= t0; it--, fodd ^= 1, aodd ^= 1)
+            d0->launch("step_bwd", it % sample_every == 0, [&] { step_bwd(gp, fodd, aodd, it); });
+          return;
+        }
+        // adj_stress(nSteps-1) + rev_vel(nSteps-2), or rev_vel(t1-1)
+        half_b(gp, t1, ring_at(t1 - 1), last ? 3 : 2);
         for (int it = t1 - 1; it >= t0; it--) {
           const bool smp = it % sample_every == 0;
-          if (d0->pair_a) {
-            d0->launch("bwd_pair_a", smp, [&] { bwd_a(sA, it, Ub); });
-          } else {  // the halves as launches of their own (same kernel, one kind each)
-            d0->launch("rev_stress", smp, [&] { bwd_a(sR, it, Ub); });
-            d0->launch("adj_vel", smp, [&] { bwd_a(sAV, it, Ub); });
-          }
+          d0->launch("bwd_pair_a", smp, [&] { half_a(gp, it, ring_at(it), 3); });
           inject(it);
-          if (it > t0 && d0->pair_b) {
-            d0->launch("bwd_pair_b", smp, [&] { bwd_b(sB, it, Ub); });
-          } else if (it > t0) {
-            d0->launch("adj_stress", smp, [&] { bwd_b(sAS, it, Ub); });
-            d0->launch("rev_vel", smp, [&] { bwd_b(sRV, it, Ub); });
-          } else {
-            bwd_b(sAS, it, Ub);
-          }
+          if (it > t0)
+            d0->launch("bwd_pair_b", smp, [&] { half_b(gp, it, ring_at(it - 1), 3); });
+          else
+            half_b(gp, it, -1, 1);
         }
       };
       if (!ckpt) {
-        // the whole backward sweep of the group, from the initial adjoint
-        // step at t = nSteps-1 (libCUFD.cu:353-373)
-        TRY(replay(graph_key("B", gp, {&mA, &mB, &mAV, &mAS, &mRV, &mR}), [&] {
-          bwd_a(sAV, nSteps - 1, Ub);
-          inject(nSteps - 1);
-          if (nSteps < 2)
-            bwd_b(sAS, nSteps - 1, Ub);
-          else
-            segment(0, steps, true);
+        TRY(replay(graph_key("B", gp), [&] {
+          initial();
+          if (nSteps >= 2) segment(0, steps, true);
         }));
         HIP_TRY(hipGetLastError());
         continue;
       }
       // checkpoints: each segment is recomputed from its checkpoint, then
       // reversed with its ring
-      if (d0->adjoint) {
-        if (nSteps < 2) continue;
-      } else {
-        bwd_a(sAV, nSteps - 1, Ub);
-        inject(nSteps - 1);
-        if (nSteps < 2) {
-          bwd_b(sAS, nSteps - 1, Ub);
-          continue;
-        }
-      }
+      if (!d0->adjoint) initial();
+      if (nSteps < 2) continue;
+      const GroupParts& rg = RG[j][q];
       const int nseg = (steps + K - 1) / K;
       for (int jj = nseg - 1; jj >= 0; jj--) {
         const int t0 = jj * K, t1 = std::min(t0 + K, steps);
+        const int odd = whole_f_ ? (t1 - t0) & 1 : 0;  // the buffers that the segment starts from
         if (jj == 0) {
-          for (size_t p = 0; p < gp.parts.size(); p++) {
+          for (size_t p = 0; p < gp.member.size(); p++) {
             DeviceState& d = *M[gp.member[p]].d;
-            TRY(d.zero_shots(d.fwd, kWaveComps, gp.parts[p].g.s0, gp.parts[p].g.ns, st));
-            TRY(d.zero_shots(d.mem, kMemComps, gp.parts[p].g.s0, gp.parts[p].g.ns, st));
+            TRY(d.zero_shots(d.fwd, kWaveComps, gp.s0[p], gp.n[p], st));
+            TRY(d.zero_shots(d.mem, kMemComps, gp.s0[p], gp.n[p], st));
           }
+          if (odd) TRY(clear_second(rg));
         } else {
-          TRY(snapshot(RG[j][q], sw.r0, jj, false));
+          TRY(snapshot(rg, sw.r0, jj, false, odd));
         }
-        for (int it = t0; it < t1; it++) {
-          fwd_stress(sRS, it, Uf);
-          fwd_vel(sRW, it, Uf);
-        }
+        TRY(forward(rg, t0, t1, [](int, int) { return Status::Ok(); }));
         if (d0->adjoint)
           xsegment(t0, t1);
         else
