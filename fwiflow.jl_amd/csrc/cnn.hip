@@ -10,16 +10,16 @@
 // gradients, one plane per channel.  Parameters are one flat FP32 vector:
 // per layer W [Cout][Cin][3][3] then b [Cout].
 //
+// The layers are products on the FP32 matrix cores (weights x pixels).  An FP32
+// MFMA adds its products to the accumulator one by one in the order of k, each
+// a fused multiply-add, so every sum has a fixed order: channels, then taps
+// (k = 9 ci + t) from the bias on; pixels of a 16x16 tile row by row; tiles.
+//
 // Kernels:
-//   k_conv       3x3 convolution over a 16x16 pixel tile per workgroup, the
-//                input tile (+1 halo) staged in LDS 8 channels at a time,
-//                weights read as wave-uniform scalars; epilogues: hidden
-//                layer (store z and GELU(z) in BF16), output layer (FP32),
-//                input-gradient (multiply by GELU'(z) of the layer below)
-//   k_flip       W [Cout][Cin][ky][kx] -> W' [Cin][Cout][2-ky][2-kx], so the
-//                input gradient is the forward convolution with W'
-//   k_wgrad      weight / bias gradient partial sums of one 16x16 tile, both
-//                operands staged in LDS; one thread per (Cin, tap) pair
+//   k_conv32     3x3 convolution to 32 channels (hidden layers; input gradients,
+//                as the convolution with the transposed and flipped weights)
+//   k_conv3      the output layer
+//   k_wgrad      weight / bias gradient partial sums of one 16x16 tile
 //   k_sum_rows   deterministic reduction of the per-tile partials
 //   k_loss_grad  masked MSE and its gradient
 //   k_adam       Adam update
@@ -50,11 +50,12 @@ namespace {
       return Status::Err(FWIFLOW_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-constexpr int kTile = 16;       // output tile edge
+constexpr int kTile = 16;       // tile edge of the weight gradient
 constexpr int kHalo = kTile + 2;
-constexpr int kCinChunk = 8;    // input channels staged in LDS per pass
 constexpr int kMaxC = 32;
 
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short bf16_t;
 
 // FP32 -> BF16, round to nearest even (finite inputs; NaN kept as NaN)
@@ -84,137 +85,236 @@ __device__ inline float load_act<bf16_t>(const bf16_t* p, size_t i) {
   return from_bf16(p[i]);
 }
 
-enum Epilogue { kHidden = 0, kOutput = 1, kInputGrad = 2 };
-
-// out[co][y][x] = b[co] + sum_{ci,ky,kx} w[co][ci][ky][kx] in[ci][y+ky-1][x+kx-1]
-template <typename TIn, int COUT, int EPI>
-__global__ __launch_bounds__(256) void k_conv(const TIn* __restrict__ in, int Cin, int H, int W,
-                                              const float* __restrict__ w,
-                                              const float* __restrict__ b,
-                                              float* __restrict__ out_f32,
-                                              bf16_t* __restrict__ z_bf16,
-                                              bf16_t* __restrict__ a_bf16,
-                                              const bf16_t* __restrict__ zin) {
-  __shared__ float tile[kCinChunk][kHalo * kHalo];
-  const int tx = threadIdx.x % kTile, ty = threadIdx.x / kTile;
-  const int x0 = blockIdx.x * kTile, y0 = blockIdx.y * kTile;
-  const int x = x0 + tx, y = y0 + ty;
+// Pixels (xa .. xa + TX - 1, ya .. ya + TY - 1) of the first C of CIN channels
+// into lds[CIN][CS] (rows of TX pixels), zero outside the map and beyond C.  A
+// wave takes whole channels, so that a lane's pixels and their offsets are the
+// same for all of them.
+template <typename TIn, int CIN, int C, int TY, int TX, int CS, int NW>
+__device__ __forceinline__ void stage(const TIn* __restrict__ in, int H, int W, int xa, int ya, float* lds) {
+  constexpr int N = TX * TY, I = (N + 63) / 64;
   const size_t plane = (size_t)H * W;
-  float acc[COUT];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  size_t off[I];
+  bool ok[I];
 #pragma unroll
-  for (int co = 0; co < COUT; ++co) acc[co] = b ? b[co] : 0.f;
-  for (int c0 = 0; c0 < Cin; c0 += kCinChunk) {
-    const int nc = min(kCinChunk, Cin - c0);
-    __syncthreads();
-    for (int k = threadIdx.x; k < nc * kHalo * kHalo; k += 256) {
-      const int c = k / (kHalo * kHalo), r = k % (kHalo * kHalo);
-      const int yy = y0 - 1 + r / kHalo, xx = x0 - 1 + r % kHalo;
-      float v = 0.f;
-      if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-        v = load_act<TIn>(in, (size_t)(c0 + c) * plane + (size_t)yy * W + xx);
-      tile[c][r] = v;
-    }
-    __syncthreads();
-    for (int c = 0; c < nc; ++c) {
-      float v[9];
-#pragma unroll
-      for (int ky = 0; ky < 3; ++ky)
-#pragma unroll
-        for (int kx = 0; kx < 3; ++kx) v[ky * 3 + kx] = tile[c][(ty + ky) * kHalo + tx + kx];
-      const float* wc = w + (size_t)(c0 + c) * 9;
-#pragma unroll
-      for (int co = 0; co < COUT; ++co) {
-        const float* wk = wc + (size_t)co * Cin * 9;
-        float s = acc[co];
-#pragma unroll
-        for (int t = 0; t < 9; ++t) s += wk[t] * v[t];
-        acc[co] = s;
-      }
-    }
+  for (int i = 0; i < I; ++i) {
+    const int r = min(lane + 64 * i, N - 1), yy = ya + r / TX, xx = xa + r % TX;
+    ok[i] = yy >= 0 && yy < H && xx >= 0 && xx < W;
+    off[i] = (size_t)min(max(yy, 0), H - 1) * W + min(max(xx, 0), W - 1);
   }
-  if (x >= W || y >= H) return;
-  const size_t p = (size_t)y * W + x;
+#pragma unroll 2
+  for (int c = wave; c < CIN; c += NW) {
+    const TIn* p = in + (size_t)min(c, C - 1) * plane;
+    float v[I];
 #pragma unroll
-  for (int co = 0; co < COUT; ++co) {
-    const size_t o = (size_t)co * plane + p;
-    if (EPI == kHidden) {
-      z_bf16[o] = to_bf16(acc[co]);
-      a_bf16[o] = to_bf16(gelu(acc[co]));
-    } else if (EPI == kOutput) {
-      out_f32[o] = acc[co];
-    } else {  // input gradient of a hidden layer's activation -> of its z
-      out_f32[o] = acc[co] * gelu_grad(from_bf16(zin[o]));
-    }
+    for (int i = 0; i < I; ++i) v[i] = load_act<TIn>(p, off[i]);
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+      if (lane + 64 * i < N) lds[c * CS + lane + 64 * i] = ok[i] && c < C ? v[i] : 0.f;
   }
 }
 
-// W [Cout][Cin][3][3] -> W' [Cin][Cout][3][3] with the taps reversed
-__global__ void k_flip(const float* __restrict__ w, int Cout, int Cin, float* __restrict__ wf) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= Cout * Cin * 9) return;
-  const int t = k % 9, ci = (k / 9) % Cin, co = k / (9 * Cin);
-  wf[((size_t)ci * Cout + co) * 9 + (8 - t)] = w[k];
-}
+constexpr int kConvX = 32, kConvY = 8;  // pixels of a convolution's tile
+constexpr int kConvS = kConvX + 2;      // and of its row with the halo
 
-// Partial dW[co][ci][t] and db[co] of one 16x16 tile: thread (ci, t) sums over
-// the tile's pixels in[ci][p + tap t] * dz[co][p] for every co.
-template <typename TIn, int COUT>
-__global__ __launch_bounds__(320) void k_wgrad(const TIn* __restrict__ in, int Cin, int H, int W,
-                                               const float* __restrict__ dz,
-                                               float* __restrict__ part) {
-  extern __shared__ float sm[];
-  float* sin = sm;                              // [Cin][18*18]
-  float* sdz = sm + (size_t)Cin * kHalo * kHalo;  // [COUT][16*16]
-  const int x0 = blockIdx.x * kTile, y0 = blockIdx.y * kTile;
+enum Epilogue { kHidden = 0, kInputGrad = 1 };
+
+// out[m][y][x] = b[m] + sum_{c,ky,kx} w(m, c, ky, kx) in[c][y+ky-1][x+kx-1] for
+// 32 channels m; in has C channels (CIN, even, in LDS).  kHidden: w = W[m][c][t];
+// kInputGrad: W is the layer above's [C][32][9] and w = W[c][m][8 - t].
+//
+// Eight waves of a row of 32 pixels each; input (+1 halo) and weights in LDS (80
+// KB: two workgroups a compute unit), 9 matrix instructions per two channels:
+// 32 channels x 32 pixels x 2 products.  A lane's pixel operand for products k,
+// k + 1 differs between the wave's halves by one of three offsets.
+// Bound by the matrix cores (1.85 GFLOP at 224x448: 11.8 us at the card's 157
+// TFLOP/s, 15.4 with the last of 3.06 rows a SIMD), before and after them by the
+// load of the tile and the GELU.  224x448, 32 -> 32 channels: 107 -> 33 us
+// against one pixel a thread with weights as scalars and vector multiply-adds
+// (4 -> 32: 25 -> 15 us); four waves of two rows 36, of one row 40, two waves 53.
+template <typename TIn, int CIN, int C, int EPI>
+__global__ __launch_bounds__(64 * kConvY) void k_conv32(const TIn* __restrict__ in, int H, int W,
+                                                        const float* __restrict__ w,
+                                                        const float* __restrict__ b,
+                                                        float* __restrict__ out_f32,
+                                                        bf16_t* __restrict__ z_bf16,
+                                                        bf16_t* __restrict__ a_bf16,
+                                                        const bf16_t* __restrict__ zin) {
+  constexpr int NW = kConvY, K = CIN * 9, CH = (kConvY + 2) * kConvS, WS = 33;
+  __shared__ float tile[CIN * CH];
+  __shared__ float wk[K * WS];  // [k][channel]
+  const int x0 = blockIdx.x * kConvX, y0 = blockIdx.y * kConvY;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const size_t plane = (size_t)H * W;
-  for (int k = threadIdx.x; k < Cin * kHalo * kHalo; k += blockDim.x) {
-    const int c = k / (kHalo * kHalo), r = k % (kHalo * kHalo);
-    const int yy = y0 - 1 + r / kHalo, xx = x0 - 1 + r % kHalo;
-    float v = 0.f;
-    if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-      v = load_act<TIn>(in, (size_t)c * plane + (size_t)yy * W + xx);
-    sin[k] = v;
+  stage<TIn, CIN, C, kConvY + 2, kConvS, CH, NW>(in, H, W, x0 - 1, y0 - 1, tile);
+  {
+    // a wave takes whole channels: of the output, or of the layer above
+    constexpr int N = EPI == kInputGrad ? 288 : C * 9, M = EPI == kInputGrad ? C : 32, I = (N + 63) / 64;
+    int to[I];
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      const int r = lane + 64 * i;
+      to[i] = EPI == kInputGrad ? (8 - r % 9) * WS + r / 9 : r * WS;
+    }
+#pragma unroll 2
+    for (int m = wave; m < M; m += NW) {
+      float v[I];
+#pragma unroll
+      for (int i = 0; i < I; ++i) v[i] = w[m * N + min(lane + 64 * i, N - 1)];
+#pragma unroll
+      for (int i = 0; i < I; ++i)
+        if (lane + 64 * i < N) wk[to[i] + m * (EPI == kInputGrad ? 9 * WS : 1)] = v[i];
+    }
   }
-  for (int k = threadIdx.x; k < COUT * kTile * kTile; k += blockDim.x) {
-    const int c = k / (kTile * kTile), r = k % (kTile * kTile);
-    const int yy = y0 + r / kTile, xx = x0 + r % kTile;
-    sdz[k] = (yy < H && xx < W) ? dz[(size_t)c * plane + (size_t)yy * W + xx] : 0.f;
-  }
+  if (C < CIN)
+    for (int i = threadIdx.x; i < (CIN - C) * 9 * 32; i += 64 * NW)
+      wk[(C * 9 + i / 32) * WS + i % 32] = 0.f;
   __syncthreads();
-  const size_t nw = (size_t)COUT * Cin * 9;
-  float* pw = part + (size_t)(blockIdx.y * gridDim.x + blockIdx.x) * (nw + COUT);
-  const int j = threadIdx.x;
-  if (j < Cin * 9) {
-    const int ci = j / 9, t = j % 9, ky = t / 3, kx = t % 3;
-    float acc[COUT];
+  const int n = lane & 31, h = lane >> 5;
+  f32x16 acc;
 #pragma unroll
-    for (int co = 0; co < COUT; ++co) acc[co] = 0.f;
-    const float* si = sin + (size_t)ci * kHalo * kHalo;
-    for (int py = 0; py < kTile; ++py)
-      for (int px = 0; px < kTile; ++px) {
-        const float a = si[(py + ky) * kHalo + px + kx];
-        const int q = py * kTile + px;
+  for (int i = 0; i < 16; ++i) acc[i] = b ? b[8 * (i / 4) + 4 * h + i % 4] : 0.f;
+  const float* wp = wk + h * WS + n;
+  const float* tp = tile + wave * kConvS + n;
+#pragma unroll 2
+  for (int c = 0; c < CIN; c += 2, wp += 18 * WS, tp += 2 * CH) {
 #pragma unroll
-        for (int co = 0; co < COUT; ++co) acc[co] += a * sdz[co * kTile * kTile + q];
-      }
+    for (int j = 0; j < 9; ++j) {
+      constexpr auto off = [](int k) { return k / 9 * CH + k % 9 / 3 * kConvS + k % 3; };
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(wp[2 * j * WS], tp[h ? off(2 * j + 1) : off(2 * j)], acc, 0, 0, 0);
+    }
+  }
+  const int x = x0 + n, y = y0 + wave;
+  if (x >= W || y >= H) return;
 #pragma unroll
-    for (int co = 0; co < COUT; ++co) pw[((size_t)co * Cin + ci) * 9 + t] = acc[co];
-  } else if (j < Cin * 9 + COUT) {
-    const int co = j - Cin * 9;
-    float s = 0.f;
-    for (int q = 0; q < kTile * kTile; ++q) s += sdz[co * kTile * kTile + q];
-    pw[nw + co] = s;
+  for (int i = 0; i < 16; ++i) {
+    const size_t o = (size_t)(8 * (i / 4) + 4 * h + i % 4) * plane + (size_t)y * W + x;
+    if (EPI == kHidden) {
+      z_bf16[o] = to_bf16(acc[i]);
+      a_bf16[o] = to_bf16(gelu(acc[i]));
+    } else {  // gradient of the activation -> of its z
+      out_f32[o] = acc[i] * gelu_grad(from_bf16(zin[o]));
+    }
   }
 }
 
-// out[k] = sum_r rows[r][k] (fixed order: deterministic)
-__global__ void k_sum_rows(const float* __restrict__ rows, int nrows, int n,
-                           float* __restrict__ out) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  float s = 0.f;
-  for (int r = 0; r < nrows; ++r) s += rows[(size_t)r * n + k];
-  out[k] = s;
+// The output layer: 32 -> 3 channels, FP32 result.  Three rows would leave nine
+// tenths of a matrix instruction idle: one pixel a thread, weights as scalars.
+// 224x448: 28 -> 14 us with all channels of the tile loaded at once.
+__global__ __launch_bounds__(256) void k_conv3(const bf16_t* __restrict__ in, int H, int W,
+                                               const float* __restrict__ w,
+                                               const float* __restrict__ b, float* __restrict__ out) {
+  constexpr int CH = (kConvY + 2) * kConvS;
+  __shared__ float tile[32 * CH];
+  const int x0 = blockIdx.x * kConvX, y0 = blockIdx.y * kConvY;
+  stage<bf16_t, 32, 32, kConvY + 2, kConvS, CH, 4>(in, H, W, x0 - 1, y0 - 1, tile);
+  __syncthreads();
+  const int n = threadIdx.x & 31, x = x0 + n, y = y0 + (threadIdx.x >> 5);
+  const float* t = tile + (threadIdx.x >> 5) * kConvS + n;
+  float acc[3] = {b[0], b[1], b[2]};
+#pragma unroll 2
+  for (int c = 0; c < 32; ++c, t += CH)
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      const float v = t[k / 3 * kConvS + k % 3];
+#pragma unroll
+      for (int co = 0; co < 3; ++co) acc[co] += w[co * 288 + c * 9 + k] * v;
+    }
+  if (x >= W || y >= H) return;
+#pragma unroll
+  for (int co = 0; co < 3; ++co) out[(size_t)co * H * W + (size_t)y * W + x] = acc[co];
+}
+
+// Partial weight and bias gradients of one 16x16 tile: column n = t CIN + ci of
+// part[co][NCOL] sums in[ci][p + tap t] dz[co][p] over the tile's pixels p, the
+// last column dz[co][p].  Both operands in LDS; one wave per 32 columns (COUT =
+// 32: 32x32x2 products) or 64 (COUT = 3: sixteen 4x4x1 blocks, 3 of 4 rows
+// used).  Bound by the matrix cores (17 us at 224x448 with the last workgroups)
+// after the tile's load.  224x448: 32 x 32 channels 120 -> 39 us, 4 x 32 73 ->
+// 15, 32 x 3 31 -> 17, against a thread per (ci, tap) with vector multiply-adds
+// (49, 23 and 24 with the tile's pixels taken one by one).
+template <int CIN>
+constexpr int kCols = CIN * 9 + 1;
+template <int CIN, int COUT>
+constexpr int kWgradThreads = COUT == 32 ? (CIN == 32 ? 640 : 256) : 320;
+template <typename TIn, int CIN, int COUT>
+__global__ __launch_bounds__((kWgradThreads<CIN, COUT>)) void k_wgrad(const TIn* __restrict__ in, int H, int W,
+                                                                    const float* __restrict__ dz,
+                                                                    float* __restrict__ part) {
+  constexpr int T = kWgradThreads<CIN, COUT>, CS = kHalo * kHalo + 1, DS = kTile * kTile + 1;
+  constexpr int NCOL = kCols<CIN>;
+  __shared__ float sin[CIN * CS];
+  __shared__ float sdz[COUT * DS];
+  const int x0 = blockIdx.x * kTile, y0 = blockIdx.y * kTile;
+  stage<TIn, CIN, CIN, kHalo, kHalo, CS, T / 64>(in, H, W, x0 - 1, y0 - 1, sin);
+  stage<float, COUT, COUT, kTile, kTile, DS, T / 64>(dz, H, W, x0, y0, sdz);
+  __syncthreads();
+  float* pw = part + (size_t)(blockIdx.y * gridDim.x + blockIdx.x) * COUT * NCOL;
+  constexpr int COLS = COUT == 32 ? 32 : 64;  // of a wave
+  const int lane = threadIdx.x & 63, col0 = ((int)threadIdx.x >> 6) * COLS;
+  const int col = col0 + lane % COLS;
+  if (col0 >= NCOL) return;
+  const int cc = min(col, NCOL - 2), t = cc / CIN;  // the bias column reads any operand
+  const float* sb = sin + cc % CIN * CS + t / 3 * kHalo + t % 3;
+  const bool one = col == NCOL - 1;
+  if (COUT == 32) {
+    const int h = lane >> 5;
+    const float* sa = sdz + (lane & 31) * DS + h;
+    f32x16 acc{};
+    for (int py = 0; py < kTile; ++py)
+#pragma unroll
+      for (int j = 0; j < kTile / 2; ++j) {
+        const float v = sb[py * kHalo + 2 * j + h];
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(sa[py * kTile + 2 * j], one ? 1.f : v, acc, 0, 0, 0);
+      }
+    if (col < NCOL)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) pw[(8 * (i / 4) + 4 * h + i % 4) * NCOL + col] = acc[i];
+  } else {
+    const float* sa = sdz + min(lane & 3, COUT - 1) * DS;
+    f32x4 acc{};
+    for (int py = 0; py < kTile; ++py)
+#pragma unroll
+      for (int j = 0; j < kTile; ++j) {
+        const float v = sb[py * kHalo + j];
+        acc = __builtin_amdgcn_mfma_f32_4x4x1f32(sa[py * kTile + j], one ? 1.f : v, acc, 0, 0, 0);
+      }
+    if (col < NCOL)
+#pragma unroll
+      for (int i = 0; i < COUT; ++i) pw[i * NCOL + col] = acc[i];
+  }
+}
+
+// grads of a layer from its partials [row][co][t CIN + ci, bias]: the rows are
+// added in order.  32 columns a workgroup; 16 half waves fetch 256 rows at a
+// time into LDS, one adds them up.  Bound by the reads' latency (224x448: 392
+// rows): 93 -> 6.7 us against one thread a column and its loads in series.
+constexpr int kSumRows = 256;
+__global__ __launch_bounds__(512) void k_sum_rows(const float* __restrict__ rows, int nrows, int Cin,
+                                                  int Cout, float* __restrict__ out) {
+  __shared__ float s[kSumRows][32];
+  const int ncol = Cin * 9 + 1, n = Cout * ncol;
+  const int c = threadIdx.x & 31, g = threadIdx.x >> 5, k = blockIdx.x * 32 + c;
+  const int kc = min(k, n - 1);
+  float sum = 0.f;
+  for (int r0 = 0; r0 < nrows; r0 += kSumRows) {
+    const int m = min(kSumRows, nrows - r0);
+    float v[kSumRows / 16];
+#pragma unroll
+    for (int i = 0; i < kSumRows / 16; ++i)
+      v[i] = rows[(size_t)(r0 + min(g + 16 * i, m - 1)) * n + kc];
+    if (r0) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kSumRows / 16; ++i) s[g + 16 * i][c] = v[i];
+    __syncthreads();
+    if (g == 0) {
+#pragma unroll 16
+      for (int i = 0; i < m; ++i) sum += s[i][c];
+    }
+  }
+  if (g || k >= n) return;
+  const int co = k / ncol, q = k % ncol;
+  out[q == ncol - 1 ? Cout * Cin * 9 + co : (co * Cin + q % Cin) * 9 + q / Cin] = sum;
 }
 
 // loss = 0.5 / count * sum mask (out - target)^2 over C planes; d out
@@ -266,7 +366,6 @@ struct CnnState {
   size_t off[kLayers] = {};  // start of each layer's W in the flat vector
   int nparams = 0;
   float *params = nullptr, *grads = nullptr, *m1 = nullptr, *m2 = nullptr;
-  float *wflip = nullptr;     // flipped weights of one layer
   float *x0 = nullptr;        // network input [4][H][W]
   bf16_t *z[3] = {}, *a[3] = {};  // hidden pre-activations and activations
   float *out = nullptr, *target = nullptr, *mask = nullptr;
@@ -295,95 +394,54 @@ struct CnnState {
 
 namespace {
 
-template <typename TIn>
-void launch_conv(CnnState& s, int layer, const TIn* in, int epi, float* out_f32, bf16_t* zb,
-                 bf16_t* ab, const bf16_t* zin, const float* w, const float* bias, int Cin,
-                 int Cout) {
-  const dim3 grid = s.tiles();
-  if (Cout == 32) {
-    if (epi == kHidden)
-      hipLaunchKernelGGL((k_conv<TIn, 32, kHidden>), grid, dim3(256), 0, s.stream, in, Cin, s.H,
-                         s.W, w, bias, out_f32, zb, ab, zin);
-    else if (epi == kOutput)
-      hipLaunchKernelGGL((k_conv<TIn, 32, kOutput>), grid, dim3(256), 0, s.stream, in, Cin, s.H,
-                         s.W, w, bias, out_f32, zb, ab, zin);
-    else
-      hipLaunchKernelGGL((k_conv<TIn, 32, kInputGrad>), grid, dim3(256), 0, s.stream, in, Cin,
-                         s.H, s.W, w, bias, out_f32, zb, ab, zin);
-  } else if (Cout == 3) {
-    hipLaunchKernelGGL((k_conv<TIn, 3, kOutput>), grid, dim3(256), 0, s.stream, in, Cin, s.H, s.W,
-                       w, bias, out_f32, zb, ab, zin);
-  } else {  // Cout == 4: input gradient of the first layer is never needed
-  }
-  (void)layer;
+template <typename TIn, int CIN, int C, int EPI>
+void conv32(CnnState& s, const TIn* in, const float* w, const float* bias, float* out_f32, bf16_t* zb,
+            bf16_t* ab, const bf16_t* zin) {
+  hipLaunchKernelGGL((k_conv32<TIn, CIN, C, EPI>),
+                     dim3((s.W + kConvX - 1) / kConvX, (s.H + kConvY - 1) / kConvY), dim3(64 * kConvY), 0,
+                     s.stream, in, s.H, s.W, w, bias, out_f32, zb, ab, zin);
 }
 
-template <typename TIn>
-void launch_wgrad(CnnState& s, const TIn* in, int Cin, int Cout, const float* dz, float* gw) {
+template <typename TIn, int CIN, int COUT>
+void wgrad(CnnState& s, const TIn* in, const float* dz, float* gw) {
   const dim3 grid = s.tiles();
-  const size_t lds = ((size_t)Cin * kHalo * kHalo + (size_t)Cout * kTile * kTile) * sizeof(float);
-  if (Cout == 32)
-    hipLaunchKernelGGL((k_wgrad<TIn, 32>), grid, dim3(320), lds, s.stream, in, Cin, s.H, s.W, dz,
-                       s.part);
-  else
-    hipLaunchKernelGGL((k_wgrad<TIn, 3>), grid, dim3(320), lds, s.stream, in, Cin, s.H, s.W, dz,
-                       s.part);
-  const int n = Cout * Cin * 9 + Cout;
-  hipLaunchKernelGGL(k_sum_rows, dim3((n + 255) / 256), dim3(256), 0, s.stream, s.part,
-                     (int)(grid.x * grid.y), n, gw);
+  hipLaunchKernelGGL((k_wgrad<TIn, CIN, COUT>), grid, dim3(kWgradThreads<CIN, COUT>), 0, s.stream, in,
+                     s.H, s.W, dz, s.part);
+  hipLaunchKernelGGL(k_sum_rows, dim3((COUT * kCols<CIN> + 31) / 32), dim3(512), 0, s.stream, s.part,
+                     (int)(grid.x * grid.y), CIN, COUT, gw);
 }
 
 Status forward(CnnState& s) {
-  const float* P = s.params;
-  // layer 0: FP32 input
-  launch_conv<float>(s, 0, s.x0, kHidden, nullptr, s.z[0], s.a[0], nullptr, P + s.off[0],
-                     P + s.off[0] + kCout[0] * kCin[0] * 9, kCin[0], kCout[0]);
+  auto W = [&](int l) { return s.params + s.off[l]; };
+  auto B = [&](int l) { return W(l) + kCout[l] * kCin[l] * 9; };
+  conv32<float, 4, 4, kHidden>(s, s.x0, W(0), B(0), nullptr, s.z[0], s.a[0], nullptr);
   for (int l = 1; l < 3; ++l)
-    launch_conv<bf16_t>(s, l, s.a[l - 1], kHidden, nullptr, s.z[l], s.a[l], nullptr,
-                        P + s.off[l], P + s.off[l] + kCout[l] * kCin[l] * 9, kCin[l], kCout[l]);
-  launch_conv<bf16_t>(s, 3, s.a[2], kOutput, s.out, nullptr, nullptr, nullptr, P + s.off[3],
-                      P + s.off[3] + kCout[3] * kCin[3] * 9, kCin[3], kCout[3]);
+    conv32<bf16_t, 32, 32, kHidden>(s, s.a[l - 1], W(l), B(l), nullptr, s.z[l], s.a[l], nullptr);
+  hipLaunchKernelGGL(k_conv3, dim3((s.W + kConvX - 1) / kConvX, (s.H + kConvY - 1) / kConvY), dim3(32 * kConvY), 0, s.stream,
+                     s.a[2], s.H, s.W, W(3), B(3), s.out);
   CNN_HIP(hipGetLastError());
   return Status::Ok();
 }
 
 // loss and parameter gradients for the staged input / target / mask
-Status backward(CnnState& s, double* loss) {
+Status backward(CnnState& s, const float* mask, double* loss) {
   const size_t plane = (size_t)s.H * s.W;
-  // mask population for the mean
-  std::vector<float> hm(plane);
-  CNN_HIP(hipMemcpyAsync(hm.data(), s.mask, plane * sizeof(float), hipMemcpyDeviceToHost,
-                         s.stream));
-  CNN_HIP(hipStreamSynchronize(s.stream));
-  double cnt = 0;
-  for (float v : hm) cnt += v != 0.f;
-  const float inv = cnt > 0 ? (float)(1.0 / (cnt * kCout[3])) : 0.f;
+  // mask population for the mean, from the caller's copy while the forward runs
+  size_t cnt = 0;
+  for (size_t k = 0; k < plane; ++k) cnt += mask[k] != 0.f;
+  const float inv = cnt > 0 ? (float)(1.0 / ((double)cnt * kCout[3])) : 0.f;
   hipLaunchKernelGGL(k_loss_grad, dim3(s.lblocks), dim3(256), 0, s.stream, s.out, s.target,
                      s.mask, kCout[3], plane, inv, s.d0, s.lpart);
-  float* G = s.grads;
-  const float* P = s.params;
-  // layer 3 (output): dz = d out
-  launch_wgrad<bf16_t>(s, s.a[2], kCin[3], kCout[3], s.d0, G + s.off[3]);
-  float* dcur = s.d0;
-  float* dnext = s.d1;
-  for (int l = 3; l >= 1; --l) {
-    // gradient w.r.t. z of layer l-1: conv of dz_l with flipped W_l, times GELU'(z_{l-1})
-    const int n = kCout[l] * kCin[l] * 9;
-    hipLaunchKernelGGL(k_flip, dim3((n + 255) / 256), dim3(256), 0, s.stream, P + s.off[l],
-                       kCout[l], kCin[l], s.wflip);
-    const int cin_t = kCout[l], cout_t = kCin[l];  // transposed roles
-    const dim3 grid = s.tiles();
-    if (cout_t == 32) {
-      hipLaunchKernelGGL((k_conv<float, 32, kInputGrad>), grid, dim3(256), 0, s.stream, dcur,
-                         cin_t, s.H, s.W, s.wflip, nullptr, dnext, nullptr, nullptr, s.z[l - 1]);
-    }
-    // weight gradient of layer l-1
-    if (l - 1 == 0)
-      launch_wgrad<float>(s, s.x0, kCin[0], kCout[0], dnext, G + s.off[0]);
-    else
-      launch_wgrad<bf16_t>(s, s.a[l - 2], kCin[l - 1], kCout[l - 1], dnext, G + s.off[l - 1]);
-    std::swap(dcur, dnext);
-  }
+  // per layer: weight gradient from dz, then dz of the layer below
+  auto W = [&](int l) { return s.params + s.off[l]; };
+  auto G = [&](int l) { return s.grads + s.off[l]; };
+  wgrad<bf16_t, 32, 3>(s, s.a[2], s.d0, G(3));
+  conv32<float, 4, 3, kInputGrad>(s, s.d0, W(3), nullptr, s.d1, nullptr, nullptr, s.z[2]);
+  wgrad<bf16_t, 32, 32>(s, s.a[1], s.d1, G(2));
+  conv32<float, 32, 32, kInputGrad>(s, s.d1, W(2), nullptr, s.d0, nullptr, nullptr, s.z[1]);
+  wgrad<bf16_t, 32, 32>(s, s.a[0], s.d0, G(1));
+  conv32<float, 32, 32, kInputGrad>(s, s.d0, W(1), nullptr, s.d1, nullptr, nullptr, s.z[0]);
+  wgrad<float, 4, 32>(s, s.x0, s.d1, G(0));
   CNN_HIP(hipGetLastError());
   std::vector<double> lp(s.lblocks);
   CNN_HIP(hipMemcpyAsync(lp.data(), s.lpart, lp.size() * sizeof(double), hipMemcpyDeviceToHost,
@@ -412,15 +470,6 @@ Status Cnn::create(int gpu, int height, int width, unsigned seed) {
   s.W = width;
   CNN_HIP(hipSetDevice(gpu));
   CNN_HIP(hipStreamCreate(&s.stream));
-  // the weight-gradient tiles stage up to 74 KB in LDS (gfx950: 160 KB per CU)
-  const int lds_max = (int)(((size_t)kMaxC * kHalo * kHalo + (size_t)kMaxC * kTile * kTile) *
-                            sizeof(float));
-  CNN_HIP(hipFuncSetAttribute((const void*)k_wgrad<bf16_t, 32>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_max));
-  CNN_HIP(hipFuncSetAttribute((const void*)k_wgrad<bf16_t, 3>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_max));
-  CNN_HIP(hipFuncSetAttribute((const void*)k_wgrad<float, 32>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_max));
   size_t o = 0;
   for (int l = 0; l < kLayers; ++l) {
     s.off[l] = o;
@@ -443,7 +492,6 @@ Status Cnn::create(int gpu, int height, int width, unsigned seed) {
   TRY(s.alloc(&s.grads, o));
   TRY(s.alloc(&s.m1, o));
   TRY(s.alloc(&s.m2, o));
-  TRY(s.alloc(&s.wflip, (size_t)kMaxC * kMaxC * 9));
   TRY(s.alloc(&s.x0, 4 * plane));
   for (int l = 0; l < 3; ++l) {
     TRY(s.alloc(&s.z[l], (size_t)kMaxC * plane));
@@ -514,7 +562,7 @@ Status Cnn::gradients(const float* input, const float* target, const float* mask
   CNN_HIP(hipSetDevice(s.dev));
   TRY(stage(input, target, mask));
   TRY(fwiflow::forward(s));
-  TRY(backward(s, loss));
+  TRY(backward(s, mask, loss));
   if (grad)
     CNN_HIP(hipMemcpy(grad, s.grads, s.nparams * sizeof(float), hipMemcpyDeviceToHost));
   return Status::Ok();
