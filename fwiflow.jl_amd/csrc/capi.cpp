@@ -52,10 +52,7 @@ Status host_checks(int calc_id, int group_size, const int* shot_ids, const char*
   TRY(fwiflow::parse_para(para_fname, para));
   if (!Lambda || !Mu || !Den) return Status::Err(FWIFLOW_ERR_ARG, "null model pointer");
   TRY(fwiflow::parse_survey(para, group_size, shot_ids, sv));
-  std::vector<float> lam, mu, den;
-  float cp_max = 0.f;
-  fwiflow::model_to_zfast(para, Lambda, Mu, Den, false, lam, mu, den, cp_max);
-  TRY(fwiflow::check_courant(para, cp_max));
+  TRY(fwiflow::check_courant(para, fwiflow::model_cp_max(para, Lambda, Mu, Den)));
   if (calc_id != 2) {
     for (const auto& sh : sv.shots) {
       const std::string fn = para.data_dir + "/Shot" + std::to_string(sh.id) + ".bin";

@@ -233,31 +233,20 @@ Status parse_survey(const Para& p, int group_size, const int* shot_ids, Survey& 
   return Status::Ok();
 }
 
-void model_to_zfast(const Para& p, const double* Lambda, const double* Mu, const double* Den,
-                    bool input_zfast, std::vector<float>& lam, std::vector<float>& mu,
-                    std::vector<float>& den, float& cp_max) {
-  const int nz = p.nz, nx = p.nx;
-  const size_t n = (size_t)nz * nx;
-  lam.resize(n);
-  mu.resize(n);
-  den.resize(n);
-  for (int j = 0; j < nx; j++)
-    for (int i = 0; i < nz; i++) {
-      const size_t src = input_zfast ? (size_t)j * nz + i : (size_t)i * nx + j;
-      const size_t dst = (size_t)j * nz + i;
-      lam[dst] = (float)(Lambda[src] * 1e6);
-      mu[dst] = (float)(Mu[src] * 1e6);
-      den[dst] = (float)Den[src];
+// Vp as velInit computes it (utilities.cu:119-121), max for the Courant number:
+// one square root, of the largest argument (rounding keeps the order).  A first
+// cell without one decides, others are passed over.
+float model_cp_max(const Para& p, const double* Lambda, const double* Mu, const double* Den) {
+  auto square = [&](size_t k) {
+    return ((float)(Lambda[k] * 1e6) + 2.0 * (float)(Mu[k] * 1e6)) / (float)Den[k];
+  };
+  double m = square(0);
+  if (m >= 0.0)
+    for (size_t k = 1, n = (size_t)p.nz * p.nx; k < n; k++) {
+      const double q = square(k);
+      m = q > m ? q : m;
     }
-  // Vp as velInit computes it (utilities.cu:119-121), max for the Courant number
-  float m = 0.f;
-  bool first = true;
-  for (size_t k = 0; k < n; k++) {
-    const float cp = (float)std::sqrt((lam[k] + 2.0 * mu[k]) / den[k]);
-    if (first || cp > m) m = cp;
-    first = false;
-  }
-  cp_max = m;
+  return (float)std::sqrt(m);
 }
 
 Status check_courant(const Para& p, float cp_max) {

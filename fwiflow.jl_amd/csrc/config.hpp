@@ -69,11 +69,8 @@ Status check_calc_id(int calc_id);
 // Geometry bounds that the kernels rely on (ring rows inside the update region etc.).
 Status check_geometry(const Para& p);
 
-// Host model preparation: transpose TF row-major [NZ][NX] to z-fastest and
-// MPa -> Pa (libCUFD.cu:72-78); also returns max Vp for the Courant check.
-void model_to_zfast(const Para& p, const double* Lambda, const double* Mu, const double* Den,
-                    bool input_zfast, std::vector<float>& lam, std::vector<float>& mu,
-                    std::vector<float>& den, float& cp_max);
+// Largest Vp of a model in MPa, as libCUFD.cu:72-96 takes it for the Courant check.
+float model_cp_max(const Para& p, const double* Lambda, const double* Mu, const double* Den);
 // utilities.cu:225-240
 Status check_courant(const Para& p, float cp_max);
 

@@ -375,6 +375,55 @@ __global__ void k_transpose(const float* __restrict__ in, float* __restrict__ ou
   }
 }
 
+// Model arrays in and gradients out: in [rows][cols] -> out [cols][rows], one
+// array per blockIdx.z, in another type.  `scaled`: the first arrays in units of
+// 1e6 (the caller's moduli are in MPa).
+// Host arrays cross the bus as the caller has them and are turned here (TF's
+// row-major [NZ][NX] to z-fastest, libCUFD.cu:72-78, and back, 480-486): the
+// host's strided passes were bound by their cache misses.  A model of 608x1780
+// 6.4 -> 0.8 ms, of 364x964 1.7 -> 0.3; gradients of the latter 1.3 -> 0.7.
+struct Turn {
+  const void* in[3];
+  void* out[3];
+};
+template <typename TI, typename TO>
+__global__ __launch_bounds__(256) void k_turn(Turn t, int rows, int cols, int scaled) {
+  __shared__ TI tile[32][33];
+  const TI* in = (const TI*)t.in[blockIdx.z];
+  TO* out = (TO*)t.out[blockIdx.z];
+  const int c0 = blockIdx.x * 32, r0 = blockIdx.y * 32;
+  for (int k = threadIdx.y; k < 32; k += 8)
+    if (r0 + k < rows && c0 + (int)threadIdx.x < cols)
+      tile[k][threadIdx.x] = in[(size_t)(r0 + k) * cols + c0 + threadIdx.x];
+  __syncthreads();
+  for (int k = threadIdx.y; k < 32; k += 8)
+    if (c0 + k < cols && r0 + (int)threadIdx.x < rows) {
+      const TI v = tile[threadIdx.x][k];
+      out[(size_t)(c0 + k) * rows + r0 + threadIdx.x] = (int)blockIdx.z < scaled ? (TO)(v * 1e6) : (TO)v;
+    }
+}
+
+// Largest Vp as velInit computes it (utilities.cu:119-121), one partial per
+// workgroup; NaNs are passed over (the host looks at the first cell's itself).
+__global__ __launch_bounds__(256) void k_vp_max(const double* __restrict__ lam, const double* __restrict__ mu,
+                                                const double* __restrict__ den, size_t n,
+                                                float* __restrict__ part) {
+  __shared__ float red[256];
+  float m = -1.f;  // below every square root
+  for (size_t k = (size_t)blockIdx.x * 256 + threadIdx.x; k < n; k += (size_t)gridDim.x * 256) {
+    const float l = (float)(lam[k] * 1e6), u = (float)(mu[k] * 1e6), d = (float)den[k];
+    const float cp = (float)sqrt((l + 2.0 * u) / d);
+    if (cp > m) m = cp;
+  }
+  red[threadIdx.x] = m;
+  __syncthreads();
+  for (int s = 128; s > 0; s >>= 1) {
+    if ((int)threadIdx.x < s) red[threadIdx.x] = fmaxf(red[threadIdx.x], red[threadIdx.x + s]);
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+}
+
 }  // namespace
 
 // ===================================================================== host
@@ -965,15 +1014,29 @@ static Status ensure_injection(DeviceState& d) {
 Status Plan::set_model(const double* Lambda, const double* Mu, const double* Den, bool zfast) {
   if (!d_) return Status::Err(FWIFLOW_ERR_ARG, "plan not created");
   if (!Lambda || !Mu || !Den) return Status::Err(FWIFLOW_ERR_ARG, "null model pointer");
-  std::vector<float> lam, mu, den;
-  model_to_zfast(para, Lambda, Mu, Den, zfast, lam, mu, den, cp_max);
-  TRY(check_courant(para, cp_max));
   DeviceState& d = *d_;
   HIP_TRY(hipSetDevice(d.dev));
-  const size_t nb = (size_t)d.g.N * sizeof(float);
-  HIP_TRY(hipMemcpyAsync(d.lam, lam.data(), nb, hipMemcpyHostToDevice, d.stream));
-  HIP_TRY(hipMemcpyAsync(d.mu, mu.data(), nb, hipMemcpyHostToDevice, d.stream));
-  HIP_TRY(hipMemcpyAsync(d.den, den.data(), nb, hipMemcpyHostToDevice, d.stream));
+  // staged in the forward memory variables (32 bytes a cell; every run clears them)
+  const size_t n = (size_t)d.g.N;
+  double* const in = (double*)d.mem;
+  const double* host[3] = {Lambda, Mu, Den};
+  for (int k = 0; k < 3; k++)
+    HIP_TRY(hipMemcpyAsync(in + k * n, host[k], n * sizeof(double), hipMemcpyHostToDevice, d.stream));
+  const int blocks = (int)std::max<size_t>(1, std::min<size_t>(512, n / 512));
+  float* const part = (float*)(in + 3 * n);
+  hipLaunchKernelGGL(k_vp_max, dim3(blocks), dim3(256), 0, d.stream, in, in + n, in + 2 * n, n, part);
+  HIP_TRY(hipGetLastError());
+  std::vector<float> top(blocks);
+  HIP_TRY(hipMemcpyAsync(top.data(), part, blocks * sizeof(float), hipMemcpyDeviceToHost, d.stream));
+  HIP_TRY(hipStreamSynchronize(d.stream));
+  const float first = (float)std::sqrt(((float)(Lambda[0] * 1e6) + 2.0 * (float)(Mu[0] * 1e6)) / (float)Den[0]);
+  cp_max = std::isnan(first) ? first : *std::max_element(top.begin(), top.end());
+  TRY(check_courant(para, cp_max));
+  const dim3 blk(32, 8);
+  const Turn t{{in, in + n, in + 2 * n}, {d.lam, d.mu, d.den}};
+  const int rows = zfast ? 1 : d.g.nz, cols = zfast ? (int)n : d.g.nx;
+  hipLaunchKernelGGL((k_turn<double, float>), dim3((cols + 31) / 32, (rows + 31) / 32, 3), blk, 0, d.stream, t,
+                     rows, cols, 2);
   hipLaunchKernelGGL(k_model_init, dim3((d.g.nz + 255) / 256, d.g.nx), dim3(256), 0, d.stream,
                      d.g, d.mu, d.den, d.amu, d.ba, d.bb);
   HIP_TRY(hipGetLastError());
@@ -2165,16 +2228,17 @@ Status Plan::gradients(double* gL, double* gM, double* gD, double* gS) {
   HIP_TRY(hipSetDevice(d.dev));
   const int nz = d.g.nz, nx = d.g.nx;
   const size_t N = (size_t)d.g.N;
-  std::vector<float> h(3 * N);
-  HIP_TRY(hipMemcpy(h.data(), d.grad, 3 * N * sizeof(float), hipMemcpyDeviceToHost));
+  // z-fastest -> row-major [NZ][NX] (libCUFD.cu:480-486), in doubles
+  double* const out = (double*)d.mem;
+  const Turn t{{d.grad, d.grad + N, d.grad + 2 * N}, {out, out + N, out + 2 * N}};
+  hipLaunchKernelGGL((k_turn<float, double>), dim3((nz + 31) / 32, (nx + 31) / 32, 3), dim3(32, 8), 0,
+                     d.stream, t, nx, nz, 0);
+  HIP_TRY(hipGetLastError());
   double* outs[3] = {gL, gM, gD};
-  for (int k = 0; k < 3; k++) {
-    if (!outs[k]) continue;
-    const float* src = h.data() + k * N;
-    // z-fastest -> row-major [NZ][NX] (libCUFD.cu:480-486)
-    for (int i = 0; i < nz; i++)
-      for (int j = 0; j < nx; j++) outs[k][(size_t)i * nx + j] = src[(size_t)j * nz + i];
-  }
+  for (int k = 0; k < 3; k++)
+    if (outs[k])
+      HIP_TRY(hipMemcpyAsync(outs[k], out + k * N, N * sizeof(double), hipMemcpyDeviceToHost, d.stream));
+  HIP_TRY(hipStreamSynchronize(d.stream));
   if (gS) {
     std::vector<float> s((size_t)d.g.ns * d.g.nSteps);
     HIP_TRY(hipMemcpy(s.data(), d.stf_grad, s.size() * sizeof(float), hipMemcpyDeviceToHost));
@@ -2196,10 +2260,12 @@ Status Plan::illumination(double* out) {
   DeviceState& d = *d_;
   HIP_TRY(hipSetDevice(d.dev));
   const int nz = d.g.nz, nx = d.g.nx;
-  std::vector<float> h((size_t)d.g.N);
-  HIP_TRY(hipMemcpy(h.data(), d.illum, h.size() * sizeof(float), hipMemcpyDeviceToHost));
-  for (int i = 0; i < nz; i++)
-    for (int j = 0; j < nx; j++) out[(size_t)i * nx + j] = h[(size_t)j * nz + i];
+  const Turn t{{d.illum}, {d.mem}};
+  hipLaunchKernelGGL((k_turn<float, double>), dim3((nz + 31) / 32, (nx + 31) / 32, 1), dim3(32, 8), 0,
+                     d.stream, t, nx, nz, 0);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipMemcpyAsync(out, d.mem, (size_t)d.g.N * sizeof(double), hipMemcpyDeviceToHost, d.stream));
+  HIP_TRY(hipStreamSynchronize(d.stream));
   return Status::Ok();
 }
 
