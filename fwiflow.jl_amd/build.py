@@ -27,11 +27,16 @@ CXXFLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", "-Wextra", "-Wno-unused-param
 # packed-FP32 instructions are disabled for all device code.  Multiply-add
 # contraction is limited to single source expressions (-ffp-contract=on), so
 # the rounding of a stencil update depends on how it is written, not on the
-# kernel it is inlined into: the split, column-marching and tiled variants of
+# kernel it is inlined into: the one-launch and two-launch forms of
 # a step then agree to the last bit wherever they share an expression.
+# The first 16 words of a kernel's arguments arrive in scalar registers: a
+# workgroup of a short launch otherwise waits for them first (one of the 3.6 us
+# of a 64x84 step; 5% of that modelling run, 3-4% of 164x264 and 127x341
+# gradients, 1% at 580x1780).
 HIPFLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Wall",
             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-            "-ffp-contract=on", "-munsafe-fp-atomics"]
+            "-ffp-contract=on", "-munsafe-fp-atomics",
+            "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 # extra compiler definitions for A/B builds of engine switches (space separated)
 HIPFLAGS += os.environ.get("FWIFLOW_HIPFLAGS", "").split()
 
