@@ -25,7 +25,6 @@ class Cnn {
                     double* loss);
 
  private:
-  Status stage(const float* input, const float* target, const float* mask);
   std::unique_ptr<CnnState> s_;
 };
 
