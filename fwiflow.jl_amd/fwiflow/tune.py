@@ -1,7 +1,7 @@
 """Launch-shape autotuner: tile width and shots per launch, measured and cached.
 
-The engine's automatic shape (64 x 4 workgroups; shots per launch from the
-Infinity-Cache rule, round(224 MB / bytes per shot)) is a model; this module
+The engine's automatic shape (workgroups two columns wide, or one; shots per
+launch from the Infinity-Cache rule, round(224 MB / bytes per shot)) is a model; this module
 measures the neighbourhood of it on the caller's own grid and shot count and
 keeps the fastest, per (grid, C-PML, shot count), in a JSON cache
 (``FWIFLOW_TUNE_CACHE`` or ``~/.cache/fwiflow/launch.json``).
@@ -11,8 +11,8 @@ A candidate is timed on the caller's model over a shortened record
 carries over to the full record): one gradient run (calc_id 1) to warm up,
 then the best of ``repeats`` runs.  Shapes only change how the shots are
 grouped into launches, never the arithmetic of a cell, so every candidate
-gives the same data and, up to the order of the gradient sums over a
-launch's shots, the same gradients (tests/test_gpu.py checks each switch).
+gives the same data and, up to the order of the gradient sums over the
+launches, the same gradients (tests/test_gpu.py checks each switch).
 """
 from __future__ import annotations
 
