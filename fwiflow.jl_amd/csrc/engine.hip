@@ -1301,13 +1301,18 @@ constexpr int kMaxPartsTable = 31;  // plans of a job
 // computed twice and a second copy of the state in the caches.  Measured, two
 // launches / one: 168 waves 1.89 / 1.20 ms, 792: 14.6 / 12.4, 2046: 10.6 /
 // 10.1, 10752: 39.2 / 38.0, 23136: 45.5 / 44.9, 36500: 60.1 / 59.8, 53760:
-// 93 / 100, 142400: 59 / 79.  Backward (adjoint and reversal both recompute
-// their rim, twice the state is copied, and a thread walks all shots): one
-// shot of 792 waves 12.4 / 10.8 ms, 682: 6.98 / 6.61, 1792: 7.89 / 7.71, 3300:
-// 11.7 / 12.0; two shots of 168 waves each 7.37 / 7.00, 792: 16.0 / 14.6,
-// 1792: 10.1 / 10.8; four of 168: 8.3 / 10.3.
-constexpr double kWholeFwdWaves = 16384, kWholeBwdWaves = 2048;
-constexpr int kWholeBwdShots = 2;
+// 93 / 100, 142400: 59 / 79.
+//
+// Backward (adjoint and reversal both recompute their rim, twice the state is
+// copied, and the reversal's workgroups walk all shots, since their sums are
+// taken in order), in waves of the adjoint's whole-step tiles, two launches /
+// one, 400 steps: one shot of 84 waves 4.16 / 3.55 ms, 1023: 4.50 / 4.26, 1272:
+// 5.08 / 4.83, 2080: 6.06 / 5.67, 3300: 11.7 / 12.0 (601 steps); two shots of 84: 4.68 /
+// 3.72, 792: 15.0 / 14.7 (1000 steps), 1023: 5.56 / 5.75; three of 84: 5.33 / 4.30, 1023: 6.86 / 7.19;
+// four of 84: 5.37 / 5.11, 368: 16.5 / 14.8 (1000 steps); six of 84: 6.18 / 6.32.
+constexpr double kWholeFwdWaves = 16384;
+constexpr double kWholeBwdWaves = 1600, kWholeBwdWaves1 = 2304;  // several shots, one
+constexpr int kWholeBwdShots = 4;
 
 enum Phase { kPhFwd = 0, kPhRec = 1, kPhBwd = 2 };
 
@@ -1332,8 +1337,9 @@ class Runner {
   DeviceState* d0 = nullptr;
   hipStream_t st = nullptr;
   int nSteps = 0, rows = 0, gf = 1, gb = 1, S = 1, K = 0, nsnap = 0;
-  // shots per slice and slices of a forward launch, threads per cell of a backward one
-  int sf_ = 1, nf_ = 1, nb_ = 1;
+  // shots per slice and slices of a forward launch and of a whole backward step,
+  // threads per cell of a half one
+  int sf_ = 1, nf_ = 1, sa_ = 1, na_ = 1, nb_ = 1;
   bool if_res = false, withAdj = false, ckpt = false;
   int tile_ = 2;  // columns of a half step's workgroup
   bool whole_f_ = false, whole_b_ = false;  // whole-step launches (forward, reference's adjoint)
@@ -1398,7 +1404,7 @@ std::string Runner::graph_key(const char* phase, const GroupParts& gp) const {
   mix(ptrs, sizeof(ptrs));
   const size_t offs[2] = {gp.steps, gp.backs};
   mix(offs, sizeof(offs));
-  const int flags[] = {d0->timing ? 1 : 0, nSteps, sf_, nf_, nb_, whole_f_, whole_b_,
+  const int flags[] = {d0->timing ? 1 : 0, nSteps, sf_, nf_, sa_, na_, nb_, whole_f_, whole_b_,
                        tile_, withAdj};
   mix(flags, sizeof(flags));
   return std::string(phase) + "/" + std::to_string(h);
@@ -1627,7 +1633,7 @@ dim3 Runner::whole_grid(const GroupParts& gp, bool backward) const {
       y = std::max(y, a.gz + (items + row - 1) / row);
     }
   }
-  return dim3((unsigned)x, (unsigned)y, (unsigned)((backward ? 1 : nf_) * (int)gp.args.size()));
+  return dim3((unsigned)x, (unsigned)y, (unsigned)((backward ? na_ : nf_) * (int)gp.args.size()));
 }
 void Runner::step_fwd(const GroupParts& gp, int odd, int it) {
   const StepArgs* t = cache.steps + gp.steps + (size_t)(1 + odd) * gp.args.size();
@@ -1638,7 +1644,7 @@ void Runner::step_fwd(const GroupParts& gp, int odd, int it) {
 void Runner::step_bwd(const GroupParts& gp, int fodd, int aodd, int it) {
   const BackArgs* t = cache.backs + gp.backs + (size_t)(1 + fodd + 2 * aodd) * gp.args.size();
   const dim3 grid = whole_grid(gp, true), b(kBZ, kStepW);
-  go(k_step_bwd, grid, b, t, it, ring_at(it));
+  go(k_step_bwd, grid, b, t, it, ring_at(it), na_, sa_);
 }
 
 Status Runner::forward(const GroupParts& gp, int t0, int t1,
@@ -1785,13 +1791,18 @@ Status Runner::run(int calc_id) {
   // the work that the SIMDs share out)
   tile_ = c0.tile_auto ? 2 : c0.tile_x;
   slice(gf, sf_, nf_);
+  slice(gb, sa_, na_);
   nb_ = threads_per_cell(gb);
   // a workgroup of four threads a cell is one column wide: exact adjoint of 15
   // shots of 224x448 96.0 -> 94.0 ms, 20 shots of 224x520 68.8 -> 66.5, reference's
   // adjoint of 20 shots of 127x341 36.7 -> 36.0
   if (c0.tile_auto && withAdj && nb_ == 4) tile_ = 1;
   whole_f_ = !c0.arena && waves(gf) <= kWholeFwdWaves;
-  whole_b_ = !c0.arena && withAdj && gb <= kWholeBwdShots && waves(gb) <= kWholeBwdWaves;
+  double tiles = 0;
+  for (const Member& m : M)
+    tiles += (double)((m.d->g.nzA - 4 + kCoreZ - 1) / kCoreZ) * m.d->g.nx * std::min(gb, m.d->g.ns);
+  whole_b_ = !c0.arena && withAdj && gb <= kWholeBwdShots &&
+             tiles <= (gb == 1 ? kWholeBwdWaves1 : kWholeBwdWaves);
   for (const Member& m : M) whole_b_ = whole_b_ && !m.d->adjoint && m.d->inj_folded;
   // memory plan of a gradient run: rows per sweep S and checkpoint interval K
   const int steps = std::max(1, nSteps - 1);  // forward steps 0 .. nSteps-2

@@ -392,10 +392,9 @@ typedef const __attribute__((address_space(4))) BackArgs CBack;
 // and el_stress_adj.cu:22-104 on the core.  The memory variables of the
 // stress update are kept where they are ever read with a non-zero coefficient:
 // the C-PML layers and the stencil's 2-cell reach.
-__device__ __forceinline__ void step_adj(CBack& B, int strip, int bx, int it,
+__device__ __forceinline__ void step_adj(CBack& B, int lo, int hi, int strip, int bx, int it,
                                          float (&lds)[6][kStepW][kBZ]) {
   const auto& A = B.s;
-  const int hi = A.ns;
   const int lane = (int)threadIdx.x, j = wave_col(0);
   const int nz = A.nz, nx = A.nx, nzA = A.nzA, nPml = A.nPml, Nb = A.Nb;
   const float dt = A.dt, dz = A.dz, dx = A.dx, rdz = A.rdz, rdx = A.rdx;
@@ -422,7 +421,7 @@ __device__ __forceinline__ void step_adj(CBack& B, int strip, int bx, int it,
   const float amu_kzh = kdiv(amu, Z.Kh, Z.rh), amu_kxh = kdiv(amu, X.Kh, X.rh);
   auto kd64 = [](double v, float K, double r) { return K == 1.f ? v : ddiv2(v, (double)K, r); };
   const float* const row = B.res + (size_t)it * A.R;
-  for (int s = 0; s < hi; ++s) {
+  for (int s = lo; s < hi; ++s) {
     const int sw = s * kWaveComps * Nb, sm = s * kMemComps * Nb;
     const int zs = ((CInt*)A.zx)[2 * s], xs = ((CInt*)A.zx)[2 * s + 1];
     const __attribute__((address_space(4))) ColInj* ci =
@@ -667,17 +666,18 @@ __device__ __forceinline__ void step_rev(CBack& B, int strip, int bx, int it,
 // does not write in place), so they are workgroups of their own: the first
 // rows of the grid the adjoint's tiles, the rest the reversal's.
 __global__ __launch_bounds__(64 * kStepW) void k_step_bwd(const BackArgs* __restrict__ args, int it,
-                                                     int itr) {
+                                                     int itr, int slices, int per_slice) {
   // velocities z, x, and the adjoint's memory variables sxzx, sxx, sxzz, szz
   __shared__ float lds[6][kStepW][kBZ];
-  CBack& B = ((CBack*)args)[blockIdx.z];
+  const Place pl = place_of((int)blockIdx.z, slices, per_slice);
+  CBack& B = ((CBack*)args)[pl.part];
   const int xcd = (int)blockIdx.x & 7, q = (int)blockIdx.x >> 3;
   int strip = (int)blockIdx.y;
   if (strip < B.s.gz) {
     const int bx = xcd * B.s.per + q;
     if (q >= B.s.per || bx >= B.s.gx) return;
-    step_adj(B, strip, bx, it, lds);
-  } else {
+    step_adj(B, pl.lo, min(pl.hi, B.s.ns), strip, bx, it, lds);
+  } else if (!pl.slice) {  // all shots: their sums are taken in order
     strip -= B.s.gz;
     const int bx = xcd * B.rper + q;
     if (strip >= B.rgz || q >= B.rper || bx >= B.rgx) return;

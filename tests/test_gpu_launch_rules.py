@@ -5,7 +5,7 @@ arithmetic and the order of the sums over shots do not depend on the launch.
 
 ``cases`` names (nz, nx, shots, steps): grid edges around the 60 x 4 core of a
 whole step and the 64 x 2 tile of a half step (12 C-PML cells a side), one
-and two shots (whole backward steps), four and nine shots (two and four
+to four shots (whole backward steps), five and nine shots (two and four
 threads a cell, the last round of eight ragged), and a launch of more than
 16384 waves (two launches a forward step, shots in slices).
 """
@@ -24,6 +24,7 @@ CASES = {
     "two_strips_4_shots": (100, 62, 4, 90),
     "two_strips_long_4_shots": (100, 62, 4, 300),
     "core_plus_one_4_shots": (41, 63, 4, 150),
+    "core_plus_one_5_shots": (41, 60, 5, 150),
     "strip_plus_one_9_shots": (105, 63, 9, 61),
     "sliced_forward": (41, 331, 24, 60),
 }
