@@ -1912,15 +1912,22 @@ Status Runner::run(int calc_id) {
       HIP_TRY(hipMemsetAsync(p, 0, (size_t)need * comps * N * sizeof(float), st));
       return Status::Ok();
     };
-    if (whole_f_ || whole_b_) {
-      const int n2 = std::min(d.g.ns, whole_b_ || ckpt ? std::max(gf, gb) : gf);
-      TRY(second(d.fwd2, d.shots2, n2, kWaveComps));
-      TRY(second(d.mem2, d.mshots2, n2, kMemComps));
-    }
-    if (whole_b_) {
-      const int n2 = std::min(d.g.ns, gb);
-      TRY(second(d.adj2, d.ashots2, n2, kWaveComps));
-      if (ckpt) TRY(second(d.madj2, d.xshots2, n2, kMemComps));
+    auto seconds = [&]() -> Status {
+      if (whole_f_ || whole_b_) {
+        const int n2 = std::min(d.g.ns, whole_b_ || ckpt ? std::max(gf, gb) : gf);
+        TRY(second(d.fwd2, d.shots2, n2, kWaveComps));
+        TRY(second(d.mem2, d.mshots2, n2, kMemComps));
+      }
+      if (whole_b_) {
+        const int n2 = std::min(d.g.ns, gb);
+        TRY(second(d.adj2, d.ashots2, n2, kWaveComps));
+        if (ckpt) TRY(second(d.madj2, d.xshots2, n2, kMemComps));
+      }
+      return Status::Ok();
+    };
+    if (!seconds().ok()) {  // no room for them: two launches a step
+      (void)hipGetLastError();
+      whole_f_ = whole_b_ = false;
     }
     if (withAdj) TRY(ensure_injection(d));
     const int npart = (int)sweeps.size() * kPartials;
