@@ -1788,24 +1788,6 @@ Status Runner::run(int calc_id) {
   if (cap < 1) return Status::Err(FWIFLOW_ERR_SHAPE, "grid too large for one shot per launch");
   gf = std::min(gf, cap);
   gb = std::min(gb, cap);
-  // two columns a workgroup unless the caller chose: against four, 580x1780
-  // 59.5 / 59.8 ms, 364x964 44.4 / 45.2, 224x448 39.6 / 41.8 (smaller steps of
-  // the work that the SIMDs share out)
-  tile_ = c0.tile_auto ? 2 : c0.tile_x;
-  slice(gf, sf_, nf_);
-  slice(gb, sa_, na_);
-  nb_ = threads_per_cell(gb);
-  // a workgroup of four threads a cell is one column wide: exact adjoint of 15
-  // shots of 224x448 96.0 -> 94.0 ms, 20 shots of 224x520 68.8 -> 66.5, reference's
-  // adjoint of 20 shots of 127x341 36.7 -> 36.0
-  if (c0.tile_auto && withAdj && nb_ == 4) tile_ = 1;
-  whole_f_ = !c0.arena && waves(gf) <= kWholeFwdWaves;
-  double tiles = 0;
-  for (const Member& m : M)
-    tiles += (double)((m.d->g.nzA - 4 + kCoreZ - 1) / kCoreZ) * m.d->g.nx * std::min(gb, m.d->g.ns);
-  whole_b_ = !c0.arena && withAdj && gb <= kWholeBwdShots &&
-             tiles <= (gb == 1 ? kWholeBwdWaves1 : kWholeBwdWaves);
-  for (const Member& m : M) whole_b_ = whole_b_ && !m.d->adjoint && m.d->inj_folded;
   // memory plan of a gradient run: rows per sweep S and checkpoint interval K
   const int steps = std::max(1, nSteps - 1);  // forward steps 0 .. nSteps-2
   double budget = c0.ring_budget;
@@ -1863,6 +1845,32 @@ Status Runner::run(int calc_id) {
     FR[j] = split_even(sweeps[j].r0, sweeps[j].r1, gf);
     if (withAdj) BR[j] = split_even(sweeps[j].r0, sweeps[j].r1, gb);
   }
+  // launch forms, by the most rows that a forward launch (of a checkpointed run
+  // also the recomputation of a backward group) and a backward launch hold
+  int mf = 1, mb = 1;
+  for (size_t j = 0; j < sweeps.size(); j++) {
+    for (RowRange rr : FR[j]) mf = std::max(mf, rr.r1 - rr.r0);
+    for (RowRange rr : BR[j]) mb = std::max(mb, rr.r1 - rr.r0);
+  }
+  if (ckpt) mf = std::max(mf, mb);
+  // two columns a workgroup unless the caller chose: against four, 580x1780
+  // 59.5 / 59.8 ms, 364x964 44.4 / 45.2, 224x448 39.6 / 41.8 (smaller steps of
+  // the work that the SIMDs share out)
+  tile_ = c0.tile_auto ? 2 : c0.tile_x;
+  slice(mf, sf_, nf_);
+  slice(mb, sa_, na_);
+  nb_ = threads_per_cell(mb);
+  // a workgroup of four threads a cell is one column wide: exact adjoint of 15
+  // shots of 224x448 96.0 -> 94.0 ms, 20 shots of 224x520 68.8 -> 66.5, reference's
+  // adjoint of 20 shots of 127x341 36.7 -> 36.0
+  if (c0.tile_auto && withAdj && nb_ == 4) tile_ = 1;
+  whole_f_ = !c0.arena && waves(mf) <= kWholeFwdWaves;
+  double tiles = 0;
+  for (const Member& m : M)
+    tiles += (double)((m.d->g.nzA - 4 + kCoreZ - 1) / kCoreZ) * m.d->g.nx * std::min(mb, m.d->g.ns);
+  whole_b_ = !c0.arena && withAdj && mb <= kWholeBwdShots &&
+             tiles <= (mb == 1 ? kWholeBwdWaves1 : kWholeBwdWaves);
+  for (const Member& m : M) whole_b_ = whole_b_ && !m.d->adjoint && m.d->inj_folded;
   // buffers
   for (const Member& m : M) {
     DeviceState& d = *m.d;
@@ -1916,12 +1924,12 @@ Status Runner::run(int calc_id) {
     };
     auto seconds = [&]() -> Status {
       if (whole_f_ || whole_b_) {
-        const int n2 = std::min(d.g.ns, whole_b_ || ckpt ? std::max(gf, gb) : gf);
+        const int n2 = std::min(d.g.ns, whole_b_ ? std::max(mf, mb) : mf);
         TRY(second(d.fwd2, d.shots2, n2, kWaveComps));
         TRY(second(d.mem2, d.mshots2, n2, kMemComps));
       }
       if (whole_b_) {
-        const int n2 = std::min(d.g.ns, gb);
+        const int n2 = std::min(d.g.ns, mb);
         TRY(second(d.adj2, d.ashots2, n2, kWaveComps));
         if (ckpt) TRY(second(d.madj2, d.xshots2, n2, kMemComps));
       }

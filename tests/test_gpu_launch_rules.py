@@ -81,3 +81,23 @@ def test_launch_rules_match_oracle_and_each_other(oracle_mod, workspace, name, m
         e = rel(a, b) if np.abs(b).max() > 1e-30 else float(np.abs(a).max())
         say(name, mode, k, f"{e:.2e}")
         assert e <= (SEIS_TOL if k < 2 else GRAD_TOL), (k, e)
+
+
+@pytest.mark.parametrize("groups", [(1, 3), (2, 5), (3, 5), (5, 2)])
+def test_recomputed_groups_may_exceed_forward_groups(workspace, groups):
+    """Backward launches recompute their own shots from the checkpoints, also
+    more of them than a forward launch holds: the same gradients as with one
+    launch for all shots, bit for bit where the backward launches are alike."""
+    c = models.case_small(nz=41, nx=60, nSteps=150, nshots=5)
+    para, stf = models.write_case(c, workspace)
+    ids = list(range(5))
+    fwiflow.fwi_obs_op(*models.moduli(c, "true"), stf, 0, ids, para)
+    m = models.moduli(c, "start")
+    fwd, bwd = groups
+    with fwiflow.Plan(para, ids) as P:
+        P.set_launch(2, 5, bwd)
+        want = _run(P, m, stf, "reference", 17)
+        P.set_launch(2, fwd, bwd)
+        got = _run(P, m, stf, "reference", 17)
+    # (the illumination adds up another way over other forward launches)
+    assert not _differing(got[:1] + got[2:], want[:1] + want[2:])
