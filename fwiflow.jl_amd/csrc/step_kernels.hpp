@@ -17,8 +17,8 @@
 // first half's results, arguments in cached device memory and tiles by index
 // arithmetic (a map of tiles and arguments in the uncached kernel argument
 // segment cost 440 scalar instructions a wave): modelling of 2 shots of 64x84
-// 2.9 -> 1.25 ms for 300 steps, 164x264 x 1 shot 9.0 -> 4.7 ms for 1000, its
-// gradient 18.7 -> 10.9 ms.  16 columns a tile: 1.42 ms and 12.5 ms.
+// 2.9 -> 1.18 ms for 300 steps, 164x264 x 1 shot 9.0 -> 4.25 ms for 1000, its
+// gradient 18.7 -> 10.2 ms.  6, 10, 12 or 16 columns a tile: 14, 2, 8, 15% slower.
 
 constexpr int kStepW = 8;         // columns of a tile
 constexpr int kCoreZ = kBZ - 4;   // depth cells of its core
@@ -698,9 +698,9 @@ __global__ __launch_bounds__(64 * kStepW) void k_step_bwd(const BackArgs* __rest
 // ones; a kernel's registers are left to its loads (limited to 64, for 8 waves
 // a SIMD, the gradient there takes 618 ms instead of 531).  Microseconds a
 // launch at 580x1780, as one launch per half with tiles from a map before and
-// here: stress 30.8 -> 28.9, velocity 24.4 -> 25.3 (3.2 shots), adjoint velocity
+// here: stress 30.8 -> 28.5, velocity 24.4 -> 24.7 (4 shots), adjoint velocity
 // with reverse stress 40.0 -> 36.5, adjoint stress with reverse velocity 33.6 ->
-// 32.5 (2.7 shots).
+// 31.9 (2.7 shots).
 //
 // The grid: x tiles in XCD bands, each band in chunks of gridDim.x / 8 tiles;
 // strips along y, chunks x places (slices and parts) along z, chunks outermost.
@@ -1281,6 +1281,12 @@ __global__ __launch_bounds__(Sliced ? 1024 : 256) void k_half_bwd_b(
 // column is gated) Azx = Axz, Bzx = Bz and Bx = Bxz, so slots 3, 5 and 7 are
 // written and read only inside the frame, and a reader takes slots 2, 4 and 6
 // for neighbours outside it.
+// Bound by L2-miss traffic on large grids (580x1780, 2 shots: 33.1 -> 28.8 us and
+// 39.9 -> 33.3 us a launch, at 5.7 and 6.0 TB/s) and by latency on small ones,
+// where 71 and 95 registers leave 7 and 5 waves a SIMD (224x448, 15 shots, four
+// threads a cell: 25.2 and 28.9 us; an objective there 143 -> 92.5 ms).  Fewer
+// registers make it slower (85 for k_exact_b: 114 ms), and so do more, for the
+// next shot's loads (107 ms).
 __device__ __forceinline__ float pml_t(float g, float K, float r, float a, float b, float& P) {
   const float tot = g + P;
   P = b * tot;
