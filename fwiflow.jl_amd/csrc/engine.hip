@@ -1295,22 +1295,29 @@ std::vector<RowRange> split_even(int a, int b, int per) {
 // 8th step
 constexpr int sample_every = 64;
 constexpr int kMaxPartsTable = 31;  // plans of a job
-// Where a time step is one launch instead of two, in waves of a half-step
-// launch (64 depth cells x 1 column x 1 shot each).  Forward: one launch less
-// and no second read of the first half's results, against the rim that is
-// computed twice and a second copy of the state in the caches.  Measured, two
-// launches / one: 168 waves 1.89 / 1.20 ms, 792: 14.6 / 12.4, 2046: 10.6 /
-// 10.1, 10752: 39.2 / 38.0, 23136: 45.5 / 44.9, 36500: 60.1 / 59.8, 53760:
-// 93 / 100, 142400: 59 / 79.
+// Where a time step is one launch instead of two, in columns of whole-step
+// tiles over all shots (the waves that a launch without rims would need).
+// Forward: one launch less and no second read of the first half's results,
+// against the rim that is computed twice and a second copy of the state in the
+// caches.  Measured, two launches / one, 500 steps: 672 columns 2.95 / 2.29 ms,
+// 3168: 4.08 / 3.56, 3429: 4.22 / 3.53, 9144: 7.41 / 6.67, 12573: 8.86 / 7.87, 13720:
+// 7.28 / 7.30, 14256: 9.78 / 9.41, 16002: 10.0 / 9.92, 16800: 8.10 / 8.88, 22272:
+// 11.8 / 12.0, 27328: 11.3 / 12.3; one shot of 6860: 5.12 / 4.90, 11040: 7.62 /
+// 7.12, 17800: 10.7 / 10.2.  (Worse inside the line: 20 shots of 600, 8.55 / 9.07.)
+// Slices of two shots instead of one where one would need more than the 8192
+// waves that the chip holds: 8 shots of 600 columns 4.95 / 4.53 ms, 10 of 792
+// 6.61 / 6.33, 2 of 4200 5.75 / 5.49; below it one is better (6 of 1840 13.6 ms in
+// twos, 14.2 in threes, 15.0 alone at 1000 steps).
 //
 // Backward (adjoint and reversal both recompute their rim, twice the state is
 // copied, and the reversal's workgroups walk all shots, since their sums are
-// taken in order), in waves of the adjoint's whole-step tiles, two launches /
-// one, 400 steps: one shot of 84 waves 4.16 / 3.55 ms, 1023: 4.50 / 4.26, 1272:
-// 5.08 / 4.83, 2080: 6.06 / 5.67, 3300: 11.7 / 12.0 (601 steps); two shots of 84: 4.68 /
-// 3.72, 792: 15.0 / 14.7 (1000 steps), 1023: 5.56 / 5.75; three of 84: 5.33 / 4.30, 1023: 6.86 / 7.19;
-// four of 84: 5.37 / 5.11, 368: 16.5 / 14.8 (1000 steps); six of 84: 6.18 / 6.32.
-constexpr double kWholeFwdWaves = 16384;
+// taken in order), two launches / one, 400 steps: one shot of 84 columns 4.16 /
+// 3.55 ms, 1023: 4.50 / 4.26, 1272: 5.08 / 4.83, 2080: 6.06 / 5.67, 3300: 11.7 /
+// 12.0 (601 steps); two shots of 84: 4.68 / 3.72, 792: 15.0 / 14.7 (1000 steps),
+// 1023: 5.56 / 5.75; three of 84: 5.33 / 4.30, 1023: 6.86 / 7.19; four of 84: 5.37 /
+// 5.11, 368: 16.5 / 14.8 (1000 steps); six of 84: 6.18 / 6.32.
+constexpr double kWholeFwdWaves = 16384, kWholeFwdWaves1 = 20480;  // several shots, one
+constexpr double kChipWaves = 8192;
 constexpr double kWholeBwdWaves = 1600, kWholeBwdWaves1 = 2304;  // several shots, one
 constexpr int kWholeBwdShots = 4;
 
@@ -1864,12 +1871,19 @@ Status Runner::run(int calc_id) {
   // shots of 224x448 96.0 -> 94.0 ms, 20 shots of 224x520 68.8 -> 66.5, reference's
   // adjoint of 20 shots of 127x341 36.7 -> 36.0
   if (c0.tile_auto && withAdj && nb_ == 4) tile_ = 1;
-  whole_f_ = !c0.arena && waves(mf) <= kWholeFwdWaves;
-  double tiles = 0;
-  for (const Member& m : M)
-    tiles += (double)((m.d->g.nzA - 4 + kCoreZ - 1) / kCoreZ) * m.d->g.nx * std::min(mb, m.d->g.ns);
+  auto tiles = [&](int shots) {  // columns of whole-step tiles, each a wave of its core
+    double t = 0;
+    for (const Member& m : M)
+      t += (double)((m.d->g.nzA - 4 + kCoreZ - 1) / kCoreZ) * m.d->g.nx * std::min(shots, m.d->g.ns);
+    return t;
+  };
+  whole_f_ = !c0.arena && tiles(mf) <= (mf == 1 ? kWholeFwdWaves1 : kWholeFwdWaves);
+  if (whole_f_) {
+    sf_ = kStepW / kCoreX * tiles(mf) > kChipWaves ? std::min(2, mf) : 1;
+    nf_ = (mf + sf_ - 1) / sf_;
+  }
   whole_b_ = !c0.arena && withAdj && mb <= kWholeBwdShots &&
-             tiles <= (mb == 1 ? kWholeBwdWaves1 : kWholeBwdWaves);
+             tiles(mb) <= (mb == 1 ? kWholeBwdWaves1 : kWholeBwdWaves);
   for (const Member& m : M) whole_b_ = whole_b_ && !m.d->adjoint && m.d->inj_folded;
   // buffers
   for (const Member& m : M) {

@@ -26,6 +26,7 @@ CASES = {
     "core_plus_one_4_shots": (41, 63, 4, 150),
     "core_plus_one_5_shots": (41, 60, 5, 150),
     "strip_plus_one_9_shots": (105, 63, 9, 61),
+    "whole_steps_in_pairs_25_shots": (41, 61, 25, 60),
     "sliced_forward": (41, 331, 24, 60),
 }
 
