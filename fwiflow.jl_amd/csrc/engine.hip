@@ -1379,7 +1379,6 @@ class Runner {
   void half_b(const GroupParts& gp, int it, int ring, int kinds);
   void exact_a(const GroupParts& gp, int it, int first);
   void exact_b(const GroupParts& gp, int it);
-  template <bool Save>
   void ring_all(const GroupParts& gp, int it, int c0, int c1);
   // whole steps: `odd` launches read the second state buffers
   dim3 whole_grid(const GroupParts& gp, bool backward) const;
@@ -1660,7 +1659,7 @@ Status Runner::forward(const GroupParts& gp, int t0, int t1,
                        const std::function<Status(int, int)>& before) {
   const bool ring = !gp.args.empty() && gp.args[0].ring;
   auto row = [&](int it) { return ring ? ring_at(it) : -1; };
-  if (!whole_f_ && ring && t1 > t0) ring_all<true>(gp, t0, 0, 3);  // the stresses that step t0 reads
+  if (!whole_f_ && ring && t1 > t0) ring_all(gp, t0, 0, 3);  // the stresses that step t0 reads
   for (int it = t0; it < t1; it++) {
     const bool smp = it % sample_every == 0;
     const int odd = whole_f_ ? (t1 - it) & 1 : 0;
@@ -1676,11 +1675,10 @@ Status Runner::forward(const GroupParts& gp, int t0, int t1,
 }
 
 // ring components [c0, c1) of step it saved from the main state buffers
-template <bool Save>
 void Runner::ring_all(const GroupParts& gp, int it, int c0, int c1) {
   int n = 0;
   for (const StepArgs& a : gp.args) n = std::max(n, a.ringlen);
-  hipLaunchKernelGGL((k_ring<Save>), dim3((n + 255) / 256, 1, (unsigned)gp.args.size()), dim3(256), 0,
+  hipLaunchKernelGGL(k_ring, dim3((n + 255) / 256, 1, (unsigned)gp.args.size()), dim3(256), 0,
                      st, cache.steps + gp.steps, ring_at(it), c0, c1);
 }
 

@@ -731,11 +731,10 @@ __device__ __forceinline__ int extra_item(int first, int chunk) {
   return ((row * (int)gridDim.x + (int)blockIdx.x) * (int)blockDim.y + (int)threadIdx.y) * kBZ + (int)threadIdx.x;
 }
 
-// every component, for the first step of a run or segment and before its reversal
-template <bool Save>
+// ring components [c0, c1) of a run's or segment's first step
 __global__ __launch_bounds__(256) void k_ring(const StepArgs* __restrict__ args, int row, int c0, int c1) {
   CStep& A = ((CStep*)args)[blockIdx.z];
-  ring_move<Save>(A, A.wo, (int)(blockIdx.x * 256 + threadIdx.x), 0, A.ns, row, c0, c1);
+  ring_move<true>(A, A.wo, (int)(blockIdx.x * 256 + threadIdx.x), 0, A.ns, row, c0, c1);
 }
 
 // el_stress.cu:50-88 + add_source (utilities.cu:521-555).  Extra rows save the
