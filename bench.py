@@ -426,7 +426,7 @@ def main():
             "unit": "GB/s",
         },
         "kernel_avg_ms": {k: round(v[0], 4) for k, v in kt.items()},
-        "launch": dict(zip(("tile_x", "shots_fwd", "shots_bwd"), P.launch()),
+        "launch": dict(zip(("tile_x", "shots_fwd", "shots_bwd"), (P.tile_width(), *P.launch()[1:])),
                        autotuned=tuned is not None),
         "launch_groups": {"forward": groups_f, "backward": groups_b},
         "device_bytes": P.device_bytes(),

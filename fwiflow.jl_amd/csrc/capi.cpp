@@ -237,6 +237,11 @@ int fwiflow_plan_launch_groups(fwiflow_plan* plan, int* forward, int* backward) 
   if (backward) *backward = plan->impl.launch_groups(1);
   return report(Status::Ok());
 }
+int fwiflow_plan_tile_width(fwiflow_plan* plan, int* tile_x) {
+  if (!plan || !tile_x) return report(Status::Err(FWIFLOW_ERR_ARG, "null argument"));
+  *tile_x = plan->impl.tile_width();
+  return report(Status::Ok());
+}
 int fwiflow_plan_set_memory_budget(fwiflow_plan* plan, double bytes) {
   PLAN_CALL(plan->impl.set_memory_budget(bytes));
 }

@@ -555,7 +555,8 @@ struct DeviceState {
   std::vector<int> roff;  // first receiver of each shot (+ total)
   // engine settings (environment variables read at plan creation)
   int tile_x = 4;          // columns of a half step's tile (blockDim.y) where chosen
-  bool tile_auto = true;   // not chosen
+  bool tile_auto = true;   // not chosen (tile_x is 4 then: such plans and those
+                           // with 4 chosen may share a job)
   int shot_group = -1;     // shots per forward launch (0: all, -1: automatic)
   int shot_group_bwd = -1; // shots per backward launch (0: all, -1: automatic)
   bool fold_inject = true; // residual injection inside the adjoint stress update
@@ -620,6 +621,7 @@ struct DeviceState {
   std::vector<float> keep_obs, keep_syn;
   // last gradient run's memory plan and shot groups
   int last_k = 0, last_rows_sg = 0, last_groups_f = 0, last_groups_b = 0;
+  int last_tile = 0;  // columns of the last run's half-step tiles (0: whole steps only)
   long long last_ring_bytes = 0, last_snap_bytes = 0;
   std::unique_ptr<JobCache> cache;  // maps of this plan's own runs
   std::vector<void*> allocs;
@@ -1133,11 +1135,12 @@ Status Plan::set_memory_budget(double bytes) {
 
 Status Plan::set_launch(int tile_x, int shots_fwd, int shots_bwd) {
   if (!d_) return Status::Err(FWIFLOW_ERR_ARG, "plan not created");
-  if (tile_x < 1 || tile_x > 4) return Status::Err(FWIFLOW_ERR_ARG, "tile width must be 1..4");
+  if (tile_x != -1 && (tile_x < 1 || tile_x > 4))
+    return Status::Err(FWIFLOW_ERR_ARG, "tile width must be 1..4, or -1 (automatic)");
   if (shots_fwd < -1 || shots_bwd < -1)
     return Status::Err(FWIFLOW_ERR_ARG, "shots per launch must be >= -1");
-  d_->tile_auto = false;
-  d_->tile_x = tile_x;
+  d_->tile_auto = tile_x == -1;
+  d_->tile_x = tile_x == -1 ? 4 : tile_x;
   d_->shot_group = shots_fwd;
   d_->shot_group_bwd = shots_bwd;
   if (d_->cache) d_->cache->clear_graphs();  // captured loops bake the old shape in
@@ -1146,7 +1149,7 @@ Status Plan::set_launch(int tile_x, int shots_fwd, int shots_bwd) {
 
 Status Plan::launch(int* tile_x, int* shots_fwd, int* shots_bwd) const {
   if (!d_) return Status::Err(FWIFLOW_ERR_ARG, "plan not created");
-  if (tile_x) *tile_x = d_->tile_x;
+  if (tile_x) *tile_x = d_->tile_auto ? -1 : d_->tile_x;
   if (shots_fwd) *shots_fwd = d_->shot_group;
   if (shots_bwd) *shots_bwd = d_->shot_group_bwd;
   return Status::Ok();
@@ -1187,6 +1190,7 @@ int Plan::shots_per_launch_bwd() const {
   if (!d_) return 0;
   return d_->last_groups_b > 0 ? (d_->g.ns + d_->last_groups_b - 1) / d_->last_groups_b : 0;
 }
+int Plan::tile_width() const { return d_ ? d_->last_tile : 0; }
 int Plan::launch_groups(int backward) const {
   if (!d_) return 0;
   return backward ? d_->last_groups_b : d_->last_groups_f;
@@ -1961,6 +1965,7 @@ Status Runner::run(int calc_id) {
     }
     if (d.illum_on && !d.illum) TRY(d.alloc(&d.illum, N));
     d.src_updated = if_res && d.cond && m.plan->para.if_src_update;
+    d.last_tile = whole_f_ && (whole_b_ || !withAdj) ? 0 : tile_;
     d.last_groups_f = 0;
     d.last_groups_b = 0;
     for (size_t j = 0; j < sweeps.size(); j++) {

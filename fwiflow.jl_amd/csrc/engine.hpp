@@ -55,6 +55,7 @@ class Plan {
   int shots_per_launch() const;      // forward sweep (largest group of the last run)
   int shots_per_launch_bwd() const;  // backward sweep
   int launch_groups(int backward) const;  // shot groups of the last run
+  int tile_width() const;                 // half-step tiles of the last run
   Status set_illumination(bool on);
   Status illumination(double* out);
 

@@ -235,17 +235,24 @@ class Plan:
         check(self._L.fwiflow_plan_set_memory_budget(self._h, float(nbytes)))
 
     def set_launch(self, tile_x, shots_fwd=-1, shots_bwd=-1):
-        """Launch shape: tile width 1-4, shots per forward / backward launch
-        (0: all, -1: automatic)."""
+        """Launch shape: tile width 1-4 (-1: automatic; steps of one launch have
+        no such tile), shots per forward / backward launch (0: all, -1: automatic)."""
         check(self._L.fwiflow_plan_set_launch(self._h, int(tile_x), int(shots_fwd),
                                               int(shots_bwd)))
 
     def launch(self):
-        """(tile width, shots per forward launch, shots per backward launch)."""
+        """(tile width, shots per forward launch, shots per backward launch) as
+        set; ``set_launch(*launch())`` changes nothing."""
         t, f, b = _lib.C.c_int(0), _lib.C.c_int(0), _lib.C.c_int(0)
         check(self._L.fwiflow_plan_launch(self._h, _lib.C.byref(t), _lib.C.byref(f),
                                           _lib.C.byref(b)))
         return int(t.value), int(f.value), int(b.value)
+
+    def tile_width(self):
+        """Tile width of the last run's two-launch steps (0: it had none)."""
+        t = _lib.C.c_int(0)
+        check(self._L.fwiflow_plan_tile_width(self._h, _lib.C.byref(t)))
+        return int(t.value)
 
     def memory_plan(self):
         """(checkpoint interval, shots per sweep, ring bytes, checkpoint bytes) of

@@ -193,13 +193,19 @@ int fwiflow_plan_set_adjoint(fwiflow_plan* plan, int mode);
  * checkpoints (default 32e9).  It sets the shots per sweep. */
 int fwiflow_plan_set_memory_budget(fwiflow_plan* plan, double bytes);
 /* Launch shape of the plan's runs: tile width in columns (1-4; a workgroup
- * is 64 cells x tile_x), shots per forward and per backward launch (0: all
- * of the plan's shots, -1: automatic, the Infinity-Cache rule).  Replaces
+ * is 64 cells x tile_x; -1: automatic), shots per forward and per backward
+ * launch (0: all of the plan's shots, -1: automatic, the Infinity-Cache rule).
+ * The width is that of steps taken in two launches; steps of one launch, which
+ * small grids take, have tiles of their own.  Replaces
  * the FWIFLOW_TILE_X / FWIFLOW_SHOT_GROUP(_BWD) defaults; what the autotuner
  * (fwiflow/tune.py) chooses and caches per grid and shot count.  No
  * counterpart in the reference (its launch shape is fixed). */
 int fwiflow_plan_set_launch(fwiflow_plan* plan, int tile_x, int shots_fwd, int shots_bwd);
+/* The shape as set (-1 where automatic). */
 int fwiflow_plan_launch(fwiflow_plan* plan, int* tile_x, int* shots_fwd, int* shots_bwd);
+/* The tile width of the last run's two-launch steps, also where it was chosen
+ * automatically (0: it had none, or there was no run yet). */
+int fwiflow_plan_tile_width(fwiflow_plan* plan, int* tile_x);
 /* The memory plan of the last gradient run: checkpoint interval (0: ring of
  * every step), shots per sweep, device bytes of the ring and of the
  * checkpoints.  Any pointer may be NULL. */
