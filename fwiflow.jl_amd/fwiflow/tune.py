@@ -2,9 +2,10 @@
 
 The engine's automatic shape (workgroups two columns wide, or one; shots per
 launch from the Infinity-Cache rule, round(224 MB / bytes per shot)) is a model; this module
-measures the neighbourhood of it on the caller's own grid and shot count and
+measures it and its neighbourhood on the caller's own grid and shot count and
 keeps the fastest, per (grid, C-PML, shot count), in a JSON cache
-(``FWIFLOW_TUNE_CACHE`` or ``~/.cache/fwiflow/launch.json``).
+(``FWIFLOW_TUNE_CACHE`` or ``~/.cache/fwiflow/launch.json``).  A shape measured
+on other kernels (``ENGINE``) is not applied.
 
 A candidate is timed on the caller's model over a shortened record
 (``steps`` time steps; every step of a run costs the same, so the ranking
@@ -26,6 +27,8 @@ import numpy as np
 from .ops import Plan
 
 ARCH = "gfx950"
+# raised when kernels change which shape is the fastest
+ENGINE = 2
 
 
 def cache_path(path=None):
@@ -59,8 +62,12 @@ def store(key, entry, path=None):
 
 
 def lookup(para_fname, nshots, path=None):
-    """The cached launch shape for this grid and shot count, or None."""
-    return load_cache(path).get(cache_key(para_fname, nshots))
+    """The cached launch shape for this grid and shot count, or None (also where
+    it was measured on another engine)."""
+    e = load_cache(path).get(cache_key(para_fname, nshots))
+    if e is not None and "candidates" in e and e.get("engine") != ENGINE:
+        return None
+    return e
 
 
 def apply_tuned(plan, para_fname, nshots, path=None):
@@ -86,12 +93,13 @@ def _short_para(para_fname, steps, ws):
     return out, n
 
 
-def autotune(para_fname, shot_ids, lam, mu, den, stf, steps=200, tiles=(4, 2), repeats=2,
+def autotune(para_fname, shot_ids, lam, mu, den, stf, steps=200, tiles=(4, 2, 1), repeats=2,
              gpu_id=0, path=None, log=None):
-    """Time launch shapes around the automatic one on ``steps`` time steps of
-    the caller's problem; cache and return the fastest as a dict
+    """Time the automatic launch shape and those around it on ``steps`` time
+    steps of the caller's problem; cache and return the fastest as a dict
     (tile_x, shots_fwd, shots_bwd, seconds per gradient run of ``steps``,
-    and every candidate's time)."""
+    and every candidate's time).  Where every step is one launch, which has
+    no such tile, only the shots are varied."""
     say = log or (lambda *a: None)
     ids = list(np.atleast_1d(shot_ids))
     stf = np.atleast_2d(np.asarray(stf, dtype=np.float64))
@@ -102,9 +110,12 @@ def autotune(para_fname, shot_ids, lam, mu, den, stf, steps=200, tiles=(4, 2), r
             P.set_stf(np.ascontiguousarray(stf[:, :n]))
             P.run(2)
             P.set_obs(P.data())
-            P.set_launch(4, -1, -1)
+            P.set_launch(-1, -1, -1)
             P.run(1)
             f0, b0 = P.shots_per_launch()
+            t0 = P.tile_width()
+            tiles = sorted({*tiles, t0}, reverse=True) if t0 else (2,)
+            t0 = t0 or 2
             ns = len(ids)
             near = lambda k: sorted({max(1, min(ns, k + d)) for d in (-1, 0, 1)})  # noqa: E731
             cands = [(t, f, b) for t in tiles for f in near(f0) for b in near(b0)]
@@ -114,14 +125,14 @@ def autotune(para_fname, shot_ids, lam, mu, den, stf, steps=200, tiles=(4, 2), r
                 P.run(1)
                 best = np.inf
                 for _ in range(repeats):
-                    t0 = time.perf_counter()
+                    start = time.perf_counter()
                     P.run(1)
-                    best = min(best, time.perf_counter() - t0)
+                    best = min(best, time.perf_counter() - start)
                 times[(t, f, b)] = best
                 say(f"tune tile {t} shots {f}/{b}: {best * 1e3:.1f} ms")
     (t, f, b), sec = min(times.items(), key=lambda kv: kv[1])
     entry = {"tile_x": t, "shots_fwd": f, "shots_bwd": b, "seconds": sec, "steps": n,
-             "automatic": [4, f0, b0], "automatic_seconds": times.get((4, f0, b0)),
+             "engine": ENGINE, "automatic": [t0, f0, b0], "automatic_seconds": times[(t0, f0, b0)],
              "candidates": {f"{k[0]}/{k[1]}/{k[2]}": v for k, v in times.items()}}
     store(cache_key(para_fname, len(ids)), entry, path)
     return entry
