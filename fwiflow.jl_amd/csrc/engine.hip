@@ -530,17 +530,21 @@ struct JobCache {
     graphs.clear();
   }
   template <typename T>
+  Status reserve(size_t n, T*& dev_ptr, size_t& cap) {
+    if (n <= cap) return Status::Ok();
+    if (dev_ptr && !arena) HIP_TRY(hipFree(dev_ptr));
+    dev_ptr = nullptr;
+    cap = 0;
+    if (arena)
+      TRY(arena->take((void**)&dev_ptr, n * sizeof(T)));
+    else
+      HIP_TRY(hipMalloc((void**)&dev_ptr, n * sizeof(T)));
+    cap = n;
+    return Status::Ok();
+  }
+  template <typename T>
   Status upload(const std::vector<T>& a, T*& dev_ptr, size_t& cap) {
-    if (a.size() > cap) {
-      if (dev_ptr && !arena) HIP_TRY(hipFree(dev_ptr));
-      dev_ptr = nullptr;
-      cap = 0;
-      if (arena)
-        TRY(arena->take((void**)&dev_ptr, a.size() * sizeof(T)));
-      else
-        HIP_TRY(hipMalloc((void**)&dev_ptr, a.size() * sizeof(T)));
-      cap = a.size();
-    }
+    TRY(reserve(a.size(), dev_ptr, cap));
     if (!a.empty()) HIP_TRY(hipMemcpy(dev_ptr, a.data(), a.size() * sizeof(T), hipMemcpyHostToDevice));
     return Status::Ok();
   }
@@ -564,6 +568,7 @@ struct DeviceState {
                            // (measured no faster at 608x1780; timed runs stay eager)
   int ckpt_every = 0;      // 0: boundary ring every step; k > 0: checkpoints every k steps
   int adjoint = 0;         // 0: the reference's adjoint; 1: the exact adjoint
+  double limit = 0;        // device bytes that the plan may hold (0: what the GPU has)
   double ring_budget = 32e9;  // device bytes a gradient run may hold for ring + checkpoints
   // model + tables
   float *lam = nullptr, *mu = nullptr, *den = nullptr, *amu = nullptr, *ba = nullptr,
@@ -662,6 +667,9 @@ struct DeviceState {
       *p = (T*)q;
       return Status::Ok();
     }
+    if (limit > 0 && (double)bytes + (double)nb > limit)
+      return Status::Err(FWIFLOW_ERR_MEMORY, std::to_string(nb) + " more bytes are over FWIFLOW_PLAN_BYTES, " +
+                                                 std::to_string(bytes) + " in use");
     hipError_t e = hipMalloc(&q, nb ? nb : 4);
     if (e != hipSuccess)
       return Status::Err(e == hipErrorOutOfMemory ? FWIFLOW_ERR_MEMORY : FWIFLOW_ERR_HIP,
@@ -816,6 +824,7 @@ Status Plan::create(const std::string& para_fname, int gpu, int group_size, cons
   d.fold_inject = env_int("FWIFLOW_FOLD_INJECT", 1) != 0;
   d.graphs = env_int("FWIFLOW_GRAPHS", 0) != 0;
   d.adjoint = env_int("FWIFLOW_EXACT_ADJOINT", 0) != 0 ? 1 : 0;
+  if (const char* v = std::getenv("FWIFLOW_PLAN_BYTES")) d.limit = std::atof(v);
   if (in_scratch) {
     // every buffer from the device's scratch array, no graphs (instantiating
     // one allocates), the device's shared stream
@@ -1390,6 +1399,7 @@ class Runner {
   void step_bwd(const GroupParts& gp, int fodd, int aodd, int it);
   void record_last(const GroupParts& gp, int it);
   void illum_last(const GroupParts& gp);
+  Status second_states(DeviceState& d, int mf, int mb);
   Status clear_second(const GroupParts& gp);
   // forward steps [t0, t1) of a group, `before(it, odd)` before each; they end
   // in the main state buffers
@@ -1702,6 +1712,28 @@ void Runner::illum_last(const GroupParts& gp) {
                        cache.steps + gp.steps);
 }
 
+// Room for the second states of the launches that take whole steps; they start
+// out zero and stay zero outside the update region.
+Status Runner::second_states(DeviceState& d, int mf, int mb) {
+  auto room = [&](float*& p, int& have, int need, int comps) -> Status {
+    need = std::min(need, d.g.ns);
+    if (have >= need) return Status::Ok();
+    const size_t n = (size_t)comps * d.g.N;
+    d.release(p, have * n);
+    have = 0;
+    TRY(d.alloc(&p, need * n));
+    have = need;
+    HIP_TRY(hipMemsetAsync(p, 0, need * n * sizeof(float), st));
+    return Status::Ok();
+  };
+  const int f = whole_f_ ? mf : 0, b = whole_b_ ? mb : 0;
+  TRY(room(d.fwd2, d.shots2, std::max(f, b), kWaveComps));
+  TRY(room(d.mem2, d.mshots2, std::max(f, ckpt ? 0 : b), kMemComps));
+  TRY(room(d.adj2, d.ashots2, b, kWaveComps));
+  TRY(room(d.madj2, d.xshots2, ckpt ? b : 0, kMemComps));
+  return Status::Ok();
+}
+
 Status Runner::clear_second(const GroupParts& gp) {
   for (size_t q = 0; q < gp.member.size(); q++) {
     DeviceState& d = *M[gp.member[q]].d;
@@ -1928,33 +1960,6 @@ Status Runner::run(int calc_id) {
       d.last_ring_bytes = (long long)(rf * sizeof(float));
       d.last_snap_bytes = (long long)(sf * sizeof(float));
     }
-    // the second states start out zero and stay zero outside the update region
-    auto second = [&](float*& p, int& have, int need, int comps) -> Status {
-      if (have >= need) return Status::Ok();
-      d.release(p, (size_t)have * comps * N);
-      have = 0;
-      TRY(d.alloc(&p, (size_t)need * comps * N));
-      have = need;
-      HIP_TRY(hipMemsetAsync(p, 0, (size_t)need * comps * N * sizeof(float), st));
-      return Status::Ok();
-    };
-    auto seconds = [&]() -> Status {
-      if (whole_f_ || whole_b_) {
-        const int n2 = std::min(d.g.ns, whole_b_ ? std::max(mf, mb) : mf);
-        TRY(second(d.fwd2, d.shots2, n2, kWaveComps));
-        TRY(second(d.mem2, d.mshots2, n2, kMemComps));
-      }
-      if (whole_b_) {
-        const int n2 = std::min(d.g.ns, mb);
-        TRY(second(d.adj2, d.ashots2, n2, kWaveComps));
-        if (ckpt) TRY(second(d.madj2, d.xshots2, n2, kMemComps));
-      }
-      return Status::Ok();
-    };
-    if (!seconds().ok()) {  // no room for them: two launches a step
-      (void)hipGetLastError();
-      whole_f_ = whole_b_ = false;
-    }
     if (withAdj) TRY(ensure_injection(d));
     const int npart = (int)sweeps.size() * kPartials;
     if (d.npartial < npart) {
@@ -1965,7 +1970,6 @@ Status Runner::run(int calc_id) {
     }
     if (d.illum_on && !d.illum) TRY(d.alloc(&d.illum, N));
     d.src_updated = if_res && d.cond && m.plan->para.if_src_update;
-    d.last_tile = whole_f_ && (whole_b_ || !withAdj) ? 0 : tile_;
     d.last_groups_f = 0;
     d.last_groups_b = 0;
     for (size_t j = 0; j < sweeps.size(); j++) {
@@ -1973,6 +1977,36 @@ Status Runner::run(int calc_id) {
       for (RowRange rr : BR[j]) d.last_groups_b += shots_in(m, rr.r1) > shots_in(m, rr.r0);
     }
   }
+  {
+    size_t nf = 0, nb = 0;  // argument table entries
+    for (size_t j = 0; j < sweeps.size(); j++) {
+      nf += FR[j].size() + (ckpt ? BR[j].size() : 0);
+      nb += BR[j].size();
+    }
+    TRY(cache.reserve(nf * M.size() * (whole_f_ ? 3 : 1), cache.steps, cache.steps_cap));
+    TRY(cache.reserve(nb * M.size() * (whole_b_ ? 5 : 1), cache.backs, cache.backs_cap));
+  }
+  // The second states come last: a run without them takes two launches a step,
+  // all members alike.
+  Status second = Status::Ok();
+  for (const Member& m : M)
+    if (second.ok()) second = second_states(*m.d, mf, mb);
+  if (!second.ok()) {
+    if (second.code != FWIFLOW_ERR_MEMORY) return second;
+    (void)hipGetLastError();
+    for (const Member& m : M) {
+      DeviceState& d = *m.d;
+      const size_t N = (size_t)d.g.N;
+      d.release(d.fwd2, (size_t)d.shots2 * kWaveComps * N);
+      d.release(d.mem2, (size_t)d.mshots2 * kMemComps * N);
+      d.release(d.adj2, (size_t)d.ashots2 * kWaveComps * N);
+      d.release(d.madj2, (size_t)d.xshots2 * kMemComps * N);
+      d.shots2 = d.mshots2 = d.ashots2 = d.xshots2 = 0;
+    }
+    whole_f_ = whole_b_ = false;
+    slice(mf, sf_, nf_);
+  }
+  for (const Member& m : M) m.d->last_tile = whole_f_ && (whole_b_ || !withAdj) ? 0 : tile_;
   // parts of every group (pointing at the buffers above)
   std::vector<std::vector<GroupParts>> FG(sweeps.size()), RG(sweeps.size()), BG(sweeps.size());
   for (size_t j = 0; j < sweeps.size(); j++) {
