@@ -1383,6 +1383,10 @@ class Runner {
     else
       hipLaunchKernelGGL(k, grid, block, 0, st, a...);
   }
+  // for half_chunk
+  static unsigned inverse(int places) {
+    return places > 1 ? (unsigned)(((1ull << 32) + places - 1) / places) : 0u;
+  }
   // grid of a half-step launch: `kinds` strips per tile row, and rows for the
   // extra items (ring, receivers, illumination) of the parts
   dim3 half_grid(const GroupParts& gp, int kinds, bool ring, bool rec, bool illum, int places) const;
@@ -1613,31 +1617,35 @@ dim3 Runner::half_grid(const GroupParts& gp, int kinds, bool ring, bool rec, boo
 void Runner::half_stress(const GroupParts& gp, int it, int ring) {
   const int pf = nf_ * (int)gp.args.size();
   go(k_half_stress<2>, half_grid(gp, 1, ring >= 0, false, true, pf), dim3(kBZ, tile_),
-     cache.steps + gp.steps, it, ring, nf_, sf_, pf);
+     cache.steps + gp.steps, it, ring, nf_, sf_, pf, inverse(pf));
 }
 void Runner::half_vel(const GroupParts& gp, int it, int ring) {
   const int pf = nf_ * (int)gp.args.size();
   go(k_half_vel<2>, half_grid(gp, 1, ring >= 0, true, false, pf), dim3(kBZ, tile_),
-     cache.steps + gp.steps, it, ring, nf_, sf_, pf);
+     cache.steps + gp.steps, it, ring, nf_, sf_, pf, inverse(pf));
 }
 void Runner::half_a(const GroupParts& gp, int it, int ring, int kinds) {
-  go(nb_ > 1 ? k_half_bwd_a<true> : k_half_bwd_a<false>, half_grid(gp, 2, ring >= 0, false, false, (int)gp.args.size()),
-     dim3(kBZ, tile_, nb_), cache.backs + gp.backs, it, ring, kinds, (int)gp.args.size());
+  const int parts = (int)gp.args.size();
+  go(nb_ > 1 ? k_half_bwd_a<true> : k_half_bwd_a<false>, half_grid(gp, 2, ring >= 0, false, false, parts),
+     dim3(kBZ, tile_, nb_), cache.backs + gp.backs, it, ring, kinds, parts, inverse(parts));
 }
 void Runner::half_b(const GroupParts& gp, int it, int ring, int kinds) {
-  go(nb_ > 1 ? k_half_bwd_b<true> : k_half_bwd_b<false>, half_grid(gp, 2, ring >= 0, false, false, (int)gp.args.size()),
-     dim3(kBZ, tile_, nb_), cache.backs + gp.backs, it, ring, kinds, (int)gp.args.size());
+  const int parts = (int)gp.args.size();
+  go(nb_ > 1 ? k_half_bwd_b<true> : k_half_bwd_b<false>, half_grid(gp, 2, ring >= 0, false, false, parts),
+     dim3(kBZ, tile_, nb_), cache.backs + gp.backs, it, ring, kinds, parts, inverse(parts));
 }
 // exact adjoint (with the reversal of the step)
 void Runner::exact_a(const GroupParts& gp, int it, int first) {
-  go(nb_ > 1 ? k_exact_a<true> : k_exact_a<false>, half_grid(gp, 1, true, false, false, (int)gp.args.size()),
+  const int parts = (int)gp.args.size();
+  go(nb_ > 1 ? k_exact_a<true> : k_exact_a<false>, half_grid(gp, 1, true, false, false, parts),
      dim3(kBZ, tile_, nb_), cache.backs + gp.backs, xt_, it, ring_at(it), first,
-     (int)gp.args.size());
+     parts, inverse(parts));
 }
 void Runner::exact_b(const GroupParts& gp, int it) {
-  go(nb_ > 1 ? k_exact_b<true> : k_exact_b<false>, half_grid(gp, 1, true, false, false, (int)gp.args.size()),
+  const int parts = (int)gp.args.size();
+  go(nb_ > 1 ? k_exact_b<true> : k_exact_b<false>, half_grid(gp, 1, true, false, false, parts),
      dim3(kBZ, tile_, nb_), cache.backs + gp.backs, xt_, srcwin_, it, ring_at(it),
-     (int)gp.args.size());
+     parts, inverse(parts));
 }
 
 dim3 Runner::whole_grid(const GroupParts& gp, bool backward) const {

@@ -709,12 +709,14 @@ __global__ __launch_bounds__(64 * kStepW) void k_step_bwd(const BackArgs* __rest
 struct HalfTile {
   int z, x;
 };
-// chunk of the workgroup; k: its place
-__device__ __forceinline__ int half_chunk(int places, int& k) {
-  int chunk = 0;
-  k = (int)blockIdx.z;
-  while (k >= places) k -= places, ++chunk;
-  return chunk;
+// chunk of the workgroup; k: its place.  inv = ceil(2^32 / places) (0 for one
+// place): the high half of b times it is b / places for 16-bit numbers.  Counted
+// off in a loop, a grid of 84 x 60024 (469 chunks) took 15.5 ms instead of 5.0
+// for 60 steps.
+__device__ __forceinline__ int half_chunk(int places, unsigned inv, int& k) {
+  const unsigned b = blockIdx.z, chunk = inv ? __umulhi(b, inv) : b;
+  k = (int)(b - chunk * (unsigned)places);
+  return (int)chunk;
 }
 // false: the workgroup is past the tiles
 __device__ __forceinline__ bool half_tile(CStep& A, int strip, int chunk, HalfTile& t) {
@@ -742,9 +744,10 @@ __global__ __launch_bounds__(256) void k_ring(const StepArgs* __restrict__ args,
 // step before.
 template <int U>
 __global__ __launch_bounds__(256) void k_half_stress(const StepArgs* __restrict__ args, int it,
-                                                     int ring, int slices, int per_slice, int places) {
+                                                     int ring, int slices, int per_slice, int places,
+                                                     unsigned inv) {
   int k;
-  const int chunk = half_chunk(places, k);
+  const int chunk = half_chunk(places, inv, k);
   const Place pl = place_of(k, slices, per_slice);
   CStep& A = ((CStep*)args)[pl.part];
   const int hi = min(pl.hi, A.ns), strip = (int)blockIdx.y;
@@ -829,9 +832,9 @@ __global__ __launch_bounds__(256) void k_half_stress(const StepArgs* __restrict_
 // of the ring (row `ring`, that of step it + 1; -1: none).
 template <int U>
 __global__ __launch_bounds__(256) void k_half_vel(const StepArgs* __restrict__ args, int it, int ring,
-                                                  int slices, int per_slice, int places) {
+                                                  int slices, int per_slice, int places, unsigned inv) {
   int k;
-  const int chunk = half_chunk(places, k);
+  const int chunk = half_chunk(places, inv, k);
   const Place pl = place_of(k, slices, per_slice);
   CStep& A = ((CStep*)args)[pl.part];
   const int hi = min(pl.hi, A.ns), strip = (int)blockIdx.y;
@@ -1199,10 +1202,10 @@ __device__ __forceinline__ void half_rev_stress(CBack& B, const HalfTile& t, int
 // kinds: 1 the adjoint half, 2 the reversal, 3 both.
 template <bool Sliced>
 __global__ __launch_bounds__(Sliced ? 1024 : 256) void k_half_bwd_a(
-    const BackArgs* __restrict__ args, int it, int ring, int kinds, int places) {
+    const BackArgs* __restrict__ args, int it, int ring, int kinds, int places, unsigned inv) {
   __shared__ float lds[Sliced ? kSumShots * 3 * kSumCells : 1];
   int part;
-  const int chunk = half_chunk(places, part);
+  const int chunk = half_chunk(places, inv, part);
   CBack& B = ((CBack*)args)[part];
   const auto& A = B.s;
   const int row = (int)blockIdx.y;
@@ -1223,10 +1226,10 @@ __global__ __launch_bounds__(Sliced ? 1024 : 256) void k_half_bwd_a(
 
 template <bool Sliced>
 __global__ __launch_bounds__(Sliced ? 1024 : 256) void k_half_bwd_b(
-    const BackArgs* __restrict__ args, int it, int ring, int kinds, int places) {
+    const BackArgs* __restrict__ args, int it, int ring, int kinds, int places, unsigned inv) {
   __shared__ float lds[Sliced ? kSumShots * 2 * kSumCells : 1];
   int part;
-  const int chunk = half_chunk(places, part);
+  const int chunk = half_chunk(places, inv, part);
   CBack& B = ((CBack*)args)[part];
   const auto& A = B.s;
   const int row = (int)blockIdx.y;
@@ -1307,10 +1310,11 @@ __device__ __forceinline__ float ldf(Rsrc X, int sx, int Nb, int own, int base, 
 
 template <bool Sliced>
 __global__ __launch_bounds__(Sliced ? 1024 : 256) void k_exact_a(const BackArgs* __restrict__ args,
-                                                 float* __restrict__ xt, int it, int ring, int first, int places) {
+                                                 float* __restrict__ xt, int it, int ring, int first,
+                                                 int places, unsigned inv) {
   __shared__ float lds[Sliced ? kSumShots * 2 * kSumCells : 1];
   int part;
-  const int chunk = half_chunk(places, part);
+  const int chunk = half_chunk(places, inv, part);
   CBack& B = ((CBack*)args)[part];
   const auto& A = B.s;
   const int strip = (int)blockIdx.y;
@@ -1410,10 +1414,10 @@ template <bool Sliced>
 __global__ __launch_bounds__(Sliced ? 1024 : 256) void k_exact_b(const BackArgs* __restrict__ args,
                                                  float* __restrict__ xt,
                                                  const float* __restrict__ srcwin, int it, int ring,
-                                                 int places) {
+                                                 int places, unsigned inv) {
   __shared__ float lds[Sliced ? kSumShots * 3 * kSumCells : 1];
   int part;
-  const int chunk = half_chunk(places, part);
+  const int chunk = half_chunk(places, inv, part);
   CBack& B = ((CBack*)args)[part];
   const auto& A = B.s;
   const int strip = (int)blockIdx.y;
