@@ -2313,23 +2313,42 @@ Status Plan::misfit(double* out) {
   return Status::Ok();
 }
 
+// Arrays of the grid, one after another at `in`, to the caller's doubles (null:
+// not asked for): z fastest -> row-major [NZ][NX] (libCUFD.cu:480-486).
+// Small grids come over as they are in one copy and are turned here: a kernel
+// and a copy an array take longer.  Gradients, us, turned on the device / here:
+// 8064 cells 66 / 39, 11904 71 / 42, 15872 75 / 54, 28672 91 / 101; illumination
+// 27 / 13, 28 / 15, 30 / 19, 35 / 39.
+constexpr size_t kHostTurn = 20480;  // cells
+static Status fetch_turned(DeviceState& d, const float* in, std::vector<double*> outs) {
+  const size_t nz = (size_t)d.g.nz, nx = (size_t)d.g.nx, N = (size_t)d.g.N, n = outs.size();
+  if (N <= kHostTurn) {
+    std::vector<float> h(n * N);
+    HIP_TRY(hipMemcpyAsync(h.data(), in, h.size() * sizeof(float), hipMemcpyDeviceToHost, d.stream));
+    HIP_TRY(hipStreamSynchronize(d.stream));
+    for (size_t k = 0; k < n; k++)
+      for (size_t z = 0; outs[k] && z < nz; z++)
+        for (size_t x = 0; x < nx; x++) outs[k][z * nx + x] = h[k * N + x * nz + z];
+    return Status::Ok();
+  }
+  double* const out = (double*)d.mem;  // every run clears it
+  Turn t{};
+  for (size_t k = 0; k < n; k++) t.in[k] = in + k * N, t.out[k] = out + k * N;
+  hipLaunchKernelGGL((k_turn<float, double>), dim3((d.g.nz + 31) / 32, (d.g.nx + 31) / 32, (unsigned)n),
+                     dim3(32, 8), 0, d.stream, t, d.g.nx, d.g.nz, 0);
+  HIP_TRY(hipGetLastError());
+  for (size_t k = 0; k < n; k++)
+    if (outs[k])
+      HIP_TRY(hipMemcpyAsync(outs[k], out + k * N, N * sizeof(double), hipMemcpyDeviceToHost, d.stream));
+  HIP_TRY(hipStreamSynchronize(d.stream));
+  return Status::Ok();
+}
+
 Status Plan::gradients(double* gL, double* gM, double* gD, double* gS) {
   if (!d_ || last_calc != 1) return Status::Err(FWIFLOW_ERR_ARG, "no calc_id 1 result");
   DeviceState& d = *d_;
   HIP_TRY(hipSetDevice(d.dev));
-  const int nz = d.g.nz, nx = d.g.nx;
-  const size_t N = (size_t)d.g.N;
-  // z-fastest -> row-major [NZ][NX] (libCUFD.cu:480-486), in doubles
-  double* const out = (double*)d.mem;
-  const Turn t{{d.grad, d.grad + N, d.grad + 2 * N}, {out, out + N, out + 2 * N}};
-  hipLaunchKernelGGL((k_turn<float, double>), dim3((nz + 31) / 32, (nx + 31) / 32, 3), dim3(32, 8), 0,
-                     d.stream, t, nx, nz, 0);
-  HIP_TRY(hipGetLastError());
-  double* outs[3] = {gL, gM, gD};
-  for (int k = 0; k < 3; k++)
-    if (outs[k])
-      HIP_TRY(hipMemcpyAsync(outs[k], out + k * N, N * sizeof(double), hipMemcpyDeviceToHost, d.stream));
-  HIP_TRY(hipStreamSynchronize(d.stream));
+  TRY(fetch_turned(d, d.grad, {gL, gM, gD}));
   if (gS) {
     std::vector<float> s((size_t)d.g.ns * d.g.nSteps);
     HIP_TRY(hipMemcpy(s.data(), d.stf_grad, s.size() * sizeof(float), hipMemcpyDeviceToHost));
@@ -2350,14 +2369,7 @@ Status Plan::illumination(double* out) {
   if (!out) return Status::Err(FWIFLOW_ERR_ARG, "null output pointer");
   DeviceState& d = *d_;
   HIP_TRY(hipSetDevice(d.dev));
-  const int nz = d.g.nz, nx = d.g.nx;
-  const Turn t{{d.illum}, {d.mem}};
-  hipLaunchKernelGGL((k_turn<float, double>), dim3((nz + 31) / 32, (nx + 31) / 32, 1), dim3(32, 8), 0,
-                     d.stream, t, nx, nz, 0);
-  HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(out, d.mem, (size_t)d.g.N * sizeof(double), hipMemcpyDeviceToHost, d.stream));
-  HIP_TRY(hipStreamSynchronize(d.stream));
-  return Status::Ok();
+  return fetch_turned(d, d.illum, {out});
 }
 
 Status Plan::data(float* syn) {
