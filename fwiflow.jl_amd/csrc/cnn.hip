@@ -25,6 +25,7 @@
 //   k_adam       Adam update
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -116,6 +117,14 @@ __device__ __forceinline__ void stage(const TIn* __restrict__ in, int H, int W, 
 
 constexpr int kConvX = 32, kConvY = 8;  // pixels of a convolution's tile
 constexpr int kConvS = kConvX + 2;      // and of its row with the halo
+// Tiles of a map, along y and z of the grid in runs of kConvRun: 65536 workgroups,
+// the most along y, would end at 524288 rows.
+constexpr int kConvRun = 32768;
+__device__ __forceinline__ int conv_row() { return (int)(blockIdx.z * kConvRun + blockIdx.y) * kConvY; }
+dim3 conv_grid(int H, int W) {
+  const int rows = (H + kConvY - 1) / kConvY;
+  return dim3((W + kConvX - 1) / kConvX, std::min(rows, kConvRun), (rows + kConvRun - 1) / kConvRun);
+}
 
 enum Epilogue { kHidden = 0, kInputGrad = 1 };
 
@@ -143,7 +152,8 @@ __global__ __launch_bounds__(64 * kConvY) void k_conv32(const TIn* __restrict__ 
   constexpr int NW = kConvY, K = CIN * 9, CH = (kConvY + 2) * kConvS, WS = 33;
   __shared__ float tile[CIN * CH];
   __shared__ float wk[K * WS];  // [k][channel]
-  const int x0 = blockIdx.x * kConvX, y0 = blockIdx.y * kConvY;
+  const int x0 = blockIdx.x * kConvX, y0 = conv_row();
+  if (y0 >= H) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const size_t plane = (size_t)H * W;
   stage<TIn, CIN, C, kConvY + 2, kConvS, CH, NW>(in, H, W, x0 - 1, y0 - 1, tile);
@@ -206,7 +216,8 @@ __global__ __launch_bounds__(256) void k_conv3(const bf16_t* __restrict__ in, in
                                                const float* __restrict__ b, float* __restrict__ out) {
   constexpr int CH = (kConvY + 2) * kConvS;
   __shared__ float tile[32 * CH];
-  const int x0 = blockIdx.x * kConvX, y0 = blockIdx.y * kConvY;
+  const int x0 = blockIdx.x * kConvX, y0 = conv_row();
+  if (y0 >= H) return;
   stage<bf16_t, 32, 32, kConvY + 2, kConvS, CH, 4>(in, H, W, x0 - 1, y0 - 1, tile);
   __syncthreads();
   const int n = threadIdx.x & 31, x = x0 + n, y = y0 + (threadIdx.x >> 5);
@@ -402,8 +413,7 @@ template <typename TIn, int CIN, int C, int EPI>
 void conv32(CnnState& s, const TIn* in, const float* w, const float* bias, float* out_f32, bf16_t* zb,
             bf16_t* ab, const bf16_t* zin) {
   hipLaunchKernelGGL((k_conv32<TIn, CIN, C, EPI>),
-                     dim3((s.W + kConvX - 1) / kConvX, (s.H + kConvY - 1) / kConvY), dim3(64 * kConvY), 0,
-                     s.stream, in, s.H, s.W, w, bias, out_f32, zb, ab, zin);
+                     conv_grid(s.H, s.W), dim3(64 * kConvY), 0, s.stream, in, s.H, s.W, w, bias, out_f32, zb, ab, zin);
 }
 
 template <typename TIn, int CIN, int COUT>
@@ -421,7 +431,7 @@ Status forward(CnnState& s) {
   conv32<float, 4, 4, kHidden>(s, s.x0, W(0), B(0), nullptr, s.z[0], s.a[0], nullptr);
   for (int l = 1; l < 3; ++l)
     conv32<bf16_t, 32, 32, kHidden>(s, s.a[l - 1], W(l), B(l), nullptr, s.z[l], s.a[l], nullptr);
-  hipLaunchKernelGGL(k_conv3, dim3((s.W + kConvX - 1) / kConvX, (s.H + kConvY - 1) / kConvY), dim3(32 * kConvY), 0, s.stream,
+  hipLaunchKernelGGL(k_conv3, conv_grid(s.H, s.W), dim3(32 * kConvY), 0, s.stream,
                      s.a[2], s.H, s.W, W(3), B(3), s.out);
   CNN_HIP(hipGetLastError());
   return Status::Ok();
