@@ -35,10 +35,13 @@ HBM_PEAK_GBS = 8000.0
 KERNEL_BYTES = {
     "stress_fwd": 32.0,   # read vz vx szz sxx sxz, write szz sxx sxz
     "vel_fwd": 28.0,      # read szz sxx sxz vz vx, write vz vx
+    "step_fwd": 40.0,     # both in one launch: read 5, write 5
     "rev_vel": 36.0,      # read 3 stress, 2 velocity, 2 adjoint velocity, write 2 velocity
     "rev_stress": 44.0,   # read 2 velocity, 3 stress, 3 adjoint stress, write 3 stress
     "adj_vel": 28.0,      # read 3 adjoint stress, 2 adjoint velocity, write 2
     "adj_stress": 32.0,   # read 2 adjoint velocity, 3 adjoint stress, write 3
+    "rev_step": 60.0,     # both reversals: read 5 and 5 adjoint, write 5
+    "adj_step": 40.0,     # both adjoint updates: read 5, write 5
     # exact adjoint (--adjoint exact), each with the reverse step of its field;
     # outside the C-PML frame 3 of the 4 stress operands and 2 of the 4
     # velocity operands are distinct (KERNEL_FRAME adds the others)
@@ -51,7 +54,8 @@ KERNEL_BYTES = {
 # (k_exact_a reads 1 and writes 2, k_exact_b reads 2 and writes 1)
 KERNEL_FRAME = {"exact_a": 12.0, "exact_b": 12.0}
 # kernels that run two of the above as one grid (disjoint workgroup ranges)
-KERNEL_PARTS = {"bwd_pair_a": ("rev_stress", "adj_vel"), "bwd_pair_b": ("adj_stress", "rev_vel")}
+KERNEL_PARTS = {"bwd_pair_a": ("rev_stress", "adj_vel"), "bwd_pair_b": ("adj_stress", "rev_vel"),
+                "step_bwd": ("rev_step", "adj_step")}
 # Measured HBM-side bytes per launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, each
 # scaled by a 1 GiB copy's counters, averaged over the launches) at this
 # workload's shot groups: profiles/stencil_kernels_608x1780_counters.md.
@@ -62,10 +66,10 @@ MEASURED_TRAFFIC = {("bwd_pair_a", 2.91): 231.0e6, ("bwd_pair_b", 2.91): 226.3e6
                     ("exact_a", 2.0): 162.9e6, ("exact_b", 2.0): 199.8e6}
 # kernels of the backward sweep (their launches cover the backward shot groups)
 BACKWARD = ("rev_vel", "rev_stress", "adj_vel", "adj_stress", "bwd_pair_a", "bwd_pair_b",
-            "exact_a", "exact_b")
+            "step_bwd", "exact_a", "exact_b")
 # C-PML memory-variable traffic per PML cell-direction (2 variables RW = 16 B)
 KERNEL_PML = {"stress_fwd": 16.0, "vel_fwd": 16.0, "adj_vel": 16.0, "adj_stress": 16.0,
-              "exact_a": 16.0, "exact_b": 16.0}
+              "exact_a": 16.0, "exact_b": 16.0, "step_fwd": 32.0, "adj_step": 32.0}
 
 
 def parse():

@@ -213,7 +213,11 @@ int fwiflow_plan_memory_plan(fwiflow_plan* plan, int* ckpt_every, int* shots_per
                              long long* ring_bytes, long long* checkpoint_bytes);
 /* Kernel timing with HIP events on the plan's stream (off by default).
  * fwiflow_plan_timing(name) returns the summed milliseconds and launch count
- * of kernel `name` since timing was enabled. */
+ * of kernel `name` since timing was enabled (every 64th launch is timed), both
+ * 0 for one that was not launched.  Names: "stress_fwd" and "vel_fwd" (forward
+ * steps of two launches) or "step_fwd" (of one, on small grids); "bwd_pair_a"
+ * and "bwd_pair_b" (backward steps of two launches) or "step_bwd" (of one);
+ * "exact_a" and "exact_b" (exact adjoint). */
 int fwiflow_plan_set_timing(fwiflow_plan* plan, int enable);
 int fwiflow_plan_timing(fwiflow_plan* plan, const char* name, double* total_ms, long long* count);
 /* Device bytes held by the plan. */
