@@ -657,8 +657,27 @@ struct DeviceState {
     if (stream && own_stream) (void)hipStreamDestroy(stream);
   }
 
+  // The second states give way to every other buffer of the plan: none of its
+  // runs is under way when it asks for one (a run allocates them last).
   template <typename T>
   Status alloc(T** p, size_t count) {
+    Status s = take(p, count);
+    if (s.code == FWIFLOW_ERR_MEMORY && drop_second()) s = take(p, count);
+    return s;
+  }
+  bool drop_second() {
+    if (!fwd2 && !mem2 && !adj2 && !madj2) return false;
+    (void)hipGetLastError();
+    const size_t N = (size_t)g.N;
+    release(fwd2, (size_t)shots2 * kWaveComps * N);
+    release(mem2, (size_t)mshots2 * kMemComps * N);
+    release(adj2, (size_t)ashots2 * kWaveComps * N);
+    release(madj2, (size_t)xshots2 * kMemComps * N);
+    shots2 = mshots2 = ashots2 = xshots2 = 0;
+    return true;
+  }
+  template <typename T>
+  Status take(T** p, size_t count) {
     void* q = nullptr;
     const size_t nb = count * sizeof(T);
     if (arena) {
@@ -1012,7 +1031,7 @@ static Status ensure_injection(DeviceState& d) {
       }
     }
   auto put = [&](auto*& p, const auto& v) -> Status {
-    TRY(d.alloc(&p, std::max<size_t>(1, v.size())));
+    if (!p) TRY(d.alloc(&p, std::max<size_t>(1, v.size())));
     if (!v.empty()) HIP_TRY(hipMemcpy(p, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice));
     return Status::Ok();
   };
@@ -1729,7 +1748,7 @@ Status Runner::second_states(DeviceState& d, int mf, int mb) {
     const size_t n = (size_t)comps * d.g.N;
     d.release(p, have * n);
     have = 0;
-    TRY(d.alloc(&p, need * n));
+    TRY(d.take(&p, need * n));
     have = need;
     HIP_TRY(hipMemsetAsync(p, 0, need * n * sizeof(float), st));
     return Status::Ok();
@@ -1927,72 +1946,79 @@ Status Runner::run(int calc_id) {
   whole_b_ = !c0.arena && withAdj && mb <= kWholeBwdShots &&
              tiles(mb) <= (mb == 1 ? kWholeBwdWaves1 : kWholeBwdWaves);
   for (const Member& m : M) whole_b_ = whole_b_ && !m.d->adjoint && m.d->inj_folded;
-  // buffers
-  for (const Member& m : M) {
-    DeviceState& d = *m.d;
-    const size_t N = (size_t)d.g.N, F = d.F();
-    if (withAdj) {
-      if (!d.adj) TRY(d.alloc(&d.adj, 5 * F));
-      if (ckpt && !d.madj) TRY(d.alloc(&d.madj, 8 * F));
-      if (!d.acc) TRY(d.alloc(&d.acc, 5 * N));
-      if (!d.grad) TRY(d.alloc(&d.grad, 3 * N));
-      if (!d.stf_grad) TRY(d.alloc(&d.stf_grad, (size_t)d.g.ns * nSteps));
-      if (d.adjoint) {
-        const size_t xf = (size_t)std::min(gb, d.g.ns) * 8 * N;
-        if (d.xt_floats < xf) {
-          d.release(d.xt, d.xt_floats);
-          d.xt_floats = 0;
-          TRY(d.alloc(&d.xt, xf));
-          d.xt_floats = xf;
+  // buffers; where a plan of a job has no room for its own, the second states
+  // that others hold from earlier runs give way
+  auto buffers = [&]() -> Status {
+    for (const Member& m : M) {
+      DeviceState& d = *m.d;
+      const size_t N = (size_t)d.g.N, F = d.F();
+      if (withAdj) {
+        if (!d.adj) TRY(d.alloc(&d.adj, 5 * F));
+        if (ckpt && !d.madj) TRY(d.alloc(&d.madj, 8 * F));
+        if (!d.acc) TRY(d.alloc(&d.acc, 5 * N));
+        if (!d.grad) TRY(d.alloc(&d.grad, 3 * N));
+        if (!d.stf_grad) TRY(d.alloc(&d.stf_grad, (size_t)d.g.ns * nSteps));
+        if (d.adjoint) {
+          const size_t xf = (size_t)std::min(gb, d.g.ns) * 8 * N;
+          if (d.xt_floats < xf) {
+            d.release(d.xt, d.xt_floats);
+            d.xt_floats = 0;
+            TRY(d.alloc(&d.xt, xf));
+            d.xt_floats = xf;
+          }
         }
-      }
-      const int rows_m = std::min(S, d.g.ns);
-      const size_t rf = (size_t)rows_m * (ckpt ? K : steps) * d.ring_step_floats();
-      if (d.ring_floats < rf || d.ring_floats > 2 * rf + (1u << 20)) {
-        d.release(d.ring, d.ring_floats);
-        d.ring_floats = 0;
-        TRY(d.alloc(&d.ring, rf));
-        d.ring_floats = rf;
-      }
-      const size_t sf = ckpt ? (size_t)nsnap * 13 * rows_m * N : 0;
-      if (d.snap_floats < sf || (sf == 0 && d.snap)) {
-        d.release(d.snap, d.snap_floats);
-        d.snap_floats = 0;
-        if (sf) {
-          TRY(d.alloc(&d.snap, sf));
-          d.snap_floats = sf;
+        const int rows_m = std::min(S, d.g.ns);
+        const size_t rf = (size_t)rows_m * (ckpt ? K : steps) * d.ring_step_floats();
+        if (d.ring_floats < rf || d.ring_floats > 2 * rf + (1u << 20)) {
+          d.release(d.ring, d.ring_floats);
+          d.ring_floats = 0;
+          TRY(d.alloc(&d.ring, rf));
+          d.ring_floats = rf;
         }
+        const size_t sf = ckpt ? (size_t)nsnap * 13 * rows_m * N : 0;
+        if (d.snap_floats < sf || (sf == 0 && d.snap)) {
+          d.release(d.snap, d.snap_floats);
+          d.snap_floats = 0;
+          if (sf) {
+            TRY(d.alloc(&d.snap, sf));
+            d.snap_floats = sf;
+          }
+        }
+        d.last_k = K;
+        d.last_rows_sg = rows_m;
+        d.last_ring_bytes = (long long)(rf * sizeof(float));
+        d.last_snap_bytes = (long long)(sf * sizeof(float));
       }
-      d.last_k = K;
-      d.last_rows_sg = rows_m;
-      d.last_ring_bytes = (long long)(rf * sizeof(float));
-      d.last_snap_bytes = (long long)(sf * sizeof(float));
+      if (withAdj) TRY(ensure_injection(d));
+      const int npart = (int)sweeps.size() * kPartials;
+      if (d.npartial < npart) {
+        d.release(d.partial, (size_t)d.npartial);
+        d.npartial = 0;
+        TRY(d.alloc(&d.partial, (size_t)npart));
+        d.npartial = npart;
+      }
+      if (d.illum_on && !d.illum) TRY(d.alloc(&d.illum, N));
+      d.src_updated = if_res && d.cond && m.plan->para.if_src_update;
+      d.last_groups_f = 0;
+      d.last_groups_b = 0;
+      for (size_t j = 0; j < sweeps.size(); j++) {
+        for (RowRange rr : FR[j]) d.last_groups_f += shots_in(m, rr.r1) > shots_in(m, rr.r0);
+        for (RowRange rr : BR[j]) d.last_groups_b += shots_in(m, rr.r1) > shots_in(m, rr.r0);
+      }
     }
-    if (withAdj) TRY(ensure_injection(d));
-    const int npart = (int)sweeps.size() * kPartials;
-    if (d.npartial < npart) {
-      d.release(d.partial, (size_t)d.npartial);
-      d.npartial = 0;
-      TRY(d.alloc(&d.partial, (size_t)npart));
-      d.npartial = npart;
-    }
-    if (d.illum_on && !d.illum) TRY(d.alloc(&d.illum, N));
-    d.src_updated = if_res && d.cond && m.plan->para.if_src_update;
-    d.last_groups_f = 0;
-    d.last_groups_b = 0;
-    for (size_t j = 0; j < sweeps.size(); j++) {
-      for (RowRange rr : FR[j]) d.last_groups_f += shots_in(m, rr.r1) > shots_in(m, rr.r0);
-      for (RowRange rr : BR[j]) d.last_groups_b += shots_in(m, rr.r1) > shots_in(m, rr.r0);
-    }
-  }
-  {
     size_t nf = 0, nb = 0;  // argument table entries
     for (size_t j = 0; j < sweeps.size(); j++) {
       nf += FR[j].size() + (ckpt ? BR[j].size() : 0);
       nb += BR[j].size();
     }
     TRY(cache.reserve(nf * M.size() * (whole_f_ ? 3 : 1), cache.steps, cache.steps_cap));
-    TRY(cache.reserve(nb * M.size() * (whole_b_ ? 5 : 1), cache.backs, cache.backs_cap));
+    return cache.reserve(nb * M.size() * (whole_b_ ? 5 : 1), cache.backs, cache.backs_cap);
+  };
+  if (Status s = buffers(); !s.ok()) {
+    bool held = false;
+    for (const Member& m : M) held = m.d->drop_second() || held;
+    if (!held) return s;
+    TRY(buffers());
   }
   // The second states come last: a run without them takes two launches a step,
   // all members alike.
@@ -2002,15 +2028,7 @@ Status Runner::run(int calc_id) {
   if (!second.ok()) {
     if (second.code != FWIFLOW_ERR_MEMORY) return second;
     (void)hipGetLastError();
-    for (const Member& m : M) {
-      DeviceState& d = *m.d;
-      const size_t N = (size_t)d.g.N;
-      d.release(d.fwd2, (size_t)d.shots2 * kWaveComps * N);
-      d.release(d.mem2, (size_t)d.mshots2 * kMemComps * N);
-      d.release(d.adj2, (size_t)d.ashots2 * kWaveComps * N);
-      d.release(d.madj2, (size_t)d.xshots2 * kMemComps * N);
-      d.shots2 = d.mshots2 = d.ashots2 = d.xshots2 = 0;
-    }
+    for (const Member& m : M) m.d->drop_second();
     whole_f_ = whole_b_ = false;
     slice(mf, sf_, nf_);
   }

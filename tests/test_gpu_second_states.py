@@ -103,3 +103,31 @@ def test_second_states_are_sized_for_the_launches_that_have_them(workspace):
         held, got = _run(P, 0)
     assert _same(got, want)
     assert most - held == 18 * 4 * cells
+
+
+@pytest.mark.parametrize("shots,every", [(2, 0), (3, 17), (5, 0)])
+def test_second_states_of_earlier_runs_give_way(workspace, shots, every):
+    """A modelling run takes one launch a step and keeps its second state; what
+    the plan asks for afterwards (observed data, a gradient's buffers,
+    illumination) has to find the room that it would have found without."""
+    para, stf, ids, m = case = _case(workspace, 41, 61, shots)
+    with _plan(case) as P:
+        most, want = _run(P, every)
+        obs = np.concatenate([np.fromfile(f"{workspace}/Data/Shot{i}.bin", np.float32) for i in ids])
+    with _plan(case, most - 4) as P:
+        held, _ = _run(P, every)
+    with env(FWIFLOW_PLAN_BYTES=str(held)):
+        P = fwiflow.Plan(para, ids)
+    with P:
+        P.set_model(*m)
+        P.set_stf(stf)
+        P.run(2)
+        assert P.tile_width() == 0
+        assert np.array_equal(P.data(), want[0])
+        P.set_obs(obs)
+        P.run(0)
+        h, got = _run(P, every)
+        assert h <= held and _same(got, want)
+        P.run(2)
+        assert np.array_equal(P.data(), want[0])
+        assert _same(_run(P, every)[1], want)
